@@ -55,8 +55,7 @@ __global__ void __launch_bounds__(kRowKernelThreads) expand_rows_kernel(DeviceSt
             state.expanded_source_meta[my_row * 3 + 2] = lane;
         }
     }
-    if (state.zero_padding)
-        for (int expert = global_wave; expert < local; expert += total_waves) zero_padding_of_expert<false>(state, expert, lane);
+    if (state.zero_padding) zero_padding_rows<false>(state, global_wave, total_waves, lane);
 }
 
 // The same expand for rows of whole 16-byte vectors, shaped for HBM: a workgroup
@@ -141,8 +140,10 @@ __global__ void __launch_bounds__(kPieceThreads) expand_pieces_kernel(DeviceStat
         ordinal = lane < topk ? state.unique_expert_ordinals[row * topk + lane] : 0;
     }
     if (state.zero_padding) {
-        const int global_wave = blockIdx.x * (kPieceThreads / kWave) + threadIdx.x / kWave;
-        if (global_wave < local) zero_padding_of_expert<true>(state, global_wave, lane);
+        // As many wavefronts as there can be gap rows; the others do not even look.
+        const int global_wave = blockIdx.x * (kPieceThreads / kWave) + threadIdx.x / kWave, total_waves = int(gridDim.x) * (kPieceThreads / kWave);
+        const int most = local * (state.alignment - 1), waves = most < total_waves ? most : total_waves;
+        if (global_wave < waves) zero_padding_rows<true>(state, global_wave, waves, lane);
     }
 }
 
@@ -283,13 +284,13 @@ hipError_t launch_expand(const DeviceState& state, hipStream_t stream) {
     const int64_t capacity = unique_capacity(state.z.dims);
     if (state.z.dims.hidden % 8 == 0) {
         // 2 KiB pieces, one workgroup each; the grid is folded so that it has about
-        // 150 000 workgroups at most (a third of a 65 536-row pool of 14 KiB rows)
-        // and at least one workgroup per piece of every local expert's padding.
+        // 150 000 workgroups at most (a third of a 65 536-row pool of 14 KiB rows).
         const int64_t pieces = (state.z.dims.hidden / 8 + kPieceThreads - 1) / kPieceThreads;
         constexpr int64_t kTargetWorkgroups = 152922;
         const int64_t fold = (capacity * pieces + kTargetWorkgroups - 1) / kTargetWorkgroups;
         int64_t span = (capacity + fold - 1) / fold;
-        const int64_t padding_groups = (state.z.local_experts + 1) / 2;  // two wavefronts per workgroup
+        // At most four gap rows per wavefront (two wavefronts per workgroup), however small the pool is.
+        const int64_t padding_groups = state.zero_padding ? (int64_t(state.z.local_experts) * (state.alignment - 1) + 7) / 8 : 0;
         if (span * pieces < padding_groups) span = (padding_groups + pieces - 1) / pieces;
         if (span * pieces > (int64_t(1) << 30)) return hipErrorInvalidValue;  // cannot happen within the supported dimensions
         hipLaunchKernelGGL(expand_pieces_kernel, dim3(unsigned(span * pieces)), dim3(kPieceThreads), 0, stream, state, int(pieces), int(span));

@@ -196,22 +196,49 @@ __device__ __forceinline__ void zero_row(uint16_t* output, int hidden, int lane)
     }
 }
 
-// Alignment gap of one local expert, rows [offset + count, next offset):
-// payload 0, expert -1, weight 0, metadata -1 (advanced_layout.cuh:250-265).
+// Alignment gaps of the local experts, rows [offset + count, next offset) of each:
+// payload 0, expert -1, weight 0, metadata -1 (advanced_layout.cuh:250-265).  The gap
+// rows of all experts are counted through, and wavefront `wave` of `waves` takes rows
+// wave, wave + waves, ...: a small batch under a wide alignment is nothing but gap rows
+// (16 tokens in 128-row tiles: 150 rows in use, 3 800 to zero), and with one wavefront
+// per expert its 124 rows one after the other were the longest path of the dispatch
+// (transport kernel at 7168 columns, 128-row alignment: T=16 535 us, 59 with the rows
+// dealt over the local-bypass workgroups; T=96 185 us, 146, which is what it takes
+// without any gap).  A wavefront finds its
+// rows without memory traffic of its own: lane l holds expert l's gap, and a wave-wide
+// scan of the gaps locates every row.
 // The prefixes are read with device-scope loads: inside the transport kernel
 // they were written by another wavefront of the same launch.
 template <bool kVector>
-__device__ __forceinline__ void zero_padding_of_expert(const DeviceState& state, int expert, int lane) {
-    const int hidden = state.z.dims.hidden;
-    const int64_t next = device_load(state.expert_offsets + expert + 1);
-    const int64_t end = next < state.expanded_capacity ? next : state.expanded_capacity;
-    for (int64_t row = device_load(state.expert_prefix + expert); row < end; ++row) {
-        zero_row<kVector>(state.expanded_payload + size_t(row) * hidden, hidden, lane);
-        if (lane == 0) {
-            state.expanded_expert_idx[row] = -1;
-            state.expanded_weights[row] = 0.0f;
-            state.expanded_source_meta[row * 3] = state.expanded_source_meta[row * 3 + 1] = state.expanded_source_meta[row * 3 + 2] = -1;
+__device__ __forceinline__ void zero_padding_rows(const DeviceState& state, int wave, int waves, int lane) {
+    const int hidden = state.z.dims.hidden, local = state.z.local_experts;
+    int before = 0;  // gap rows of the experts in front of this group of 64
+    for (int begin = 0; begin < local; begin += kWave) {
+        const int expert = begin + lane;
+        int first = 0, gap = 0;
+        if (expert < local) {
+            first = device_load(state.expert_prefix + expert);
+            const int64_t next = device_load(state.expert_offsets + expert + 1);
+            const int64_t end = next < state.expanded_capacity ? next : state.expanded_capacity;
+            gap = end > first ? int(end - first) : 0;
         }
+        int through = gap;
+        for (int offset = 1; offset < kWave; offset <<= 1) {
+            const int other = __shfl_up(through, offset);
+            if (lane >= offset) through += other;
+        }
+        const int total = __shfl(through, kWave - 1);
+        for (int index = (wave + waves - before % waves) % waves; index < total; index += waves) {
+            const int owner = __builtin_ctzll(__ballot(through > index));
+            const int64_t row = __shfl(first, owner) + (index - (__shfl(through, owner) - __shfl(gap, owner)));
+            zero_row<kVector>(state.expanded_payload + size_t(row) * hidden, hidden, lane);
+            if (lane == 0) {
+                state.expanded_expert_idx[row] = -1;
+                state.expanded_weights[row] = 0.0f;
+                state.expanded_source_meta[row * 3] = state.expanded_source_meta[row * 3 + 1] = state.expanded_source_meta[row * 3 + 2] = -1;
+            }
+        }
+        before += total;
     }
 }
 

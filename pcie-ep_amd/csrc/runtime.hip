@@ -321,14 +321,16 @@ int build_state(pcie_ep_runtime* rt, const pcie_ep_dispatch_args* a, DeviceState
     s.worker_groups = rt->worker_groups;
     s.tx_waves = rt->tx_waves;
     s.rx_waves = rt->rx_waves;
-    // One local-bypass wavefront per ~8 own tokens, at most 32 workgroups: the work
-    // (HBM only) then ends long before the host link has moved the remote rows.
+    s.fuse_expand = rt->config.fuse_receive_expand ? 1 : 0;
+    // One local-bypass wavefront per ~8 own tokens and, where it clears alignment gaps, per
+    // ~8 rows that those can have, at most 32 workgroups: the work (HBM only) then ends long
+    // before the host link has moved the remote rows.
     {
         const int waves_per_group = transport_threads(s) / kWave;
-        const int wanted = (a->num_tokens / 8 + waves_per_group) / waves_per_group;
+        const int gap_rows = a->expand && a->zero_padding && s.fuse_expand ? rt->z.local_experts * (a->alignment - 1) : 0;
+        const int wanted = ((a->num_tokens > gap_rows ? a->num_tokens : gap_rows) / 8 + waves_per_group) / waves_per_group;
         s.local_groups = wanted < 1 ? 1 : (wanted > 32 ? 32 : wanted);
     }
-    s.fuse_expand = rt->config.fuse_receive_expand ? 1 : 0;
     s.expand = a->expand ? 1 : 0;
     s.alignment = a->alignment;
     s.num_tokens = a->num_tokens;

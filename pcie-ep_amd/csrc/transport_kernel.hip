@@ -816,11 +816,11 @@ __device__ __forceinline__ void rx_control(const DeviceState& state, TransportQu
 // ---------------------------------------------------------------------------------------
 // Local bypass, padding and the final reduction
 // ---------------------------------------------------------------------------------------
-// Work items: own tokens 0 .. T-1, then (with zero padding on an expanded
-// layout) the local experts' alignment gaps.  Every wavefront of the local
-// workgroups claims items one at a time until none is left.
+// Every wavefront of the local workgroups claims own tokens 0 .. T-1 one at a time
+// until none is left, then (with zero padding on an expanded layout) clears its
+// share of the alignment gaps' rows; `wave` is its position among the `waves` of them.
 template <bool kVector>
-__device__ __forceinline__ void local_rows(const DeviceState& state, TransportQueues& q, int lane) {
+__device__ __forceinline__ void local_rows(const DeviceState& state, TransportQueues& q, int lane, int wave, int waves) {
     const uint64_t epoch = dispatch_epoch(state);
     // Destination rows depend on the receive prefixes of this epoch.
     int ready = 0;
@@ -835,16 +835,13 @@ __device__ __forceinline__ void local_rows(const DeviceState& state, TransportQu
     }
     if (!broadcast_first(ready)) return;
     if (!wait_for_plan(state, q, lane)) return;
-    const bool padding = state.expand && state.fuse_expand && state.zero_padding;
-    const int items = state.num_tokens + (padding ? state.z.local_experts : 0);
     while (true) {
         uint32_t claimed = 0;
         if (lane == 0) claimed = aborted(q) ? 0xFFFFFFFFu : device_add(&q.local_head.value, 1u);
         const int item = broadcast_first(int(claimed));
-        if (item < 0 || item >= items) return;
-        if (item >= state.num_tokens) {
-            zero_padding_of_expert<kVector>(state, item - state.num_tokens, lane);
-        } else if (!local_token_rows<kVector>(state, item, lane)) {
+        if (item < 0) return;
+        if (item >= state.num_tokens) break;
+        if (!local_token_rows<kVector>(state, item, lane)) {
             if (lane == 0) {
                 record_error(state, kErrExpandedCapacity);
                 raise_abort(q);
@@ -852,6 +849,7 @@ __device__ __forceinline__ void local_rows(const DeviceState& state, TransportQu
             return;
         }
     }
+    if (state.expand && state.fuse_expand && state.zero_padding) zero_padding_rows<kVector>(state, wave, waves, lane);
 }
 
 // Called by every role wavefront as its last act.  Everything the reduction
@@ -1514,7 +1512,7 @@ __global__ void __launch_bounds__(kTransportMaxThreads) transport_kernel(DeviceS
         return;  // the prologue kernel in front of this one failed
     }
     if (block >= channel_groups + payload_groups) {
-        if (begun) local_rows<kVector>(state, q, lane);
+        if (begun) local_rows<kVector>(state, q, lane, (block - channel_groups - payload_groups) * waves_per_group + wave, state.local_groups * waves_per_group);
         return finish_role(state, q, lane, roles);
     }
     if (block < channel_groups) {

@@ -177,6 +177,19 @@ def test_separate_expand_with_more_padding_work_than_rows():
         check_case(buffer, "wide-grid-one-row", [1], alignment=256, capture=False)
 
 
+@pytest.mark.parametrize("fuse", [True, False])
+@pytest.mark.parametrize("world,experts,alignment,hidden", [(8, 8, 256, 1024), (2, 128, 128, 264), (2, 130, 2, 129), (1, 200, 64, 2048), (8, 256, 128, 7168)])
+def test_alignment_gaps_of_small_batches(world, experts, alignment, hidden, fuse):
+    """A few tokens under a wide alignment: nearly every row is a gap row, dealt out over
+    all wavefronts that clear them.  One local expert, exactly 64 (one per lane), 65 and
+    200 (several groups of lanes), gaps of one row, scalar rows, and no token at all."""
+    print(f"case: gaps world={world} experts={experts} alignment={alignment} hidden={hidden} fuse={fuse}", flush=True)
+    mode = {} if fuse else {"fuse_receive_expand": False, "receive_expand_mode": "scalar"}
+    with make_buffer(world=world, tmax=9, hidden=hidden, topk=4, experts=experts, channels=3, payload_slots=4, descriptor_slots=4, **mode) as buffer:
+        check_case(buffer, "gaps", [9, 3, 1, 0, 2, 9, 5, 7][:world], alignment=alignment, capture=world > 1)
+        check_case(buffer, "gaps-empty", [0] * world, alignment=alignment, seed=9, capture=world > 1)
+
+
 def test_numa_bound_staging_segments():
     """The pinned segments can be bound to a NUMA node (the far-node staging of the
     cached-replay configuration); node 0 exists on every box.  Results do not change."""
