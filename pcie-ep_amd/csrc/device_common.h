@@ -633,4 +633,88 @@ struct RowScalars {
     uint16_t v[kPassScalars];
 };
 
+// Rows that are not whole 16-byte vectors: the whole vectors move as above, from and to
+// any address (unaligned 16-byte accesses to device memory are one instruction like aligned
+// ones; a row then starts in the middle of a line that its neighbour ends in, so these
+// stores are not streamed past the L2, which merges them), and the 1..15 bytes behind them
+// are `rest` bytes in the low end of one more vector, moved by one lane in pieces of
+// 8, 4, 2 and 1 bytes.  Nothing beyond the row is touched.
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+typedef uint64_t u64_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
+__device__ __forceinline__ u32x4 load_rest(const char* address, int rest) {
+    uint64_t low = 0, high = 0;
+    int shift = 0;
+    if (rest & 8) {
+        low = *reinterpret_cast<const u64_any*>(address);
+        address += 8;
+    }
+    if (rest & 4) {
+        high = *reinterpret_cast<const u32_any*>(address);
+        address += 4;
+        shift = 32;
+    }
+    if (rest & 2) {
+        high |= uint64_t(*reinterpret_cast<const u16_any*>(address)) << shift;
+        address += 2;
+        shift += 16;
+    }
+    if (rest & 1) high |= uint64_t(*reinterpret_cast<const uint8_t*>(address)) << shift;
+    if (!(rest & 8)) {
+        low = high;
+        high = 0;
+    }
+    return u32x4{uint32_t(low), uint32_t(low >> 32), uint32_t(high), uint32_t(high >> 32)};
+}
+__device__ __forceinline__ void store_rest(char* address, int rest, const u32x4& value) {
+    uint64_t bits = uint64_t(value[0]) | uint64_t(value[1]) << 32;
+    if (rest & 8) {
+        *reinterpret_cast<u64_any*>(address) = bits;
+        address += 8;
+        bits = uint64_t(value[2]) | uint64_t(value[3]) << 32;
+    }
+    if (rest & 4) {
+        *reinterpret_cast<u32_any*>(address) = uint32_t(bits);
+        address += 4;
+        bits >>= 32;
+    }
+    if (rest & 2) {
+        *reinterpret_cast<u16_any*>(address) = uint16_t(bits);
+        address += 2;
+        bits >>= 16;
+    }
+    if (rest & 1) *reinterpret_cast<uint8_t*>(address) = uint8_t(bits);
+}
+// Vector `index` of a row in device memory; kVector: the row lies on a 16-byte boundary.
+template <bool kVector>
+__device__ __forceinline__ u32x4 row_load_vector(const void* row, int index) {
+    if constexpr (kVector) return __builtin_nontemporal_load(static_cast<const u32x4*>(row) + index);
+    else return static_cast<const u32x4_any*>(row)[index];
+}
+template <bool kVector>
+__device__ __forceinline__ void row_store_vector(void* row, int index, const u32x4& value) {
+    if constexpr (kVector) __builtin_nontemporal_store(value, static_cast<u32x4*>(row) + index);
+    else static_cast<u32x4_any*>(row)[index] = value;
+}
+template <bool kVector>
+__device__ __forceinline__ void row_load_pass(RowVectors& row, const uint16_t* source, int first, int count, int lane) {
+#pragma unroll
+    for (int j = 0; j < kPassItems; ++j) {
+        const int index = first + j * kWave + lane;
+        if (index < count) row.v[j] = row_load_vector<kVector>(source, index);
+    }
+}
+template <bool kVector>
+__device__ __forceinline__ void row_store_pass(const RowVectors& row, uint16_t* destination, int first, int count, int lane) {
+#pragma unroll
+    for (int j = 0; j < kPassItems; ++j) {
+        const int index = first + j * kWave + lane;
+        if (index < count) row_store_vector<kVector>(destination, index, row.v[j]);
+    }
+}
+// Bytes behind the whole vectors of a BF16 row, 0 where kVector says that there are none.
+template <bool kVector>
+__device__ __forceinline__ int row_rest(int hidden) { return kVector ? 0 : hidden % 8 * 2; }
+
 }  // namespace pcie_ep

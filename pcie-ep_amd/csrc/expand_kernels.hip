@@ -147,24 +147,106 @@ __global__ void __launch_bounds__(kPieceThreads) expand_pieces_kernel(DeviceStat
     }
 }
 
+// The FP8 wire codec on rows in device memory (the dispatch has it inside its row movers).
+// Bound by HBM: 3 bytes per element either way.  A row is split over one, two or four
+// wavefronts of a workgroup of four, so that a lane holds at most four 16-byte vectors of a
+// row of up to 8192 elements: the row is read once and waits in registers for its maximum,
+// and with few registers per lane a compute unit holds all the wavefronts it can, which is
+// what keeps enough reads in flight.  8192 rows of 7168, both directions: 59.5 us = 5.9 TB/s;
+// with one wavefront per row, which read the row twice and moved 16 elements per lane, 89.3 us.
+// A lane moves 8 elements at a time, 16 bytes of BF16 and 8 of codes, so that every access of
+// a wavefront is one contiguous run.  Longer rows take further passes, and their maximum
+// a sweep of its own.
+constexpr int kCodecItems = 4;  // vectors of 8 elements a lane holds
+constexpr int kCodecWaves = kRowKernelThreads / kWave;
+// Wavefronts per row: as few as hold the row, at most all four.
+int codec_split(int hidden) { return hidden <= kCodecItems * kWave * 8 ? 1 : (hidden <= 2 * kCodecItems * kWave * 8 ? 2 : 4); }
+
 template <bool kVector>
-__global__ void __launch_bounds__(kRowKernelThreads) quantize_kernel(const uint16_t* x, uint8_t* codes, float* scales, int tokens, int hidden) {
-    const int lane = threadIdx.x % kWave;
-    const int waves_per_block = blockDim.x / kWave;
-    const int total_waves = gridDim.x * waves_per_block;
-    for (int token = blockIdx.x * waves_per_block + threadIdx.x / kWave; token < tokens; token += total_waves) {
-        const float scale = quantize_row<kVector>(x + size_t(token) * hidden, DeviceCodes{codes + size_t(token) * hidden}, hidden, lane);
-        if (lane == 0) scales[token] = scale;
+__device__ __forceinline__ void store_codes(uint8_t* codes, int index, const u32x4& v, float inverse) {
+    const uint64_t word = uint64_t(fp8_quantize_word(v[0], v[1], inverse)) | uint64_t(fp8_quantize_word(v[2], v[3], inverse)) << 32;
+    if constexpr (kVector) __builtin_nontemporal_store(word, reinterpret_cast<uint64_t*>(codes) + index);
+    else reinterpret_cast<u64_any*>(codes)[index] = word;
+}
+template <bool kVector>
+__global__ void __launch_bounds__(kRowKernelThreads) quantize_kernel(const uint16_t* x, uint8_t* codes, float* scales, int tokens, int hidden, int split) {
+    __shared__ float maxima[kCodecWaves];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int token = blockIdx.x * (kCodecWaves / split) + wave / split, part = wave % split;
+    const bool present = token < tokens;  // every wavefront reaches the barrier below
+    const uint16_t* input = x + size_t(present ? token : 0) * hidden;
+    uint8_t* output = codes + size_t(present ? token : 0) * hidden;
+    const int vectors = present ? hidden / 8 : 0, rest = present ? row_rest<kVector>(hidden) : 0, step = split * kWave;
+    // Item j of this lane is vector part * 64 + lane + j * step; the elements behind the whole vectors are one more of the last part's first lane.
+    const int first = part * kWave + lane;
+    u32x4 held[kCodecItems], last = {0u, 0u, 0u, 0u};
+    float amax = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kCodecItems; ++j) {
+        held[j] = u32x4{0u, 0u, 0u, 0u};
+        if (first + j * step < vectors) held[j] = row_load_vector<kVector>(input, first + j * step);
+    }
+    const bool holds_rest = rest && part == split - 1 && lane == 0;
+    if (holds_rest) last = load_rest(reinterpret_cast<const char*>(input + vectors * 8), rest);
+#pragma unroll
+    for (int j = 0; j < kCodecItems; ++j) amax = vector_amax(amax, held[j]);
+    amax = vector_amax(amax, last);
+    for (int index = first + kCodecItems * step; index < vectors; index += step) amax = vector_amax(amax, row_load_vector<false>(input, index));
+    amax = wave_max(amax);
+    if (split > 1) {
+        if (lane == 0) maxima[wave] = amax;
+        __syncthreads();
+        for (int other = wave - part; other < wave - part + split; ++other) amax = fmaxf(amax, maxima[other]);
+    }
+    const float scale = fp8_scale_from_amax(amax), inverse = 1.0f / scale;
+    if (first == 0 && present) scales[token] = scale;
+#pragma unroll
+    for (int j = 0; j < kCodecItems; ++j)
+        if (first + j * step < vectors) store_codes<kVector>(output, first + j * step, held[j], inverse);
+    for (int index = first + kCodecItems * step; index < vectors; index += step) store_codes<kVector>(output, index, row_load_vector<false>(input, index), inverse);
+    if (holds_rest) {
+        const u32x4 word = {fp8_quantize_word(last[0], last[1], inverse), fp8_quantize_word(last[2], last[3], inverse), 0u, 0u};
+        store_rest(reinterpret_cast<char*>(output) + vectors * 8, rest / 2, word);
     }
 }
 
 template <bool kVector>
-__global__ void __launch_bounds__(kRowKernelThreads) dequantize_kernel(const uint8_t* codes, const float* scales, uint16_t* out, int tokens, int hidden) {
-    const int lane = threadIdx.x % kWave;
-    const int waves_per_block = blockDim.x / kWave;
-    const int total_waves = gridDim.x * waves_per_block;
-    for (int token = blockIdx.x * waves_per_block + threadIdx.x / kWave; token < tokens; token += total_waves)
-        dequantize_row<kVector>(codes + size_t(token) * hidden, scales[token], out + size_t(token) * hidden, hidden, lane);
+__global__ void __launch_bounds__(kRowKernelThreads) dequantize_kernel(const uint8_t* codes, const float* scales, uint16_t* out, int tokens, int hidden, int split) {
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int token = blockIdx.x * (kCodecWaves / split) + wave / split, part = wave % split;
+    if (token >= tokens) return;
+    const float scale = scales[token];
+    const uint8_t* input = codes + size_t(token) * hidden;
+    uint16_t* output = out + size_t(token) * hidden;
+    const int vectors = hidden / 8, rest = row_rest<kVector>(hidden), step = split * kWave;
+    for (int first = part * kWave + lane; first < vectors; first += kCodecItems * step) {
+        uint64_t held[kCodecItems];
+#pragma unroll
+        for (int j = 0; j < kCodecItems; ++j) {
+            const int index = first + j * step;
+            if (index >= vectors) continue;
+            if constexpr (kVector) held[j] = __builtin_nontemporal_load(reinterpret_cast<const uint64_t*>(input) + index);
+            else held[j] = reinterpret_cast<const u64_any*>(input)[index];
+        }
+#pragma unroll
+        for (int j = 0; j < kCodecItems; ++j) {
+            const int index = first + j * step;
+            if (index >= vectors) continue;
+            uint32_t a, b, c, d;
+            fp8_dequantize_word(uint32_t(held[j]), scale, a, b);
+            fp8_dequantize_word(uint32_t(held[j] >> 32), scale, c, d);
+            row_store_vector<kVector>(output, index, u32x4{a, b, c, d});
+        }
+    }
+    if (rest && part == split - 1 && lane == 0) {
+        const u32x4 last = load_rest(reinterpret_cast<const char*>(input) + vectors * 8, rest / 2);
+        u32x4 value;
+        uint32_t a, b, c, d;
+        fp8_dequantize_word(last[0], scale, a, b);
+        fp8_dequantize_word(last[1], scale, c, d);
+        value = u32x4{a, b, c, d};
+        store_rest(reinterpret_cast<char*>(output + vectors * 8), rest, value);
+    }
 }
 
 // Plain device copy: every wavefront moves one contiguous 8 KiB (8 x 16-byte
@@ -341,19 +423,26 @@ hipError_t launch_host_copy(void* host, void* device, int64_t bytes, bool to_dev
     return hipGetLastError();
 }
 
+// Rows on the widest boundaries that their vectors need: whole vectors, and the arrays where allocators put them.
+static bool codec_vector(const void* bf16, const void* codes, int hidden) {
+    return hidden % 8 == 0 && reinterpret_cast<uintptr_t>(bf16) % 16 == 0 && reinterpret_cast<uintptr_t>(codes) % 8 == 0;
+}
+
 hipError_t launch_quantize(const uint16_t* x, uint8_t* codes, float* scales, int tokens, int hidden, hipStream_t stream) {
     if (tokens <= 0) return hipSuccess;
-    const dim3 grid(row_grid(tokens)), block(kRowKernelThreads);
-    if (hidden % 16 == 0) hipLaunchKernelGGL(quantize_kernel<true>, grid, block, 0, stream, x, codes, scales, tokens, hidden);
-    else hipLaunchKernelGGL(quantize_kernel<false>, grid, block, 0, stream, x, codes, scales, tokens, hidden);
+    const int split = codec_split(hidden), rows = kCodecWaves / split;
+    const dim3 grid(unsigned((int64_t(tokens) + rows - 1) / rows)), block(kRowKernelThreads);
+    if (codec_vector(x, codes, hidden)) hipLaunchKernelGGL(quantize_kernel<true>, grid, block, 0, stream, x, codes, scales, tokens, hidden, split);
+    else hipLaunchKernelGGL(quantize_kernel<false>, grid, block, 0, stream, x, codes, scales, tokens, hidden, split);
     return hipGetLastError();
 }
 
 hipError_t launch_dequantize(const uint8_t* codes, const float* scales, uint16_t* out, int tokens, int hidden, hipStream_t stream) {
     if (tokens <= 0) return hipSuccess;
-    const dim3 grid(row_grid(tokens)), block(kRowKernelThreads);
-    if (hidden % 16 == 0) hipLaunchKernelGGL(dequantize_kernel<true>, grid, block, 0, stream, codes, scales, out, tokens, hidden);
-    else hipLaunchKernelGGL(dequantize_kernel<false>, grid, block, 0, stream, codes, scales, out, tokens, hidden);
+    const int split = codec_split(hidden), rows = kCodecWaves / split;
+    const dim3 grid(unsigned((int64_t(tokens) + rows - 1) / rows)), block(kRowKernelThreads);
+    if (codec_vector(out, codes, hidden)) hipLaunchKernelGGL(dequantize_kernel<true>, grid, block, 0, stream, codes, scales, out, tokens, hidden, split);
+    else hipLaunchKernelGGL(dequantize_kernel<false>, grid, block, 0, stream, codes, scales, out, tokens, hidden, split);
     return hipGetLastError();
 }
 

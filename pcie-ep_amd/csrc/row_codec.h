@@ -30,13 +30,7 @@ __device__ __forceinline__ void copy_row(const uint16_t* input, uint16_t* output
     }
 }
 
-// Where a quantised row goes: device memory, or a host slot through buffer
-// stores with the system-scope cache policy.
-struct DeviceCodes {
-    uint8_t* output;
-    __device__ __forceinline__ void vector(int group, u32x4 codes) const { reinterpret_cast<u32x4*>(output)[group] = codes; }
-    __device__ __forceinline__ void single(int index, uint8_t code) const { output[index] = code; }
-};
+// Where a quantised row goes: a host slot through buffer stores with the system-scope cache policy.
 struct HostCodes {
     __amdgpu_buffer_rsrc_t slot;
     __device__ __forceinline__ void vector(int group, u32x4 codes) const { host_store_b128(slot, uint32_t(group) * 16u, codes); }
@@ -63,6 +57,14 @@ __device__ __forceinline__ void copy_row_to_host(const uint16_t* input, __amdgpu
     }
 }
 
+__device__ __forceinline__ float vector_amax(float amax, const u32x4& v) {
+#pragma unroll
+    for (int word = 0; word < 4; ++word) {
+        amax = fmaxf(amax, fabsf(bits_float(v[word] << 16)));
+        amax = fmaxf(amax, fabsf(bits_float(v[word] & 0xFFFF0000u)));
+    }
+    return amax;
+}
 // Returns the row scale.  kVector requires hidden % 16 == 0.
 template <bool kVector, typename Sink>
 __device__ __forceinline__ float quantize_row(const uint16_t* input, const Sink& sink, int hidden, int lane) {
@@ -122,23 +124,6 @@ __device__ __forceinline__ void dequantize_vector(const u32x4& codes, float scal
             hi[(word - 2) * 2] = a;
             hi[(word - 2) * 2 + 1] = b;
         }
-    }
-}
-
-template <bool kVector>
-__device__ __forceinline__ void dequantize_row(const uint8_t* codes, float scale, uint16_t* output, int hidden, int lane) {
-    if constexpr (kVector) {
-        const int groups = hidden / 16;
-        const u32x4* source = reinterpret_cast<const u32x4*>(codes);
-        u32x4* destination = reinterpret_cast<u32x4*>(output);
-        for (int group = lane; group < groups; group += kWave) {
-            u32x4 lo, hi;
-            dequantize_vector(source[group], scale, lo, hi);
-            destination[group * 2] = lo;
-            destination[group * 2 + 1] = hi;
-        }
-    } else {
-        for (int index = lane; index < hidden; index += kWave) output[index] = fp8_dequantize_element(codes[index], scale);
     }
 }
 

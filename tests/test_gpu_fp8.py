@@ -66,6 +66,28 @@ def test_quantize_kernel_all_bf16_bit_patterns():
     assert torch.equal(codes.cpu(), want_codes)
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("hidden", [1, 7, 8, 15, 2047, 2048, 2056, 4096, 4097, 8192, 8193, 20000])
+def test_codec_splits_rests_and_unaligned_arrays(hidden, offset):
+    """One, two and four wavefronts per row, rows of one pass and of several, 0 to 7 elements behind
+    the whole vectors, a row count that leaves wavefronts of the last workgroup without a row, and
+    arrays that start in the middle of a vector.  Bytes, scales and decoded values are exact."""
+    from pcie_ep.quantization import dequantize_fp8, quantize_fp8
+
+    tokens = 7
+    x = _heavy_tailed(tokens, hidden, 23)
+    x[3] = 0
+    device = torch.zeros(offset + x.numel(), dtype=torch.bfloat16, device="cuda")
+    device[offset:] = x.flatten().cuda()
+    codes, scales = quantize_fp8(device[offset:].view(tokens, hidden))
+    want_codes, want_scales = fp8_oracle.quantize(x)
+    assert torch.equal(scales.cpu().view(torch.int32), want_scales.view(torch.int32)) and torch.equal(codes.cpu(), want_codes)
+    shifted = torch.zeros(offset + x.numel(), dtype=torch.uint8, device="cuda")
+    shifted[offset:] = codes.flatten()
+    decoded = dequantize_fp8(shifted[offset:].view(tokens, hidden), scales).cpu()
+    assert torch.equal(decoded.view(torch.int16), fp8_oracle.dequantize(want_codes, want_scales).view(torch.int16))
+
+
 @pytest.mark.parametrize("hidden,channels", [(7168, 8), (136, 2), (129, 2)])
 def test_fp8_wire_dispatch(hidden, channels):
     world, experts, topk = 8, 256, 8
