@@ -365,18 +365,6 @@ __device__ __forceinline__ uint32_t host_load_b32(__amdgpu_buffer_rsrc_t resourc
 __device__ __forceinline__ void host_store_b32(__amdgpu_buffer_rsrc_t resource, uint32_t byte_offset, uint32_t value) {
     __builtin_amdgcn_raw_buffer_store_b32(value, resource, int(byte_offset), 0, kHostPolicy);
 }
-__device__ __forceinline__ uint16_t host_load_b16(__amdgpu_buffer_rsrc_t resource, uint32_t byte_offset) {
-    return __builtin_amdgcn_raw_buffer_load_b16(resource, int(byte_offset), 0, kHostPolicy);
-}
-__device__ __forceinline__ void host_store_b16(__amdgpu_buffer_rsrc_t resource, uint32_t byte_offset, uint16_t value) {
-    __builtin_amdgcn_raw_buffer_store_b16(value, resource, int(byte_offset), 0, kHostPolicy);
-}
-__device__ __forceinline__ uint8_t host_load_b8(__amdgpu_buffer_rsrc_t resource, uint32_t byte_offset) {
-    return __builtin_amdgcn_raw_buffer_load_b8(resource, int(byte_offset), 0, kHostPolicy);
-}
-__device__ __forceinline__ void host_store_b8(__amdgpu_buffer_rsrc_t resource, uint32_t byte_offset, uint8_t value) {
-    __builtin_amdgcn_raw_buffer_store_b8(value, resource, int(byte_offset), 0, kHostPolicy);
-}
 template <typename T>
 __device__ __forceinline__ T host_field_load(const T* address) {
     return __hip_atomic_load(address, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -624,14 +612,6 @@ __device__ __forceinline__ void row_store_vectors(const RowVectors& row, u32x4* 
         }
     }
 }
-
-// Scalar fall-back for rows whose byte length is not a multiple of 16: the
-// same structure with 2-byte items (the reference also falls back to scalar
-// copies for such hidden sizes: csrc/kernels/host_staged/fused_receive.cuh:116-126).
-constexpr int kPassScalars = 32;
-struct RowScalars {
-    uint16_t v[kPassScalars];
-};
 
 // Rows that are not whole 16-byte vectors: the whole vectors move as above, from and to
 // any address (unaligned 16-byte accesses to device memory are one instruction like aligned

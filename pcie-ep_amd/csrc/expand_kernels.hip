@@ -18,8 +18,8 @@ namespace {
 // Stand-alone expand: unique rows -> expert-major rows (dispatch.cuh:8-65).
 // Algorithmic HBM traffic: unique_count rows read + expanded_count rows written
 // (+ 36 bytes of row metadata per expanded row).
-// This version serves rows that are not whole 16-byte vectors (2-byte items,
-// one wavefront per row); expand_pieces_kernel below is the one for vector rows.
+// This version serves rows that are not whole 16-byte vectors (the ragged form of
+// the row code, one wavefront per row); expand_pieces_kernel below is the one for vector rows.
 __global__ void __launch_bounds__(kRowKernelThreads) expand_rows_kernel(DeviceState state) {
     if (load_error_code(state)) return;
     const SegmentLayout& z = state.z;

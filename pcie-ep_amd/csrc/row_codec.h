@@ -13,48 +13,40 @@ __device__ __forceinline__ float wave_max(float value) {
     return value;
 }
 
-// BF16 row copy.  kVector requires hidden % 8 == 0 and 16-byte aligned rows.
-template <bool kVector, bool kStreamOut>
+// A row helper's kVector says that the row is whole 16-byte vectors on 16-byte
+// boundaries (hidden % 8 == 0; of 16-code vectors too where it goes over the FP8 wire:
+// hidden % 16 == 0).  Any other row takes the ragged form of the same code.
+
+// BF16 row copy within device memory.
+template <bool kVector>
 __device__ __forceinline__ void copy_row(const uint16_t* input, uint16_t* output, int hidden, int lane) {
-    if constexpr (kVector) {
-        const int vectors = hidden / 8;
-        const u32x4* source = reinterpret_cast<const u32x4*>(input);
-        u32x4* destination = reinterpret_cast<u32x4*>(output);
-        for (int first = 0; first < vectors; first += kPassItems * kWave) {
-            RowVectors row;
-            row_load_vectors<true>(row, source, first, vectors, lane);
-            row_store_vectors<kStreamOut>(row, destination, first, vectors, lane);
-        }
-    } else {
-        for (int index = lane; index < hidden; index += kWave) output[index] = input[index];
+    const int vectors = hidden / 8, rest = row_rest<kVector>(hidden);
+    for (int first = 0; first < vectors; first += kPassItems * kWave) {
+        RowVectors row;
+        row_load_pass<kVector>(row, input, first, vectors, lane);
+        row_store_pass<kVector>(row, output, first, vectors, lane);
     }
+    if (rest && lane == 0)
+        store_rest(reinterpret_cast<char*>(output + vectors * 8), rest, load_rest(reinterpret_cast<const char*>(input + vectors * 8), rest));
 }
 
-// Where a quantised row goes: a host slot through buffer stores with the system-scope cache policy.
-struct HostCodes {
-    __amdgpu_buffer_rsrc_t slot;
-    __device__ __forceinline__ void vector(int group, u32x4 codes) const { host_store_b128(slot, uint32_t(group) * 16u, codes); }
-    __device__ __forceinline__ void single(int index, uint8_t code) const { host_store_b8(slot, uint32_t(index), code); }
-};
-
-// BF16 row from device memory into a host slot.
+// BF16 row from device memory into a host slot.  A ragged row's last vector is stored
+// whole, zeros behind the row: the slot's payload is padded to 16 bytes.
 template <bool kVector>
 __device__ __forceinline__ void copy_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane) {
-    if constexpr (kVector) {
-        const int vectors = hidden / 8;
-        const u32x4* source = reinterpret_cast<const u32x4*>(input);
-        for (int first = 0; first < vectors; first += kPassItems * kWave) {
-            RowVectors row;
-            row_load_vectors<true>(row, source, first, vectors, lane);
+    const int vectors = hidden / 8, rest = row_rest<kVector>(hidden);
+    u32x4 last = {0u, 0u, 0u, 0u};
+    if (rest && lane == 0) last = load_rest(reinterpret_cast<const char*>(input + vectors * 8), rest);
+    for (int first = 0; first < vectors; first += kPassItems * kWave) {
+        RowVectors row;
+        row_load_pass<kVector>(row, input, first, vectors, lane);
 #pragma unroll
-            for (int j = 0; j < kPassItems; ++j) {
-                const int index = first + j * kWave + lane;
-                if (index < vectors) host_store_b128(slot, uint32_t(index) * 16u, row.v[j]);
-            }
+        for (int j = 0; j < kPassItems; ++j) {
+            const int index = first + j * kWave + lane;
+            if (index < vectors) host_store_b128(slot, uint32_t(index) * 16u, row.v[j]);
         }
-    } else {
-        for (int index = lane; index < hidden; index += kWave) host_store_b16(slot, uint32_t(index) * 2u, input[index]);
     }
+    if (rest && lane == 0) host_store_b128(slot, uint32_t(vectors) * 16u, last);
 }
 
 __device__ __forceinline__ float vector_amax(float amax, const u32x4& v) {
@@ -65,48 +57,63 @@ __device__ __forceinline__ float vector_amax(float amax, const u32x4& v) {
     }
     return amax;
 }
-// Returns the row scale.  kVector requires hidden % 16 == 0.
-template <bool kVector, typename Sink>
-__device__ __forceinline__ float quantize_row(const uint16_t* input, const Sink& sink, int hidden, int lane) {
-    // Sweep 1: row amax in FP32.  Sweep 2 re-reads the row (it is L2 resident).
+// 16 BF16 (two vectors, elements in order) -> 16 codes.
+__device__ __forceinline__ u32x4 quantize_vector(const u32x4& lo, const u32x4& hi, float inverse) {
+    return u32x4{fp8_quantize_word(lo[0], lo[1], inverse), fp8_quantize_word(lo[2], lo[3], inverse), fp8_quantize_word(hi[0], hi[1], inverse),
+                 fp8_quantize_word(hi[2], hi[3], inverse)};
+}
+
+// BF16 row from device memory as FP8 codes into a host slot; returns the row scale.  Every
+// lane takes 16 elements (two 16-byte loads) at a time to 16 codes (one 16-byte store).
+// A row of up to 8192 elements is read once and waits in registers for its maximum.  A
+// ragged row's last codes are stored as a whole vector, zeros behind the row.
+template <bool kVector>
+__device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane) {
+    constexpr int kGroups = kPassItems / 2;  // 16-element groups a lane holds
+    const int groups = hidden / 16, rest = kVector ? 0 : hidden % 16 * 2;
     float amax = 0.0f;
-    if constexpr (kVector) {
-        const int vectors = hidden / 8;
-        const u32x4* source = reinterpret_cast<const u32x4*>(input);
-        for (int index = lane; index < vectors; index += kWave) {
-            const u32x4 v = source[index];
+    u32x4 last_lo = {0u, 0u, 0u, 0u}, last_hi = {0u, 0u, 0u, 0u};
+    if (rest && lane == 0) {
+        const char* from = reinterpret_cast<const char*>(input + groups * 16);
+        last_lo = rest < 16 ? load_rest(from, rest) : *reinterpret_cast<const u32x4_any*>(from);
+        if (rest > 16) last_hi = load_rest(from + 16, rest - 16);
+        amax = vector_amax(vector_amax(amax, last_lo), last_hi);
+    }
+    RowVectors row;
+    const bool resident = groups <= kGroups * kWave;
+    if (resident) {
 #pragma unroll
-            for (int word = 0; word < 4; ++word) {
-                amax = fmaxf(amax, fabsf(bf16_to_float(uint16_t(v[word] & 0xFFFFu))));
-                amax = fmaxf(amax, fabsf(bf16_to_float(uint16_t(v[word] >> 16))));
+        for (int j = 0; j < kGroups; ++j) {
+            const int group = j * kWave + lane;
+            row.v[2 * j] = row.v[2 * j + 1] = u32x4{0u, 0u, 0u, 0u};
+            if (group < groups) {
+                row.v[2 * j] = row_load_vector<kVector>(input, 2 * group);
+                row.v[2 * j + 1] = row_load_vector<kVector>(input, 2 * group + 1);
             }
         }
+#pragma unroll
+        for (int j = 0; j < kPassItems; ++j) amax = vector_amax(amax, row.v[j]);
     } else {
-        for (int index = lane; index < hidden; index += kWave) amax = fmaxf(amax, fabsf(bf16_to_float(input[index])));
+        for (int index = lane; index < groups * 2; index += kWave) amax = vector_amax(amax, row_load_vector<false>(input, index));
     }
     amax = wave_max(amax);
     const float scale = fp8_scale_from_amax(amax);
     // Multiply by the correctly rounded FP32 reciprocal, as the reference does
     // (quantization.cuh:66; pcie_ep/quantization.py:27-29), not a division per element.
     const float inverse = 1.0f / scale;
-    if constexpr (kVector) {
-        // 16 elements (two 16-byte loads) -> 16 codes (one 16-byte store) per lane.
-        const int groups = hidden / 16;
-        const u32x4* source = reinterpret_cast<const u32x4*>(input);
-        for (int group = lane; group < groups; group += kWave) {
-            const u32x4 lo = source[group * 2], hi = source[group * 2 + 1];
-            u32x4 codes;
+    if (resident) {
 #pragma unroll
-            for (int word = 0; word < 4; ++word) {
-                const uint32_t a = word < 2 ? lo[word * 2] : hi[(word - 2) * 2];
-                const uint32_t b = word < 2 ? lo[word * 2 + 1] : hi[(word - 2) * 2 + 1];
-                codes[word] = fp8_quantize_word(a, b, inverse);
-            }
-            sink.vector(group, codes);
+        for (int j = 0; j < kGroups; ++j) {
+            const int group = j * kWave + lane;
+            if (group < groups) host_store_b128(slot, uint32_t(group) * 16u, quantize_vector(row.v[2 * j], row.v[2 * j + 1], inverse));
         }
     } else {
-        for (int index = lane; index < hidden; index += kWave) sink.single(index, fp8_quantize_element(input[index], inverse));
+        for (int group = lane; group < groups; group += kWave) {
+            const u32x4 lo = row_load_vector<false>(input, 2 * group), hi = row_load_vector<false>(input, 2 * group + 1);
+            host_store_b128(slot, uint32_t(group) * 16u, quantize_vector(lo, hi, inverse));
+        }
     }
+    if (rest && lane == 0) host_store_b128(slot, uint32_t(groups) * 16u, quantize_vector(last_lo, last_hi, inverse));
     return scale;
 }
 
@@ -127,58 +134,36 @@ __device__ __forceinline__ void dequantize_vector(const u32x4& codes, float scal
     }
 }
 
-// Store one BF16 row (already read into registers pass by pass) to every
+// Store one BF16 row (read once, into registers, pass by pass) to every
 // destination row named by the lanes whose `my_row >= 0`.
 template <bool kVector>
 __device__ __forceinline__ void scatter_row(const uint16_t* input, uint16_t* output_base, int hidden, int64_t my_row, int lane) {
     const uint64_t destinations = __ballot(my_row >= 0);
     if (!destinations) return;
-    if constexpr (kVector) {
-        const int vectors = hidden / 8;
-        const u32x4* source = reinterpret_cast<const u32x4*>(input);
-        for (int first = 0; first < vectors; first += kPassItems * kWave) {
-            RowVectors row;
-            row_load_vectors<true>(row, source, first, vectors, lane);
-            uint64_t remaining = destinations;
-            while (remaining) {
-                const int owner = __builtin_ctzll(remaining);
-                remaining &= remaining - 1;
-                const int64_t out_row = __shfl(my_row, owner);
-                row_store_vectors<true>(row, reinterpret_cast<u32x4*>(output_base + size_t(out_row) * hidden), first, vectors, lane);
-            }
-        }
-    } else {
-        for (int first = 0; first < hidden; first += kPassScalars * kWave) {
-            RowScalars items;
-#pragma unroll
-            for (int j = 0; j < kPassScalars; ++j) {
-                const int index = first + j * kWave + lane;
-                if (index < hidden) items.v[j] = input[index];
-            }
-            uint64_t remaining = destinations;
-            while (remaining) {
-                const int owner = __builtin_ctzll(remaining);
-                remaining &= remaining - 1;
-                uint16_t* output = output_base + size_t(__shfl(my_row, owner)) * hidden;
-#pragma unroll
-                for (int j = 0; j < kPassScalars; ++j) {
-                    const int index = first + j * kWave + lane;
-                    if (index < hidden) output[index] = items.v[j];
-                }
-            }
+    const int vectors = hidden / 8, rest = row_rest<kVector>(hidden);
+    u32x4 last = {0u, 0u, 0u, 0u};
+    if (rest && lane == 0) last = load_rest(reinterpret_cast<const char*>(input + vectors * 8), rest);
+    // Also a row shorter than one vector takes one pass, for its rest.
+    for (int first = 0; first == 0 || first < vectors; first += kPassItems * kWave) {
+        RowVectors row;
+        row_load_pass<kVector>(row, input, first, vectors, lane);
+        uint64_t remaining = destinations;
+        while (remaining) {
+            const int owner = __builtin_ctzll(remaining);
+            remaining &= remaining - 1;
+            uint16_t* output = output_base + size_t(__shfl(my_row, owner)) * hidden;
+            row_store_pass<kVector>(row, output, first, vectors, lane);
+            if (rest && first == 0 && lane == 0) store_rest(reinterpret_cast<char*>(output + vectors * 8), rest, last);
         }
     }
 }
 
 template <bool kVector>
 __device__ __forceinline__ void zero_row(uint16_t* output, int hidden, int lane) {
-    if constexpr (kVector) {
-        u32x4* destination = reinterpret_cast<u32x4*>(output);
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-        for (int index = lane; index < hidden / 8; index += kWave) __builtin_nontemporal_store(zero, destination + index);
-    } else {
-        for (int index = lane; index < hidden; index += kWave) output[index] = 0;
-    }
+    const int vectors = hidden / 8, rest = row_rest<kVector>(hidden);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    for (int index = lane; index < vectors; index += kWave) row_store_vector<kVector>(output, index, zero);
+    if (rest && lane == 0) store_rest(reinterpret_cast<char*>(output + vectors * 8), rest, zero);
 }
 
 // Alignment gaps of the local experts, rows [offset + count, next offset) of each:
@@ -261,7 +246,7 @@ __device__ __forceinline__ bool local_token_rows(const DeviceState& state, int t
         }
     } else {
         const int64_t row = int64_t(device_load(state.source_offsets + me)) + state.plan_rank_ord[size_t(token) * ranks + me];
-        copy_row<kVector, true>(input, state.unique_payload + size_t(row) * hidden, hidden, lane);
+        copy_row<kVector>(input, state.unique_payload + size_t(row) * hidden, hidden, lane);
         if (lane < topk) {
             state.unique_topk_idx[row * topk + lane] = is_local ? expert : -1;
             state.unique_topk_weights[row * topk + lane] = is_local ? weight : 0.0f;

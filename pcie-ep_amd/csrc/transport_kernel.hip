@@ -900,7 +900,7 @@ __device__ __forceinline__ void finish_role(const DeviceState& state, TransportQ
 template <bool kFp8, bool kVector>
 __device__ __forceinline__ float tx_copy_row(const DeviceState& state, const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int lane) {
     const int hidden = state.z.dims.hidden;
-    if constexpr (kFp8) return quantize_row<kVector>(input, HostCodes{slot}, hidden, lane);
+    if constexpr (kFp8) return quantize_row_to_host<kVector>(input, slot, hidden, lane);
     copy_row_to_host<kVector>(input, slot, hidden, lane);
     return 1.0f;
 }
@@ -986,7 +986,7 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         if (lane == kWave - 1) test_delay(state.tx_delay);
         const __amdgpu_buffer_rsrc_t slot_resource = host_resource(slot_base, uint32_t(z.meta_offset + z.meta_bytes));
         const float scale = tx_copy_row<kFp8, kVector>(state, state.x + size_t(token) * z.dims.hidden,
-                                                       host_resource(slot_base, uint32_t(z.payload_bytes)), lane);
+                                                       host_resource(slot_base, uint32_t(z.meta_offset)), lane);
         if (lane == 0) scratch[2] = float_bits(scale);
         fence_lds();
         if (lane == meta_dwords - 1 || (lane == kWave - 1 && meta_dwords > kWave)) test_delay(state.metadata_delay);
@@ -1045,7 +1045,8 @@ __device__ __forceinline__ bool rx_row(const DeviceState& state, TransportQueues
         const char* slot_base = replica ? replica_slot_at(z, state.replica_in[source], channel, slot) : slot_at(z, state.seg[source], channel, slot);
         uint64_t* slot_ack = replica ? replica_ack_at(z, state.seg[source], channel, z.dims.rank_domain[me], slot, me)
                                      : ack_at(z, state.seg[source], channel, slot, me);
-        const __amdgpu_buffer_rsrc_t payload = host_resource(slot_base, uint32_t(z.payload_bytes));
+        // A ragged row's last wire vector is read whole: the slot's payload is padded to 16 bytes, the padding is not used.
+        const __amdgpu_buffer_rsrc_t payload = host_resource(slot_base, uint32_t(z.meta_offset));
         const __amdgpu_buffer_rsrc_t slot_meta = host_resource(slot_base + z.meta_offset, uint32_t(z.meta_bytes));
         if (lane == kWave - 1) test_delay(state.rx_delay);
         // Tickets are handed out from the first descriptor on, but no row is requested
@@ -1088,19 +1089,18 @@ __device__ __forceinline__ bool rx_row(const DeviceState& state, TransportQueues
         // Metadata first (it arrives first), payload right behind it.
         const u32x4 meta_vector = host_load_b128(slot_meta, uint32_t(lane) * 16u);  // 16 bytes per lane; out of range reads as 0
 
+        // Whole wire vectors of the row, and with a ragged row (any length and any alignment of the destination rows:
+        // one more wire vector, of which `rest` bytes of BF16 are stored).  Byte by byte such a row was one host read
+        // and one store per element: 1536 tokens of 1000 columns on the FP8 wire, 8 ranks, top-4: 609 -> 315 us per dispatch.
         RowVectors row;
         const int wire_vectors = kFp8 ? hidden / 16 : hidden / 8;
-        const int wire_per_pass = kFp8 ? (kPassItems / 2) * kWave : kPassItems * kWave;
-        if constexpr (kVector) {
-            // First (usually only) pass of the row.
-            if constexpr (kFp8) {
+        const int rest = kVector ? 0 : (kFp8 ? hidden % 16 : hidden % 8) * 2;
+        const int wire_total = wire_vectors + (rest ? 1 : 0);
+        constexpr int kWireItems = kFp8 ? kPassItems / 2 : kPassItems;  // a code vector fills two BF16 vectors
+        constexpr int kWirePass = kWireItems * kWave;
+        // First (usually only) pass of the row; lanes behind the row read 0.
 #pragma unroll
-                for (int j = 0; j < kPassItems / 2; ++j) row.v[j] = host_load_b128(payload, uint32_t(j * kWave + lane) * 16u);
-            } else {
-#pragma unroll
-                for (int j = 0; j < kPassItems; ++j) row.v[j] = host_load_b128(payload, uint32_t(j * kWave + lane) * 16u);
-            }
-        }
+        for (int j = 0; j < kWireItems; ++j) row.v[j] = host_load_b128(payload, uint32_t(j * kWave + lane) * 16u);
         PCIE_EP_PROFILE(profile.first(kProfileFirstRequestNs);)
         if (lane < kScratchDwords / 4) {
             scratch[lane * 4] = meta_vector[0];
@@ -1183,80 +1183,65 @@ __device__ __forceinline__ bool rx_row(const DeviceState& state, TransportQueues
         uint16_t* output_base = scatter ? state.expanded_payload : state.unique_payload;
         if (lane == kWave - 1) test_delay(state.scatter_delay);
 
-        if constexpr (kVector) {
-            const int out_vectors = hidden / 8;
-            for (int first_wire = 0; first_wire < wire_vectors; first_wire += wire_per_pass) {
-                if (first_wire > 0) {
-                    if constexpr (kFp8) {
+        for (int first_wire = 0; first_wire < wire_total; first_wire += kWirePass) {
+            if (first_wire > 0) {
 #pragma unroll
-                        for (int j = 0; j < kPassItems / 2; ++j) row.v[j] = host_load_b128(payload, uint32_t(first_wire + j * kWave + lane) * 16u);
-                    } else {
+                for (int j = 0; j < kWireItems; ++j) row.v[j] = host_load_b128(payload, uint32_t(first_wire + j * kWave + lane) * 16u);
+            }
+            const bool last_pass = first_wire + kWirePass >= wire_total;
+            if (last_pass) {
+                // All loads of the staged row have returned: release the host slot.
+                if (lane == 0) host_store_release(slot_ack, payload_sequence);
+                PCIE_EP_PROFILE(if (sampled) { wait_memory_ops(); profile.add(kProfileRxRequestSum, profile.now() - request_begin); })
+            }
+            if constexpr (kFp8) {
+                // 16 codes -> 16 BF16 (two 16-byte vectors); expanded in place from the top.
 #pragma unroll
-                        for (int j = 0; j < kPassItems; ++j) row.v[j] = host_load_b128(payload, uint32_t(first_wire + j * kWave + lane) * 16u);
-                    }
-                }
-                const bool last_pass = first_wire + wire_per_pass >= wire_vectors;
-                if (last_pass) {
-                    // All loads of the staged row have returned: release the host slot.
-                    if (lane == 0) host_store_release(slot_ack, payload_sequence);
-                    PCIE_EP_PROFILE(if (sampled) { wait_memory_ops(); profile.add(kProfileRxRequestSum, profile.now() - request_begin); })
-                }
-                if constexpr (kFp8) {
-                    // 16 codes -> 16 BF16 (two 16-byte vectors); expanded in place from the top.
-#pragma unroll
-                    for (int j = kPassItems / 2 - 1; j >= 0; --j) {
-                        u32x4 lo, hi;
-                        dequantize_vector(row.v[j], scale, lo, hi);
-                        row.v[2 * j] = lo;
-                        row.v[2 * j + 1] = hi;
-                    }
-                }
-                uint64_t remaining = destinations;
-                while (remaining) {
-                    const int branch = __builtin_ctzll(remaining);
-                    remaining &= remaining - 1;
-                    const int64_t out_row = __shfl(my_row, branch);
-                    u32x4* output = reinterpret_cast<u32x4*>(output_base + size_t(out_row) * hidden);
-                    if constexpr (kFp8) {
-                        // Wire vector i holds elements [16 i, 16 i + 16) -> output vectors 2 i and 2 i + 1.
-#pragma unroll
-                        for (int j = 0; j < kPassItems / 2; ++j) {
-                            const int index = first_wire + j * kWave + lane;
-                            if (index < wire_vectors) {
-                                __builtin_nontemporal_store(row.v[2 * j], output + 2 * index);
-                                __builtin_nontemporal_store(row.v[2 * j + 1], output + 2 * index + 1);
-                            }
-                        }
-                    } else {
-                        row_store_vectors<true>(row, output, first_wire, out_vectors, lane);
-                    }
+                for (int j = kWireItems - 1; j >= 0; --j) {
+                    u32x4 lo, hi;
+                    dequantize_vector(row.v[j], scale, lo, hi);
+                    row.v[2 * j] = lo;
+                    row.v[2 * j + 1] = hi;
                 }
             }
-        } else {
-            // Scalar fall-back (row length not a multiple of 16 bytes): 2-byte items.
-            for (int first = 0; first < hidden; first += kPassScalars * kWave) {
-                RowScalars items;
+            // The ragged row's last wire vector is item (wire_vectors - first_wire) / 64 of lane wire_vectors % 64.
+            constexpr int kOutPerWire = kFp8 ? 2 : 1;
+            u32x4 last[kOutPerWire] = {};
+            if (!kVector && rest && last_pass) {
+                const int item = (wire_vectors - first_wire) / kWave;
 #pragma unroll
-                for (int j = 0; j < kPassScalars; ++j) {
-                    const int index = first + j * kWave + lane;
-                    if (index < hidden) {
-                        if constexpr (kFp8) items.v[j] = fp8_dequantize_element(host_load_b8(payload, uint32_t(index)), scale);
-                        else items.v[j] = host_load_b16(payload, uint32_t(index) * 2u);
+                for (int j = 0; j < kWireItems; ++j) {
+                    if (j != item) continue;
+#pragma unroll
+                    for (int half = 0; half < kOutPerWire; ++half) last[half] = row.v[j * kOutPerWire + half];
+                }
+            }
+            uint64_t remaining = destinations;
+            while (remaining) {
+                const int branch = __builtin_ctzll(remaining);
+                remaining &= remaining - 1;
+                uint16_t* output = output_base + size_t(__shfl(my_row, branch)) * hidden;
+#pragma unroll
+                for (int j = 0; j < kWireItems; ++j) {
+                    const int index = first_wire + j * kWave + lane;
+                    if (index < wire_vectors) {
+                        // Wire vector i of an FP8 row holds elements [16 i, 16 i + 16): output vectors 2 i and 2 i + 1.
+#pragma unroll
+                        for (int half = 0; half < kOutPerWire; ++half)
+                            row_store_vector<kVector>(output, index * kOutPerWire + half, row.v[j * kOutPerWire + half]);
                     }
                 }
-                if (first + kPassScalars * kWave >= hidden) {
-                    if (lane == 0) host_store_release(slot_ack, payload_sequence);
-                }
-                uint64_t remaining = destinations;
-                while (remaining) {
-                    const int branch = __builtin_ctzll(remaining);
-                    remaining &= remaining - 1;
-                    const int64_t out_row = __shfl(my_row, branch);
-                    uint16_t* output = output_base + size_t(out_row) * hidden;
-#pragma unroll
-                    for (int j = 0; j < kPassScalars; ++j) {
-                        const int index = first + j * kWave + lane;
-                        if (index < hidden) output[index] = items.v[j];
+                if (!kVector && rest && last_pass && lane == wire_vectors % kWave) {
+                    char* tail = reinterpret_cast<char*>(output) + size_t(wire_vectors) * (kOutPerWire * 16);
+                    if constexpr (kFp8) {
+                        if (rest >= 16) {
+                            row_store_vector<false>(tail, 0, last[0]);
+                            store_rest(tail + 16, rest - 16, last[1]);
+                        } else {
+                            store_rest(tail, rest, last[0]);
+                        }
+                    } else {
+                        store_rest(tail, rest, last[0]);
                     }
                 }
             }
@@ -1592,8 +1577,8 @@ hipError_t launch_transport(const DeviceState& state, hipStream_t stream) {
         dynamic_lds = prologue_lds_bytes(state.z, int(block.x) / kWave);
     }
     const bool fp8 = state.z.dims.wire_fp8 != 0;
-    // BF16 rows need 16-byte granularity on both sides; FP8 additionally needs
-    // whole 16-code vectors on the wire.
+    // Rows of whole 16-byte vectors on both sides (FP8: of whole 16-code vectors on the wire) lie on 16-byte
+    // boundaries and have nothing behind their vectors; all others take the ragged form of the row code.
     const bool vector = fp8 ? state.z.dims.hidden % 16 == 0 : state.z.dims.hidden % 8 == 0;
     if (fp8 && vector) hipLaunchKernelGGL((transport_kernel<true, true>), grid, block, dynamic_lds, stream, state);
     else if (fp8) hipLaunchKernelGGL((transport_kernel<true, false>), grid, block, dynamic_lds, stream, state);

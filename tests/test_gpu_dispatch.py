@@ -190,6 +190,32 @@ def test_alignment_gaps_of_small_batches(world, experts, alignment, hidden, fuse
         check_case(buffer, "gaps-empty", [0] * world, alignment=alignment, seed=9, capture=world > 1)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hidden", [1, 7, 9, 15, 1000, 1001, 8190, 8197])
+def test_ragged_rows(hidden, fp8):
+    """Rows with something behind their whole vectors, on either wire: 1 to 15 bytes, rows shorter than a
+    vector, the rest in the last item of a pass (8190) and alone in a pass of its own (8197, FP8); expanded
+    while receiving, by the expand kernel and not at all, with cleared gap rows between the rows; own
+    tokens that start in the middle of a vector."""
+    wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
+    for mode in ({}, {"fuse_receive_expand": False, "receive_expand_mode": "scalar"}):
+        with make_buffer(world=4, tmax=23, hidden=hidden, topk=4, experts=16, channels=2, payload_slots=3, descriptor_slots=3, **wire, **mode) as buffer:
+            check_case(buffer, f"ragged-h{hidden}", [23, 17, 0, 5], alignment=16, fp8=fp8)
+            if mode:
+                continue
+            check_case(buffer, f"ragged-h{hidden}-unique", [23, 17, 0, 5], expand=False, seed=9, fp8=fp8)
+            inputs = make_inputs(4, [23, 1, 20, 23], hidden, 16, 4, "random", seed=10, gaussian=fp8)
+            x, idx, weights = inputs[0]
+            flat = torch.zeros(1 + x.numel(), dtype=torch.bfloat16, device="cuda")
+            flat[1:] = x.flatten().cuda()
+            if hidden % 8:
+                shifted = [(flat[1:].view(x.shape), idx.cuda(), weights.cuda())] + inputs[1:]
+                result, _ = run_dispatch(buffer, shifted, expand=True, capture=True)
+                verify_dispatch(result, inputs, 0, 4, 16, 4, True, 1, False, fp8_wire=fp8)
+                verify_captured(buffer.peers, inputs, 0, 4, 16, 4, fp8_wire=fp8)
+                del result
+
+
 def test_numa_bound_staging_segments():
     """The pinned segments can be bound to a NUMA node (the far-node staging of the
     cached-replay configuration); node 0 exists on every box.  Results do not change."""
