@@ -34,13 +34,12 @@ class GraphDispatch:
         self._generation = owner._generation
         self._frozen = tuple(memory_signature(t) if t is not None else None for t in request.inputs)
         self._open = True
-        # The instantiated graph is launched on the communication stream directly
-        # (torch's own replay launches on the current stream, and making the
-        # communication stream current around every replay is a measurable part of
-        # a small replay's CPU time).
+        # The instantiated graph is launched directly on the stream that the dispatch
+        # is to run on (torch's own replay launches on the current stream, and making
+        # another stream current around every replay is a measurable part of a small
+        # replay's CPU time).
         self._exec = C.c_void_p(int(graph.raw_cuda_graph_exec()))
         self._launch_exec = _native.library().pcie_ep_graph_launch
-        self._raw_stream = C.c_void_p(int(owner.get_comm_stream().cuda_stream))
 
     # The captured inputs under the reference's attribute names.
     x = property(lambda self: self._request.x)
@@ -66,11 +65,11 @@ class GraphDispatch:
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("GraphDispatch.replay cannot be nested in another capture")
 
-            def replayed() -> Dict[str, Any]:
-                _native.check(self._launch_exec(self._exec, self._raw_stream), invalid=RuntimeError)
+            def replayed(stream: int) -> Dict[str, Any]:
+                _native.check(self._launch_exec(self._exec, C.c_void_p(stream)), invalid=RuntimeError)
                 return self._result
 
-            return owner._launch(self._request, replayed, (self,), previous_event, async_with_compute_stream, through_torch=False)
+            return owner._launch(self._request, replayed, (self,), previous_event, async_with_compute_stream)
 
     def close(self) -> None:
         if self._open:
@@ -102,7 +101,7 @@ def capture_dispatch(owner: Any, x: torch.Tensor, topk_idx: Optional[torch.Tenso
         except Exception as error:
             raise collective("preparation", error) from error
         graph = torch.cuda.CUDAGraph()
-        stream = owner.get_comm_stream()
+        stream = owner._ordering.stream
         try:
             with torch.cuda.stream(stream):
                 record_tensors(request.inputs, stream)

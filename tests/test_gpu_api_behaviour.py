@@ -136,6 +136,48 @@ def test_previous_event_orders_the_dispatch_after_a_side_stream(inputs):
         assert buffer.get_comm_stream() is not torch.cuda.current_stream()
 
 
+def test_synchronous_dispatches_run_in_line_until_the_comm_stream_is_handed_out(inputs):
+    """Synchronous dispatches on two streams with asynchronous ones between them, every input still being
+    produced when its dispatch is called; then the communication stream is asked for: it comes after the
+    dispatch that ran on the caller's stream, and the next synchronous one runs on it."""
+    with make_buffer(tmax=TOKENS, hidden=HIDDEN, channels=2) as buffer:
+        x, idx, weights = (item.cuda() for item in inputs[0])
+        ordering = buffer._ordering
+        first, second = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+
+        def step(stream, asynchronous=False):
+            arm(buffer, inputs)
+            with torch.cuda.stream(stream):
+                staged = torch.zeros_like(x)
+                torch.cuda._sleep(4_000_000)
+                staged.copy_(x)
+                result = buffer.dispatch(staged, idx, weights, do_expand=True, async_with_compute_stream=asynchronous)
+                if asynchronous:
+                    result[4].current_stream_wait()
+                copies = tuple(item.clone() for item in result[:3])
+            return result, copies
+
+        def check(result, copies):
+            buffer.peers.wait(30_000)
+            verify_dispatch((*copies, *result[3:]), inputs, 0, WORLD, EXPERTS, TOPK, True, 1, False)
+
+        for stream, asynchronous in ((first, False), (second, False), (second, True), (first, False), (first, False), (first, True)):
+            outcome = step(stream, asynchronous)
+            assert ordering._last[0] == ordering._key(ordering.stream if asynchronous else stream)
+            check(*outcome)
+            del outcome
+        result, copies = step(second)
+        comm = buffer.get_comm_stream()
+        comm.synchronize()
+        assert result[4].event.query()
+        check(result, copies)
+        del result, copies
+        outcome = step(first)
+        assert ordering._last[0] == ordering._key(comm)
+        check(*outcome)
+
+
 def test_cumulative_expert_statistics_accumulate_on_the_gpu(inputs):
     with make_buffer(tmax=TOKENS, hidden=HIDDEN, channels=2) as buffer:
         total = torch.zeros(EXPERTS // WORLD, dtype=torch.int32, device="cuda")
