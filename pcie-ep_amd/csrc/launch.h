@@ -28,6 +28,19 @@ constexpr int kDefaultTxWaves = 2;
 constexpr int kDefaultRxWaves = 2;
 constexpr int kMaxTxWaves = 4;
 constexpr int kMaxRxWaves = 6;
+// Receive tickets a payload wavefront takes at once, at most.  Two while a row is short: its ACK and its claim then
+// cost more than its bytes (see rx_rows).  Measured with 1500 tokens, 8 ranks, us per dispatch with one row at a time
+// and with two.  BF16: 512 columns 275 / 227, 1024 296 / 276, 1200 428 / 422, 1600 480 / 490, 2048 576 / 585: up to
+// 2.75 KB of slot.  FP8, whose rows also keep their wavefront busy for longer: 1000 columns 308 / 245, 2048 457 / 339,
+// 2880 514 / 452, 4096 583 / 570: up to what two rows' registers hold.  Four rows at a time are
+// slower than two everywhere (1000 columns 254, 2048 366): fewer wavefronts share the work.
+constexpr int kMaxReceiveBatch = 2;
+constexpr int kReceiveScratchDwords = 128;  // metadata records of a batch: two up to top-13, one up to top-32
+constexpr int kBatchedBf16SlotBytes = 2816, kBatchedFp8Columns = 4096;
+inline int receive_batch(const SegmentLayout& z) {
+    const bool is_short = z.dims.wire_fp8 ? z.dims.hidden <= kBatchedFp8Columns : z.meta_offset + z.meta_bytes <= kBatchedBf16SlotBytes;
+    return is_short && kMaxReceiveBatch * z.meta_bytes <= kReceiveScratchDwords * 4 ? kMaxReceiveBatch : 1;
+}
 // Upper bound of the payload workgroups: with at most 32 control and 32 local-bypass workgroups the grid then has at
 // most 256 workgroups of at most 768 threads, and an MI355X (256 compute units, each able to hold at least one such
 // workgroup next to other work) keeps all of them resident at once.  The roles wait for each other through device

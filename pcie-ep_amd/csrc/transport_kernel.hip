@@ -70,7 +70,7 @@ namespace pcie_ep {
 
 namespace {
 
-constexpr int kScratchDwords = 128;  // per wavefront: one slot metadata record or one ticket
+constexpr int kScratchDwords = kReceiveScratchDwords;  // per wavefront: slot metadata records (of one or kMaxReceiveBatch rows)
 constexpr int kMaxWaves = 12;
 
 struct WaveScratch {
@@ -139,11 +139,11 @@ __device__ __forceinline__ bool ring_entry_free(const uint64_t* taken, uint64_t 
     return previous < 0 || device_load(taken + previous % kRing) == sequence(epoch, previous);
 }
 
-// Consumer side: claim the next ticket, then wait until its entry is complete.
+// Consumer side: claim the next tickets, then wait until an entry is complete.
 // Returns 1 when available, -1 when there is no such ticket or on abort.
-__device__ __forceinline__ int claim_ticket(QueueCounter& head, int lane) {
+__device__ __forceinline__ int claim_tickets(QueueCounter& head, int count, int lane) {
     uint32_t ticket = 0;
-    if (lane == 0) ticket = device_add(&head.value, 1u);
+    if (lane == 0) ticket = device_add(&head.value, uint32_t(count));
     return broadcast_first(int(ticket));
 }
 __device__ __forceinline__ int wait_ticket(const DeviceState& state, TransportQueues& q, const uint64_t* ready, QueueCounter& head, int ticket,
@@ -1017,218 +1017,288 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
 // ---------------------------------------------------------------------------------------
 // RX + scatter worker
 // ---------------------------------------------------------------------------------------
-// Reads the row of receive ticket `ticket_index` (already marked ready) from its
-// host slot and stores it to its destination rows.  Returns false when the
-// wavefront must stop.
-template <bool kFp8, bool kVector>
-__device__ __forceinline__ bool rx_row(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int ticket_index, WorkerCounters& counters,
-                       const Deadline& deadline, bool& gate_open, bool& prefixes_known PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
+// Reads the rows of receive tickets first_ticket .. first_ticket + count - 1 (already
+// marked ready, count <= kRows) from their host slots and stores them to their
+// destination rows.  Returns false when the wavefront must stop.
+//
+// Short rows are not bound by their bytes but by what a row costs the link and the queues whatever its
+// length: its ACK, eight bytes in a line of host memory that the source's thread keeps
+// fetching (33 ns each: a second store of every ACK adds exactly that), and its claim, an atomic on one word
+// (12 ns).  They are therefore taken kRows at a time (receive_batch): consecutive tickets
+// are mostly neighbouring slots of one source, so that their ACKs leave as one store.
+template <bool kFp8, bool kVector, int kRows>
+__device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int first_ticket, int count,
+                       WorkerCounters& counters, const Deadline& deadline, bool& gate_open, bool& prefixes_known PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
     const SegmentLayout& z = state.z;
     const int topk = z.dims.topk, me = state.local_rank, local = z.local_experts;
     const int hidden = z.dims.hidden;
     const uint64_t epoch = dispatch_epoch(state);
     const bool scatter = state.expand && state.fuse_expand;
     const __amdgpu_buffer_rsrc_t ring = device_resource(q.rx, sizeof(q.rx));
-    {
-        const uint32_t entry_base = uint32_t(ticket_index % kRing) * uint32_t(sizeof(RxEntry));
-        const uint32_t word = device_load_b32(ring, entry_base + uint32_t(lane < 8 ? lane : 0) * 4u);
-        const int source = __shfl(int(word), 0), slot = __shfl(int(word), 1), ticket_token = __shfl(int(word), 2);
-        const int channel = __shfl(int(word), 3);
-        const uint64_t payload_sequence = uint64_t(uint32_t(__shfl(int(word), 4))) | uint64_t(uint32_t(__shfl(int(word), 5))) << 32;
-        const int channel_ordinal = __shfl(int(word), 6);
-        const bool replica = __shfl(int(word), 7) != 0;
-        PCIE_EP_PROFILE(profile.first(kProfileFirstEntryNs);)
-        // The ticket now lives in registers: its ring entry may be reused while
-        // this wavefront is still moving the row.
-        wait_memory_ops();
-        if (lane == 0) device_store(q.rx_taken + ticket_index % kRing, sequence(epoch, ticket_index));
-        const char* slot_base = replica ? replica_slot_at(z, state.replica_in[source], channel, slot) : slot_at(z, state.seg[source], channel, slot);
-        uint64_t* slot_ack = replica ? replica_ack_at(z, state.seg[source], channel, z.dims.rank_domain[me], slot, me)
-                                     : ack_at(z, state.seg[source], channel, slot, me);
-        // A ragged row's last wire vector is read whole: the slot's payload is padded to 16 bytes, the padding is not used.
-        const __amdgpu_buffer_rsrc_t payload = host_resource(slot_base, uint32_t(z.meta_offset));
-        const __amdgpu_buffer_rsrc_t slot_meta = host_resource(slot_base + z.meta_offset, uint32_t(z.meta_bytes));
-        if (lane == kWave - 1) test_delay(state.rx_delay);
-        // Tickets are handed out from the first descriptor on, but no row is requested
-        // before the producer of the prefixes has put its reads of the count mailboxes
-        // on the link (a few hundred bytes that everything waits for must not queue
-        // behind megabytes of row reads).  That producer has seen every source's counts by
-        // then.  The prologue of the same launch may still be laying out thousands of own
-        // tokens: count stores that leave with rows already in flight are acknowledged some
-        // 12 us later than on an idle link (measured), so a peer whose counts came early
-        // learns this rank's that much later.  It holds its first rows in registers for as
-        // long, with their requests on the link - no link time is lost - and among ranks
-        // that start together every gate opens after the last counts have arrived anyway.
-        // The wavefront waits here with its ticket read and its addresses computed:
-        // the requests leave the moment the gate opens.
-        while (!gate_open) {
-            int gate = 0;
-            if (lane == 0) {
-                if (device_load(state.receive_prefix_state) & kPrefixRequested) gate = 1;
-                else if (aborted(q) || device_load(state.receive_prefix_state + 1) == kPrefixFailed) gate = -1;
-                else if (deadline.expired(state)) {
-                    record_error(state, kErrRingProgressWait);
-                    raise_abort(q);
-                    gate = -1;
-                }
-            }
-            gate = broadcast_first(gate);
-            if (gate < 0) return false;
-            if (gate > 0) gate_open = true;
-            else __builtin_amdgcn_s_sleep(24);
-        }
-        PCIE_EP_PROFILE(profile.first(kProfileGateOpenNs);)
-        // Column 0 of the receive/expand diagnostic: this row's host read starts
-        // while an earlier row of the channel has not finished its scatter (the
-        // conservative proof point of fused_receive.cuh:216-225; a count, not a time).
-        if (state.overlap_diagnostic && lane == 0 && channel_ordinal > 0 &&
-            int(device_load(&q.rx_retired[channel].value)) < channel_ordinal)
-            atomicAdd(reinterpret_cast<unsigned long long*>(state.receive_expand_overlap + channel * 2), 1ull);
-
-        PCIE_EP_PROFILE(const uint64_t request_begin = sampled ? profile.now() : 0;)
-        // Metadata first (it arrives first), payload right behind it.
-        const u32x4 meta_vector = host_load_b128(slot_meta, uint32_t(lane) * 16u);  // 16 bytes per lane; out of range reads as 0
-
-        // Whole wire vectors of the row, and with a ragged row (any length and any alignment of the destination rows:
-        // one more wire vector, of which `rest` bytes of BF16 are stored).  Byte by byte such a row was one host read
-        // and one store per element: 1536 tokens of 1000 columns on the FP8 wire, 8 ranks, top-4: 609 -> 315 us per dispatch.
-        RowVectors row;
-        const int wire_vectors = kFp8 ? hidden / 16 : hidden / 8;
-        const int rest = kVector ? 0 : (kFp8 ? hidden % 16 : hidden % 8) * 2;
-        const int wire_total = wire_vectors + (rest ? 1 : 0);
-        constexpr int kWireItems = kFp8 ? kPassItems / 2 : kPassItems;  // a code vector fills two BF16 vectors
-        constexpr int kWirePass = kWireItems * kWave;
-        // First (usually only) pass of the row; lanes behind the row read 0.
+    constexpr int kEntryWords = int(sizeof(RxEntry) / 4);
+    static_assert(kRows * kEntryWords <= kWave, "one lane per ticket word");
+    // Lane 8 r + w: word w of row r's ticket.  Rows beyond `count` repeat the first one's ticket; their loads are
+    // empty and nothing of theirs is stored.
+    const int lane_row = lane / kEntryWords < count ? lane / kEntryWords : 0;
+    const uint32_t word = device_load_b32(ring, uint32_t((first_ticket + lane_row) % kRing) * uint32_t(sizeof(RxEntry)) + uint32_t(lane % kEntryWords) * 4u);
+    const auto entry = [&](int row, int index) { return __builtin_amdgcn_readlane(int(word), row * kEntryWords + index); };
+    int source[kRows], ticket_token[kRows], channel[kRows];
+    uint64_t payload_sequence[kRows];
+    const char* slot_base[kRows];
+    PCIE_EP_PROFILE(profile.first(kProfileFirstEntryNs);)
+    // The tickets now live in registers: their ring entries may be reused while
+    // this wavefront is still moving the rows.
+    wait_memory_ops();
+    if (lane < count) device_store(q.rx_taken + (first_ticket + lane) % kRing, sequence(epoch, first_ticket + lane));
+    uint64_t* slot_ack = nullptr;  // lane r: row r's
+    uint64_t ack_sequence = 0;
 #pragma unroll
-        for (int j = 0; j < kWireItems; ++j) row.v[j] = host_load_b128(payload, uint32_t(j * kWave + lane) * 16u);
-        PCIE_EP_PROFILE(profile.first(kProfileFirstRequestNs);)
-        if (lane < kScratchDwords / 4) {
-            scratch[lane * 4] = meta_vector[0];
-            scratch[lane * 4 + 1] = meta_vector[1];
-            scratch[lane * 4 + 2] = meta_vector[2];
-            scratch[lane * 4 + 3] = meta_vector[3];
+    for (int r = 0; r < kRows; ++r) {
+        source[r] = entry(r, 0);
+        const int slot = entry(r, 1);
+        ticket_token[r] = entry(r, 2);
+        channel[r] = entry(r, 3);
+        payload_sequence[r] = uint64_t(uint32_t(entry(r, 4))) | uint64_t(uint32_t(entry(r, 5))) << 32;
+        const bool replica = entry(r, 7) != 0;
+        slot_base[r] = replica ? replica_slot_at(z, state.replica_in[source[r]], channel[r], slot) : slot_at(z, state.seg[source[r]], channel[r], slot);
+        uint64_t* ack = replica ? replica_ack_at(z, state.seg[source[r]], channel[r], z.dims.rank_domain[me], slot, me)
+                                : ack_at(z, state.seg[source[r]], channel[r], slot, me);
+        if (lane == r) {
+            slot_ack = ack;
+            ack_sequence = payload_sequence[r];
         }
-        fence_lds();
-        PCIE_EP_PROFILE(profile.first(kProfileFirstDataNs);)
-        const int token = int(scratch[0]);
-        const float scale = bits_float(scratch[2]);
-        if (token != ticket_token || payload_sequence != sequence(epoch, token)) {
-            // Terminal: never forge an ACK for a slot whose identity is unknown
-            // (advanced_dispatch.cuh:607-610).
-            if (lane == 0) {
-                record_error(state, kErrPayloadSequence);
+    }
+    if (lane == kWave - 1) test_delay(state.rx_delay);
+    // Tickets are handed out from the first descriptor on, but no row is requested
+    // before the producer of the prefixes has put its reads of the count mailboxes
+    // on the link (a few hundred bytes that everything waits for must not queue
+    // behind megabytes of row reads).  That producer has seen every source's counts by
+    // then.  The prologue of the same launch may still be laying out thousands of own
+    // tokens: count stores that leave with rows already in flight are acknowledged some
+    // 12 us later than on an idle link (measured), so a peer whose counts came early
+    // learns this rank's that much later.  It holds its first rows in registers for as
+    // long, with their requests on the link - no link time is lost - and among ranks
+    // that start together every gate opens after the last counts have arrived anyway.
+    // The wavefront waits here with its tickets read and its addresses computed:
+    // the requests leave the moment the gate opens.
+    while (!gate_open) {
+        int gate = 0;
+        if (lane == 0) {
+            if (device_load(state.receive_prefix_state) & kPrefixRequested) gate = 1;
+            else if (aborted(q) || device_load(state.receive_prefix_state + 1) == kPrefixFailed) gate = -1;
+            else if (deadline.expired(state)) {
+                record_error(state, kErrRingProgressWait);
                 raise_abort(q);
+                gate = -1;
             }
-            return false;
         }
-
-        // The row has been requested; where it goes depends on the receive prefixes,
-        // which may still be on their way in the first microseconds of the kernel.
-        PCIE_EP_PROFILE(const uint64_t prefix_begin = sampled ? profile.now() : 0;)
-        while (!prefixes_known) {
-            const int verdict = receive_prefix_verdict(state, epoch, lane);
-            if (verdict < 0 || broadcast_first(aborted(q) ? 1 : 0)) return false;
-            if (verdict > 0) prefixes_known = true;
-            // The row itself is microseconds away: a slow poll costs nothing, and a couple of hundred
-            // wavefronts polling fast would slow down the very stores of the prefixes they wait for.
-            else __builtin_amdgcn_s_sleep(48);
+        gate = broadcast_first(gate);
+        if (gate < 0) return false;
+        if (gate > 0) gate_open = true;
+        else __builtin_amdgcn_s_sleep(24);
+    }
+    PCIE_EP_PROFILE(profile.first(kProfileGateOpenNs);)
+    // Column 0 of the receive/expand diagnostic: a row's host read starts
+    // while an earlier row of the channel has not finished its scatter (the
+    // conservative proof point of fused_receive.cuh:216-225; a count, not a time).
+    if (state.overlap_diagnostic && lane < count) {
+        int my_channel = 0, channel_ordinal = 0;
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            if (lane == r) {
+                my_channel = channel[r];
+                channel_ordinal = entry(r, 6);
+            }
         }
+        if (channel_ordinal > 0 && int(device_load(&q.rx_retired[my_channel].value)) < channel_ordinal)
+            atomicAdd(reinterpret_cast<unsigned long long*>(state.receive_expand_overlap + my_channel * 2), 1ull);
+    }
 
-        PCIE_EP_PROFILE(if (sampled) profile.add(kProfileRxPrefixWaitSum, profile.now() - prefix_begin);)
-        // Destination rows, one lane per branch.  Everything the row numbers are
-        // made of comes from the peer: the token must be addressed to this rank and
-        // its ordinals must lie inside the counts that peer announced, or a store
-        // would land in another expert's rows or before the pool.  Same verdict as a
-        // wrong identity: terminal, and the slot is not ACKed.
-        int64_t my_row = -1;
-        int my_expert = -1;
-        bool out_of_range = lane == 0 && !((scratch[1] >> me) & 1u);
+    PCIE_EP_PROFILE(const uint64_t request_begin = sampled ? profile.now() : 0;)
+    // Whole wire vectors of a row, and with a ragged row (any length and any alignment of the destination rows:
+    // one more wire vector, of which `rest` bytes of BF16 are stored).  Byte by byte such a row was one host read
+    // and one store per element: 1536 tokens of 1000 columns on the FP8 wire, 8 ranks, top-4: 606 -> 315 us per dispatch.
+    constexpr int kWireItems = kFp8 ? kPassItems / 2 : kPassItems;  // a code vector fills two BF16 vectors
+    constexpr int kRowItems = kWireItems / kRows;                   // wire vectors a lane holds of one row
+    constexpr int kOutPerWire = kFp8 ? 2 : 1;
+    constexpr int kWirePass = kRowItems * kWave;
+    const int wire_vectors = kFp8 ? hidden / 16 : hidden / 8;
+    const int rest = kVector ? 0 : (kFp8 ? hidden % 16 : hidden % 8) * 2;
+    const int wire_total = wire_vectors + (rest ? 1 : 0);
+    // Several rows are rows of one pass (receive_batch).
+    static_assert(kRows == 1 || (kFp8 ? kBatchedFp8Columns : kBatchedBf16SlotBytes) <= kWirePass * 16, "a batched row must fit its share of the registers");
+    // Metadata first (it arrives first), payload right behind it; lanes behind a row read 0.  A ragged row's last wire
+    // vector is read whole: the slot's payload is padded to 16 bytes, the padding is not used.
+    u32x4 meta_vector[kRows];
+    RowVectors row;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+        meta_vector[r] = host_load_b128(host_resource(slot_base[r] + z.meta_offset, r < count ? uint32_t(z.meta_bytes) : 0u), uint32_t(lane) * 16u);
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        const __amdgpu_buffer_rsrc_t payload = host_resource(slot_base[r], r < count ? uint32_t(z.meta_offset) : 0u);
+        // First (usually only) pass of the row.
+#pragma unroll
+        for (int j = 0; j < kRowItems; ++j) row.v[r * kRowItems + j] = host_load_b128(payload, uint32_t(j * kWave + lane) * 16u);
+    }
+    PCIE_EP_PROFILE(profile.first(kProfileFirstRequestNs);)
+    const int meta_dwords = z.meta_bytes / 4;  // a multiple of four; kRows records fit the scratch (receive_batch)
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        if (r < count && lane < meta_dwords / 4) {
+            uint32_t* record = scratch + r * meta_dwords + lane * 4;
+            record[0] = meta_vector[r][0];
+            record[1] = meta_vector[r][1];
+            record[2] = meta_vector[r][2];
+            record[3] = meta_vector[r][3];
+        }
+    }
+    fence_lds();
+    PCIE_EP_PROFILE(profile.first(kProfileFirstDataNs);)
+    bool stranger = false;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        const int token = int(scratch[r < count ? r * meta_dwords : 0]);
+        stranger |= r < count && (token != ticket_token[r] || payload_sequence[r] != sequence(epoch, token));
+    }
+    if (__any(stranger)) {
+        // Terminal: never forge an ACK for a slot whose identity is unknown
+        // (advanced_dispatch.cuh:607-610).
+        if (lane == 0) {
+            record_error(state, kErrPayloadSequence);
+            raise_abort(q);
+        }
+        return false;
+    }
+
+    // The rows have been requested; where they go depends on the receive prefixes,
+    // which may still be on their way in the first microseconds of the kernel.
+    PCIE_EP_PROFILE(const uint64_t prefix_begin = sampled ? profile.now() : 0;)
+    while (!prefixes_known) {
+        const int verdict = receive_prefix_verdict(state, epoch, lane);
+        if (verdict < 0 || broadcast_first(aborted(q) ? 1 : 0)) return false;
+        if (verdict > 0) prefixes_known = true;
+        // The row itself is microseconds away: a slow poll costs nothing, and a couple of hundred
+        // wavefronts polling fast would slow down the very stores of the prefixes they wait for.
+        else __builtin_amdgcn_s_sleep(48);
+    }
+
+    PCIE_EP_PROFILE(if (sampled) profile.add(kProfileRxPrefixWaitSum, profile.now() - prefix_begin);)
+    // Destination rows, one lane per branch.  Everything the row numbers are
+    // made of comes from the peer: the token must be addressed to this rank and
+    // its ordinals must lie inside the counts that peer announced, or a store
+    // would land in another expert's rows or before the pool.  Same verdict as a
+    // wrong identity: terminal, and the slot is not ACKed.
+    // The prefixes of all rows are requested before the first is used.
+    int my_expert[kRows], before[kRows], through[kRows], offset[kRows], first[kRows], end[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        my_expert[r] = -1;
+        before[r] = through[r] = offset[r] = first[r] = end[r] = 0;
+        if (r >= count) continue;
         if (lane < topk) {
-            const int global_expert = int(scratch[kMetaBranchOffset / 4 + lane]);
+            const int global_expert = int(scratch[r * meta_dwords + kMetaBranchOffset / 4 + lane]);
             const int expert = global_expert - me * local;
             if (global_expert >= 0 && expert >= 0 && expert < local) {
-                const int ordinal = int(scratch[kMetaBranchOffset / 4 + topk + lane]);
-                const int before = device_load(state.source_expert_prefix + source * local + expert);
-                const int through = source + 1 < z.dims.num_ranks ? device_load(state.source_expert_prefix + (source + 1) * local + expert)
-                                                                  : device_load(state.expert_counts + expert);
-                out_of_range |= ordinal < 0 || ordinal >= through - before;
-                if (scatter) {
-                    my_expert = expert;
-                    my_row = int64_t(device_load(state.expert_offsets + expert)) + before + ordinal;
-                }
+                my_expert[r] = expert;
+                before[r] = device_load(state.source_expert_prefix + source[r] * local + expert);
+                through[r] = source[r] + 1 < z.dims.num_ranks ? device_load(state.source_expert_prefix + (source[r] + 1) * local + expert)
+                                                              : device_load(state.expert_counts + expert);
+                if (scatter) offset[r] = device_load(state.expert_offsets + expert);
             }
         }
         if (lane == 0) {
-            const int ordinal = int(scratch[kMetaRankOrdinalsOffset / 4 + me]);
-            const int first = device_load(state.source_offsets + source);
-            out_of_range |= ordinal < 0 || ordinal >= device_load(state.source_offsets + source + 1) - first;
-            if (!scatter) my_row = int64_t(first) + ordinal;
+            first[r] = device_load(state.source_offsets + source[r]);
+            end[r] = device_load(state.source_offsets + source[r] + 1);
         }
-        if (__any(out_of_range)) {
-            if (lane == 0) {
-                record_error(state, kErrPayloadSequence);
-                raise_abort(q);
-            }
-            return false;
+    }
+    int64_t my_row[kRows];
+    const int64_t capacity = scatter ? state.expanded_capacity : unique_capacity(z.dims);
+    bool out_of_range = false, beyond = false;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        my_row[r] = -1;
+        if (r >= count) continue;
+        const uint32_t* record = scratch + r * meta_dwords;
+        out_of_range |= lane == 0 && !((record[1] >> me) & 1u);
+        if (my_expert[r] >= 0) {
+            const int ordinal = int(record[kMetaBranchOffset / 4 + topk + lane]);
+            out_of_range |= ordinal < 0 || ordinal >= through[r] - before[r];
+            if (scatter) my_row[r] = int64_t(offset[r]) + before[r] + ordinal;
         }
-        const int64_t capacity = scatter ? state.expanded_capacity : unique_capacity(z.dims);
-        if (__any(my_row >= capacity)) {
-            if (lane == 0) {
-                record_error(state, kErrExpandedCapacity);
-                raise_abort(q);
-            }
-            return false;
+        if (lane == 0) {
+            const int ordinal = int(record[kMetaRankOrdinalsOffset / 4 + me]);
+            out_of_range |= ordinal < 0 || ordinal >= end[r] - first[r];
+            if (!scatter) my_row[r] = int64_t(first[r]) + ordinal;
         }
-        const uint64_t destinations = __ballot(my_row >= 0);
-        uint16_t* output_base = scatter ? state.expanded_payload : state.unique_payload;
-        if (lane == kWave - 1) test_delay(state.scatter_delay);
+        beyond |= my_row[r] >= capacity;
+    }
+    if (__any(out_of_range)) {
+        if (lane == 0) {
+            record_error(state, kErrPayloadSequence);
+            raise_abort(q);
+        }
+        return false;
+    }
+    if (__any(beyond)) {
+        if (lane == 0) {
+            record_error(state, kErrExpandedCapacity);
+            raise_abort(q);
+        }
+        return false;
+    }
+    uint16_t* output_base = scatter ? state.expanded_payload : state.unique_payload;
+    if (lane == kWave - 1) test_delay(state.scatter_delay);
 
-        for (int first_wire = 0; first_wire < wire_total; first_wire += kWirePass) {
-            if (first_wire > 0) {
+    for (int first_wire = 0; first_wire < wire_total; first_wire += kWirePass) {  // one pass with several rows
+        if (kRows == 1 && first_wire > 0) {
+            const __amdgpu_buffer_rsrc_t payload = host_resource(slot_base[0], uint32_t(z.meta_offset));
 #pragma unroll
-                for (int j = 0; j < kWireItems; ++j) row.v[j] = host_load_b128(payload, uint32_t(first_wire + j * kWave + lane) * 16u);
-            }
-            const bool last_pass = first_wire + kWirePass >= wire_total;
-            if (last_pass) {
-                // All loads of the staged row have returned: release the host slot.
-                if (lane == 0) host_store_release(slot_ack, payload_sequence);
-                PCIE_EP_PROFILE(if (sampled) { wait_memory_ops(); profile.add(kProfileRxRequestSum, profile.now() - request_begin); })
-            }
-            if constexpr (kFp8) {
-                // 16 codes -> 16 BF16 (two 16-byte vectors); expanded in place from the top.
+            for (int j = 0; j < kRowItems; ++j) row.v[j] = host_load_b128(payload, uint32_t(first_wire + j * kWave + lane) * 16u);
+        }
+        const bool last_pass = kRows > 1 || first_wire + kWirePass >= wire_total;
+        if (last_pass) {
+            // All loads of the staged rows have returned: release the host slots.
+            if (lane < count) host_store_release(slot_ack, ack_sequence);
+            PCIE_EP_PROFILE(if (sampled) { wait_memory_ops(); profile.add(kProfileRxRequestSum, profile.now() - request_begin); })
+        }
+        if constexpr (kFp8) {
+            // 16 codes -> 16 BF16 (two 16-byte vectors); expanded in place from the top.
 #pragma unroll
-                for (int j = kWireItems - 1; j >= 0; --j) {
-                    u32x4 lo, hi;
-                    dequantize_vector(row.v[j], scale, lo, hi);
-                    row.v[2 * j] = lo;
-                    row.v[2 * j + 1] = hi;
-                }
+            for (int j = kWireItems - 1; j >= 0; --j) {
+                u32x4 lo, hi;
+                dequantize_vector(row.v[j], bits_float(scratch[(j / kRowItems < count ? j / kRowItems : 0) * meta_dwords + 2]), lo, hi);
+                row.v[2 * j] = lo;
+                row.v[2 * j + 1] = hi;
             }
+        }
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            if (r >= count) break;
             // The ragged row's last wire vector is item (wire_vectors - first_wire) / 64 of lane wire_vectors % 64.
-            constexpr int kOutPerWire = kFp8 ? 2 : 1;
             u32x4 last[kOutPerWire] = {};
             if (!kVector && rest && last_pass) {
                 const int item = (wire_vectors - first_wire) / kWave;
 #pragma unroll
-                for (int j = 0; j < kWireItems; ++j) {
+                for (int j = 0; j < kRowItems; ++j) {
                     if (j != item) continue;
 #pragma unroll
-                    for (int half = 0; half < kOutPerWire; ++half) last[half] = row.v[j * kOutPerWire + half];
+                    for (int half = 0; half < kOutPerWire; ++half) last[half] = row.v[(r * kRowItems + j) * kOutPerWire + half];
                 }
             }
-            uint64_t remaining = destinations;
+            uint64_t remaining = __ballot(my_row[r] >= 0);
             while (remaining) {
                 const int branch = __builtin_ctzll(remaining);
                 remaining &= remaining - 1;
-                uint16_t* output = output_base + size_t(__shfl(my_row, branch)) * hidden;
+                uint16_t* output = output_base + size_t(__shfl(my_row[r], branch)) * hidden;
 #pragma unroll
-                for (int j = 0; j < kWireItems; ++j) {
+                for (int j = 0; j < kRowItems; ++j) {
                     const int index = first_wire + j * kWave + lane;
                     if (index < wire_vectors) {
                         // Wire vector i of an FP8 row holds elements [16 i, 16 i + 16): output vectors 2 i and 2 i + 1.
 #pragma unroll
                         for (int half = 0; half < kOutPerWire; ++half)
-                            row_store_vector<kVector>(output, index * kOutPerWire + half, row.v[j * kOutPerWire + half]);
+                            row_store_vector<kVector>(output, index * kOutPerWire + half, row.v[(r * kRowItems + j) * kOutPerWire + half]);
                     }
                 }
                 if (!kVector && rest && last_pass && lane == wire_vectors % kWave) {
@@ -1246,35 +1316,46 @@ __device__ __forceinline__ bool rx_row(const DeviceState& state, TransportQueues
                 }
             }
         }
+    }
 
-        // Row metadata (advanced_layout.cuh:207-215; layout.cuh:31-48).
+    // Row metadata (advanced_layout.cuh:207-215; layout.cuh:31-48).
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        if (r >= count) break;
+        const uint32_t* record = scratch + r * meta_dwords;
         if (scatter) {
-            if (my_row >= 0) {
-                state.expanded_expert_idx[my_row] = my_expert;
-                state.expanded_weights[my_row] = bits_float(scratch[kMetaBranchOffset / 4 + 2 * topk + lane]);
-                state.expanded_source_meta[my_row * 3] = source;
-                state.expanded_source_meta[my_row * 3 + 1] = token;
-                state.expanded_source_meta[my_row * 3 + 2] = lane;
+            if (my_row[r] >= 0) {
+                state.expanded_expert_idx[my_row[r]] = my_expert[r];
+                state.expanded_weights[my_row[r]] = bits_float(record[kMetaBranchOffset / 4 + 2 * topk + lane]);
+                state.expanded_source_meta[my_row[r] * 3] = source[r];
+                state.expanded_source_meta[my_row[r] * 3 + 1] = ticket_token[r];
+                state.expanded_source_meta[my_row[r] * 3 + 2] = lane;
             }
         } else {
-            const int64_t out_row = __shfl(my_row, 0);
+            const int64_t out_row = __shfl(my_row[r], 0);
             if (lane < topk) {
-                const int expert = int(scratch[kMetaBranchOffset / 4 + lane]);
+                const int expert = int(record[kMetaBranchOffset / 4 + lane]);
                 const bool is_local = expert >= me * local && expert < (me + 1) * local;
                 state.unique_topk_idx[out_row * topk + lane] = is_local ? expert - me * local : -1;
-                state.unique_topk_weights[out_row * topk + lane] = is_local ? bits_float(scratch[kMetaBranchOffset / 4 + 2 * topk + lane]) : 0.0f;
-                state.unique_expert_ordinals[out_row * topk + lane] = int(scratch[kMetaBranchOffset / 4 + topk + lane]);
+                state.unique_topk_weights[out_row * topk + lane] = is_local ? bits_float(record[kMetaBranchOffset / 4 + 2 * topk + lane]) : 0.0f;
+                state.unique_expert_ordinals[out_row * topk + lane] = int(record[kMetaBranchOffset / 4 + topk + lane]);
             }
             if (lane == 0) {
-                state.unique_source_meta[out_row * 3] = source;
-                state.unique_source_meta[out_row * 3 + 1] = token;
+                state.unique_source_meta[out_row * 3] = source[r];
+                state.unique_source_meta[out_row * 3 + 1] = ticket_token[r];
                 state.unique_source_meta[out_row * 3 + 2] = -1;
             }
         }
-        ++counters.reads;
-        PCIE_EP_PROFILE(if (sampled) profile.add(kProfileRxScatterSum, profile.now() - request_begin);)
-        fence_lds();  // scratch is reused by the next ticket
-        if (lane == 0) device_add(&q.rx_retired[channel].value, 1u);
+    }
+    counters.reads += count;
+    PCIE_EP_PROFILE(if (sampled) profile.add(kProfileRxScatterSum, profile.now() - request_begin);)
+    fence_lds();  // scratch is reused by the next tickets
+    if (lane < count) {
+        int my_channel = channel[0];
+#pragma unroll
+        for (int r = 1; r < kRows; ++r)
+            if (lane == r) my_channel = channel[r];
+        device_add(&q.rx_retired[my_channel].value, 1u);
     }
     return true;
 }
@@ -1315,7 +1396,7 @@ constexpr int kMinTxWaves = 16;
 constexpr uint64_t kIdleCrossoverUs = 30;
 constexpr int kPreGateRows = 32;
 
-template <bool kFp8, bool kVector>
+template <bool kFp8, bool kVector, int kRows>
 __device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int order, int waves) {
     const uint64_t epoch = dispatch_epoch(state);
     Deadline deadline(now_ticks());
@@ -1326,7 +1407,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
     uint64_t idle_since = 0;  // 0: the last look found work
     while (true) {
         // 0: nothing to do now, 1: transmit, 2: receive, -1: both directions are finished or the kernel aborts.
-        int choice = 0;
+        int choice = 0, claims = 1;
         PCIE_EP_PROFILE(const uint64_t look_begin = profile.now();)
         int gate_seen = gate_open ? 1 : 0;
         if (lane == 0) {
@@ -1334,7 +1415,8 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
             else {
                 const int tx_head = int(device_load(&q.tx_head.value)), rx_head = int(device_load(&q.rx_head.value));
                 const bool tx_backlog = tx_head < int(device_load(&q.tx_tail.value));
-                bool rx_backlog = rx_head < int(device_load(&q.rx_tail.value));
+                const int rx_tail = int(device_load(&q.rx_tail.value));
+                bool rx_backlog = rx_head < rx_tail;
                 // Receive tickets are there long before the first row may be requested (rx_row
                 // holds the gate).  Only the first kPreGateRows of them are claimed ahead of
                 // it, by wavefronts that then wait with their addresses ready: if every
@@ -1369,6 +1451,11 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                     // therefore never do while a row may still come in.
                     if (own_done || (prefer_tx && now - idle_since > kIdleCrossoverUs * state.clock_khz / 1000)) choice = prefer_tx ? 2 : 1;
                 }
+                // A receiving wavefront takes its share of the tickets that are there, at most a batch.
+                if (kRows > 1 && choice == 2) {
+                    const int share = (rx_tail - rx_head) / waves;
+                    claims = share < 1 ? 1 : (share < kRows ? share : kRows);
+                }
                 if (choice) idle_since = 0;
                 else {
                     if (tx_done && rx_done) choice = -1;
@@ -1395,18 +1482,35 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
         const bool transmit = choice == 1;
         QueueCounter& head = transmit ? q.tx_head : q.rx_head;
         PCIE_EP_PROFILE(profile.first(kProfileFirstClaimNs); const uint64_t claim_begin = profile.now(); if (!profile.values[kProfileFirstLookNs]) profile.values[kProfileFirstLookNs] = look_begin;)
-        const int ticket_index = claim_ticket(head, lane);
+        if constexpr (kRows > 1) claims = broadcast_first(claims);
+        int ticket_index = claim_tickets(head, claims, lane);
+        const int end = ticket_index + claims;
         // Several wavefronts may have seen the same backlog: a claim beyond the last
         // ticket of the dispatch is simply dropped, an earlier one waits for its tag.
-        if (wait_ticket(state, q, transmit ? q.tx_ready : q.rx_ready, head, ticket_index, epoch, lane, deadline) < 0) {
-            if (broadcast_first(aborted(q) ? 1 : 0)) break;
-            continue;
+        // Rows whose tickets are ready never wait for a later ticket of the same claim: a
+        // source may publish that one only when it has seen these rows acknowledged.
+        bool go_on = true;
+        while (go_on && ticket_index < end) {
+            if (wait_ticket(state, q, transmit ? q.tx_ready : q.rx_ready, head, ticket_index, epoch, lane, deadline) < 0) {
+                if (broadcast_first(aborted(q) ? 1 : 0)) go_on = false;
+                break;
+            }
+            PCIE_EP_PROFILE(profile.first(kProfileFirstTaggedNs); profile.add(kProfileTicketWaitSum, profile.now() - claim_begin); const bool sampled = rows_moved++ % kProfileSampleStride == 0;
+                            if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows); profile.add(transmit ? kProfileTxRows : kProfileRxRows);)
+            int count = 1;
+            if (transmit) {
+                go_on = tx_row<kFp8, kVector>(state, q, scratch, lane, ticket_index, deadline, counters PCIE_EP_PROFILE(, profile, sampled));
+            } else {
+                if constexpr (kRows > 1) {
+                    const bool ready = lane < end - ticket_index &&
+                                       (lane == 0 || device_load(q.rx_ready + (ticket_index + lane) % kRing) == sequence(epoch, ticket_index + lane));
+                    count = __builtin_ctzll(~__ballot(ready));
+                }
+                go_on = rx_rows<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, count, counters, deadline, gate_open, prefixes_known PCIE_EP_PROFILE(, profile, sampled));
+            }
+            ticket_index += count;
+            PCIE_EP_PROFILE(profile.last(kProfileLastRowNs);)
         }
-        PCIE_EP_PROFILE(profile.first(kProfileFirstTaggedNs); profile.add(kProfileTicketWaitSum, profile.now() - claim_begin); const bool sampled = rows_moved++ % kProfileSampleStride == 0;
-                        if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows); profile.add(transmit ? kProfileTxRows : kProfileRxRows);)
-        const bool go_on = transmit ? tx_row<kFp8, kVector>(state, q, scratch, lane, ticket_index, deadline, counters PCIE_EP_PROFILE(, profile, sampled))
-                                    : rx_row<kFp8, kVector>(state, q, scratch, lane, ticket_index, counters, deadline, gate_open, prefixes_known PCIE_EP_PROFILE(, profile, sampled));
-        PCIE_EP_PROFILE(profile.last(kProfileLastRowNs);)
         if (!go_on) break;
     }
     // Workers serve every channel; their counts go to channel 0's row of the
@@ -1428,7 +1532,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
 // wavefront 1 RX control); workgroups b >= C hold payload wavefronts only.  With
 // no payload workgroups configured the control workgroups carry the payload
 // wavefronts themselves.
-template <bool kFp8, bool kVector>
+template <bool kFp8, bool kVector, int kRows>
 __global__ void __launch_bounds__(kTransportMaxThreads) transport_kernel(DeviceState launch_state) {
     // The launch argument is read where it lies, in the kernel-argument segment:
     // every field is then a scalar load from constant memory and every pointer in
@@ -1539,7 +1643,7 @@ __global__ void __launch_bounds__(kTransportMaxThreads) transport_kernel(DeviceS
     // direction's share is spread over the workgroups before it doubles up in one.
     const int groups = payload_groups ? payload_groups : channels;
     const int group = payload_groups ? block - channel_groups : block;
-    if (begun) payload_worker<kFp8, kVector>(state, q, scratch, lane, wave * groups + group, groups * payload_waves);
+    if (begun) payload_worker<kFp8, kVector, kRows>(state, q, scratch, lane, wave * groups + group, groups * payload_waves);
     finish_role(state, q, lane, roles);
     // Every role loop has an explicit completion, abort or timeout exit and no
     // workgroup barrier follows the entry verdict.
@@ -1553,18 +1657,27 @@ int transport_threads(const DeviceState& state) {
     return (control > payload ? control : payload) * kWave;
 }
 
+// The instantiation that `state` selects.  Rows of whole 16-byte vectors on both sides (FP8: of whole 16-code
+// vectors on the wire) lie on 16-byte boundaries and have nothing behind their vectors; all others take the
+// ragged form of the row code.
+static auto transport_instance(const DeviceState& state) {
+    const bool fp8 = state.z.dims.wire_fp8 != 0;
+    const bool vector = fp8 ? state.z.dims.hidden % 16 == 0 : state.z.dims.hidden % 8 == 0;
+    if (receive_batch(state.z) > 1) {
+        if (fp8) return vector ? transport_kernel<true, true, kMaxReceiveBatch> : transport_kernel<true, false, kMaxReceiveBatch>;
+        return vector ? transport_kernel<false, true, kMaxReceiveBatch> : transport_kernel<false, false, kMaxReceiveBatch>;
+    }
+    if (fp8) return vector ? transport_kernel<true, true, 1> : transport_kernel<true, false, 1>;
+    return vector ? transport_kernel<false, true, 1> : transport_kernel<false, false, 1>;
+}
+
 // How many transport workgroups one compute unit holds at once (registers, LDS and
 // wavefront slots of the instantiation that `state` selects).
 hipError_t transport_workgroups_per_unit(const DeviceState& state, int* per_unit) {
     const int threads = transport_threads(state);
     if (threads > kTransportMaxThreads) return hipErrorInvalidValue;
-    const bool fp8 = state.z.dims.wire_fp8 != 0;
-    const bool vector = fp8 ? state.z.dims.hidden % 16 == 0 : state.z.dims.hidden % 8 == 0;
     const size_t lds = state.fused ? prologue_lds_bytes(state.z, threads / kWave) : 0;
-    if (fp8 && vector) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_unit, transport_kernel<true, true>, threads, lds);
-    if (fp8) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_unit, transport_kernel<true, false>, threads, lds);
-    if (vector) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_unit, transport_kernel<false, true>, threads, lds);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_unit, transport_kernel<false, false>, threads, lds);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_unit, transport_instance(state), threads, lds);
 }
 
 hipError_t launch_transport(const DeviceState& state, hipStream_t stream) {
@@ -1576,14 +1689,7 @@ hipError_t launch_transport(const DeviceState& state, hipStream_t stream) {
         if (!fused_prologue_fits(state.z, int(block.x), state.z.dims.max_tokens)) return hipErrorInvalidValue;
         dynamic_lds = prologue_lds_bytes(state.z, int(block.x) / kWave);
     }
-    const bool fp8 = state.z.dims.wire_fp8 != 0;
-    // Rows of whole 16-byte vectors on both sides (FP8: of whole 16-code vectors on the wire) lie on 16-byte
-    // boundaries and have nothing behind their vectors; all others take the ragged form of the row code.
-    const bool vector = fp8 ? state.z.dims.hidden % 16 == 0 : state.z.dims.hidden % 8 == 0;
-    if (fp8 && vector) hipLaunchKernelGGL((transport_kernel<true, true>), grid, block, dynamic_lds, stream, state);
-    else if (fp8) hipLaunchKernelGGL((transport_kernel<true, false>), grid, block, dynamic_lds, stream, state);
-    else if (vector) hipLaunchKernelGGL((transport_kernel<false, true>), grid, block, dynamic_lds, stream, state);
-    else hipLaunchKernelGGL((transport_kernel<false, false>), grid, block, dynamic_lds, stream, state);
+    hipLaunchKernelGGL(transport_instance(state), grid, block, dynamic_lds, stream, state);
     return hipGetLastError();
 }
 

@@ -216,6 +216,20 @@ def test_ragged_rows(hidden, fp8):
                 del result
 
 
+@pytest.mark.parametrize("hidden,topk,fp8", [(1312, 8, False), (1313, 8, False), (4096, 8, True), (4095, 8, True), (4097, 8, True), (64, 13, False), (64, 14, True)])
+def test_short_rows_are_received_in_pairs(hidden, topk, fp8):
+    """Both sides of the line up to which a wavefront takes two rows at a time: longest rows, ragged ones that
+    fill the last register of a pair's half, and the largest metadata.  More tokens than wavefronts, so that
+    pairs are taken; rings of one slot, where the second row of a pair comes only after the first was
+    acknowledged; both layouts."""
+    wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
+    for channels, slots in ((16, 64), (2, 1)):
+        with make_buffer(tmax=400, hidden=hidden, topk=topk, channels=channels, payload_slots=slots, descriptor_slots=slots, **wire) as buffer:
+            tokens = [400] * 8 if slots > 1 else [40, 7, 40, 0, 1, 33, 40, 12]
+            check_case(buffer, f"pairs-h{hidden}-k{topk}-s{slots}", tokens, alignment=16, fp8=fp8)
+            check_case(buffer, f"pairs-h{hidden}-k{topk}-s{slots}-unique", tokens, expand=False, seed=9, fp8=fp8)
+
+
 def test_numa_bound_staging_segments():
     """The pinned segments can be bound to a NUMA node (the far-node staging of the
     cached-replay configuration); node 0 exists on every box.  Results do not change."""
