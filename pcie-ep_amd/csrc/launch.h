@@ -41,6 +41,12 @@ inline int receive_batch(const SegmentLayout& z) {
     const bool is_short = z.dims.wire_fp8 ? z.dims.hidden <= kBatchedFp8Columns : z.meta_offset + z.meta_bytes <= kBatchedBf16SlotBytes;
     return is_short && kMaxReceiveBatch * z.meta_bytes <= kReceiveScratchDwords * 4 ? kMaxReceiveBatch : 1;
 }
+// Receive tickets a payload wavefront claims at once where rows come in pairs (at most its share of those that are
+// there; it moves them one pair after the other): the atomic on the one counter is paid once.  Us per dispatch with 2
+// and with 8: FP8 1000 columns 250 / 229, FP8 1024 with 3000 tokens 559 / 489, BF16 1024 280 / 259, BF16 512 217 / 211.
+// Wavefronts that may transmit keep to one pair, and long rows are claimed one by one: bound to several rows they
+// would not transmit meanwhile (2048 columns, hotspot top-2: 249 / 283).
+constexpr int kReceiveClaims = 8;
 // Upper bound of the payload workgroups: with at most 32 control and 32 local-bypass workgroups the grid then has at
 // most 256 workgroups of at most 768 threads, and an MI355X (256 compute units, each able to hold at least one such
 // workgroup next to other work) keeps all of them resident at once.  The roles wait for each other through device

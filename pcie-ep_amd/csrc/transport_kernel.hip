@@ -1404,6 +1404,8 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
     PCIE_EP_PROFILE(RoleProfile profile(state.clock_khz); uint64_t idle_begin = 0; int rows_moved = 0;)
     bool prefixes_known = false, gate_open = false;
     const int lead = int(kTxLeadBytes / int64_t(state.z.meta_offset + state.z.meta_bytes));
+    // A wavefront that may be wanted for transmitting binds itself to one batch at a time.
+    const int most_claims = 2 * order < waves || kRows == 1 ? kRows : kReceiveClaims;
     uint64_t idle_since = 0;  // 0: the last look found work
     while (true) {
         // 0: nothing to do now, 1: transmit, 2: receive, -1: both directions are finished or the kernel aborts.
@@ -1451,10 +1453,10 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                     // therefore never do while a row may still come in.
                     if (own_done || (prefer_tx && now - idle_since > kIdleCrossoverUs * state.clock_khz / 1000)) choice = prefer_tx ? 2 : 1;
                 }
-                // A receiving wavefront takes its share of the tickets that are there, at most a batch.
-                if (kRows > 1 && choice == 2) {
+                // A receiving wavefront takes its share of the tickets that are there, at most most_claims.
+                if (choice == 2) {
                     const int share = (rx_tail - rx_head) / waves;
-                    claims = share < 1 ? 1 : (share < kRows ? share : kRows);
+                    claims = share < 1 ? 1 : (share < most_claims ? share : most_claims);
                 }
                 if (choice) idle_since = 0;
                 else {
@@ -1482,7 +1484,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
         const bool transmit = choice == 1;
         QueueCounter& head = transmit ? q.tx_head : q.rx_head;
         PCIE_EP_PROFILE(profile.first(kProfileFirstClaimNs); const uint64_t claim_begin = profile.now(); if (!profile.values[kProfileFirstLookNs]) profile.values[kProfileFirstLookNs] = look_begin;)
-        if constexpr (kRows > 1) claims = broadcast_first(claims);
+        claims = broadcast_first(claims);
         int ticket_index = claim_tickets(head, claims, lane);
         const int end = ticket_index + claims;
         // Several wavefronts may have seen the same backlog: a claim beyond the last
@@ -1502,7 +1504,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 go_on = tx_row<kFp8, kVector>(state, q, scratch, lane, ticket_index, deadline, counters PCIE_EP_PROFILE(, profile, sampled));
             } else {
                 if constexpr (kRows > 1) {
-                    const bool ready = lane < end - ticket_index &&
+                    const bool ready = lane < kRows && lane < end - ticket_index &&
                                        (lane == 0 || device_load(q.rx_ready + (ticket_index + lane) % kRing) == sequence(epoch, ticket_index + lane));
                     count = __builtin_ctzll(~__ballot(ready));
                 }
