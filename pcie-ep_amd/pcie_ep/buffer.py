@@ -70,6 +70,7 @@ class _Ordering:
         start = torch.cuda.Event()
         start.record(self.stream)
         self._last: Tuple[Tuple[int, int], Any] = (self._stream_key, start)
+        self._order = threading.RLock()  # held while a dispatch is placed and its place recorded
         self._consumers: Dict[Tuple[int, int], Any] = {}
         self._guard = threading.Lock()
         self._made_wait: Optional[Tuple[int, int]] = None  # the stream the last dispatch made wait for its result
@@ -97,7 +98,7 @@ class _Ordering:
     def expose(self) -> Any:
         """The communication stream, for a program's own use: from now on every dispatch runs on
         it, and what is put on it comes after the dispatches so far."""
-        with self._guard:
+        with self._order:
             self._in_line = False
             if self._last[0] != self._stream_key:
                 self.stream.wait_event(self._last[1])
@@ -108,56 +109,55 @@ class _Ordering:
         """Put ``work`` (called with the stream it is to use) on the communication
         stream, or, where a synchronous dispatch may run in line, on the caller's,
         ordered after the inputs' producer, all consumers and the dispatch before;
-        returns (its value, the completion event, the caller's stream).
+        with ``synchronous`` the caller's stream waits for it.  Returns (its value,
+        the completion event, the caller's stream).
         ``make_current`` makes that stream the current one around ``work`` (needed by work that
         launches through PyTorch); work that takes the stream explicitly skips that
         switch, which is a measurable part of a small dispatch's CPU cost."""
         caller = torch.cuda.current_stream(self.device)
-        own_key = self._stream_key
-        caller_key = (caller.device.index, int(caller.cuda_stream))
-        if synchronous and previous_event is None and caller_key != own_key:
-            with self._guard:  # the stream is not handed out between this decision and the record of where the dispatch ran
-                if self._in_line:
-                    if self._last[0] != caller_key:
-                        caller.wait_event(self._last[1])
-                    for key, stream in self._consumers.items():
-                        if key != caller_key:
-                            caller.wait_stream(stream)
-                    value = work(caller)
-                    done = torch.cuda.Event()
-                    done.record(caller)
-                    self._last = (caller_key, done)
-                    return value, done, caller
-        if previous_event is None:
-            # A producer stream with nothing pending has produced the inputs already:
-            # asking is much cheaper than an event record plus a cross-stream wait.
-            # A stream this buffer has just made wait for a result (synchronous mode)
-            # is busy until that result is there: then the question is skipped too.
-            if caller_key != own_key and (caller_key == self._made_wait or not caller.query()):
-                self.stream.wait_stream(caller)
-            self._made_wait = None
-        else:
-            caller_key = own_key
-            if isinstance(previous_event, EventOverlap):
-                previous_event.stream_wait(self.stream)
+        own_key, caller_key = self._stream_key, self._key(caller)
+        # The stream is not handed out between the decision where the dispatch runs and the record of it.
+        with self._order:
+            if synchronous and previous_event is None and self._in_line and caller_key != own_key:
+                stream, ordered = caller, (caller_key,)
             else:
-                self.stream.wait_event(previous_event)
-        if self._last[0] != own_key:
-            self.stream.wait_event(self._last[1])
-        if self._consumers:
-            with self._guard:
-                consumers = list(self._consumers.items())
-            for key, stream in consumers:
-                if key != own_key and key != caller_key:
-                    self.stream.wait_stream(stream)
-        if make_current:
-            with torch.cuda.stream(self.stream):
-                value = work(self.stream)
-        else:
-            value = work(self.stream)
-        done = torch.cuda.Event()
-        done.record(self.stream)
-        self._last = (own_key, done)
+                stream, ordered = self.stream, (own_key, caller_key if previous_event is None else own_key)
+                if previous_event is None:
+                    # A producer stream with nothing pending has produced the inputs already:
+                    # asking is much cheaper than an event record plus a cross-stream wait.
+                    # A stream this buffer has just made wait for a result (synchronous mode)
+                    # is busy until that result is there: then the question is skipped too.
+                    if caller_key != own_key and (caller_key == self._made_wait or not caller.query()):
+                        stream.wait_stream(caller)
+                    self._made_wait = None
+                elif isinstance(previous_event, EventOverlap):
+                    previous_event.stream_wait(stream)
+                else:
+                    stream.wait_event(previous_event)
+            if self._last[0] != ordered[0]:
+                stream.wait_event(self._last[1])
+            if self._consumers:
+                with self._guard:
+                    consumers = list(self._consumers.items())
+                for key, consumer in consumers:
+                    if key not in ordered:
+                        stream.wait_stream(consumer)
+            done = torch.cuda.Event()
+            try:
+                if make_current and ordered[0] != caller_key:
+                    with torch.cuda.stream(stream):
+                        value = work(stream)
+                else:
+                    value = work(stream)
+            finally:
+                # Also when `work` raises: it may have launched the dispatch before it did, and the
+                # next one, on whichever stream, must not reset the queues of a running one.
+                done.record(stream)
+                self._last = (ordered[0], done)
+            if synchronous:
+                if ordered[0] != caller_key:
+                    caller.wait_event(done)
+                self._made_wait = caller_key
         return value, done, caller
 
 
@@ -346,9 +346,6 @@ class HostStagedEPBuffer:
         outputs = (result["recv_x"], result.get("recv_topk_idx"),
                    result.get("recv_topk_weights") if request.weights is not None else None, handle)
         if not asynchronous:
-            if self._ordering._last[0] != self._ordering._key(caller):  # not in line
-                caller.wait_event(done)
-            self._ordering._made_wait = self._ordering._key(caller)
             # The result tensors belong to a pool that was allocated on one stream
             # and lives as long as the buffer; only a consumer on another stream
             # needs to be made known to the caching allocator.
