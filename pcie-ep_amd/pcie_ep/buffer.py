@@ -38,7 +38,7 @@ from .overlap import EventOverlap, record_tensors
 from .peers import PeerGroup
 from .request import DispatchRequest, admit
 from .runtime import NativeRuntime
-from .streams import MaskedStream
+from .streams import MaskedStream, unit_mask
 
 _next_buffer_id = itertools.count(1)
 
@@ -55,6 +55,11 @@ class _Ordering:
     on it or rely on a dispatch being there: every later dispatch runs on it.  Nor is the
     caller's stream used where several ranks' kernels wait for each other on one GPU
     (`in_line` false): which streams those run on is their caller's arrangement.
+
+    The caller's stream must also be able to hold a dispatch, whose workgroups wait for each
+    other: it is used only if its kernels may use the units the communication stream's may.  On
+    a stream masked to a few they would not all be running, and the dispatch would end in the
+    ring-progress timeout.
     """
 
     def __init__(self, device: int, compute_units: int = 0, stream: Any = None, in_line: bool = True) -> None:
@@ -66,6 +71,7 @@ class _Ordering:
         self.stream = stream if stream is not None else (self.masked.stream if self.masked else torch.cuda.Stream(device=device))
         self.stream.wait_stream(torch.cuda.current_stream(device))
         self._stream_key = self._key(self.stream)
+        self._units = unit_mask(self.stream) if self._in_line else None
         # The stream the last dispatch ran on and its completion event; at first, what the communication stream was just made wait for.
         start = torch.cuda.Event()
         start.record(self.stream)
@@ -104,6 +110,10 @@ class _Ordering:
                 self.stream.wait_event(self._last[1])
         return self.stream
 
+    def _holds_dispatch(self, caller: Any) -> bool:
+        # The default stream cannot be masked.
+        return int(caller.cuda_stream) == 0 or (self._units is not None and unit_mask(caller) == self._units)
+
     def submit(self, work: Callable[[Any], Any], previous_event: Any = None, make_current: bool = True,
                synchronous: bool = False) -> Tuple[Any, Any, Any]:
         """Put ``work`` (called with the stream it is to use) on the communication
@@ -118,7 +128,7 @@ class _Ordering:
         own_key, caller_key = self._stream_key, self._key(caller)
         # The stream is not handed out between the decision where the dispatch runs and the record of it.
         with self._order:
-            if synchronous and previous_event is None and self._in_line and caller_key != own_key:
+            if synchronous and previous_event is None and self._in_line and caller_key != own_key and self._holds_dispatch(caller):
                 stream, ordered = caller, (caller_key,)
             else:
                 stream, ordered = self.stream, (own_key, caller_key if previous_event is None else own_key)

@@ -17,7 +17,7 @@ bits is spread evenly over the chip.
 from __future__ import annotations
 
 import ctypes as C
-from typing import Any, Tuple
+from typing import Any, Optional, Tuple
 
 import torch
 
@@ -30,6 +30,8 @@ def _runtime() -> C.CDLL:
         _hip = C.CDLL("libamdhip64.so")
         _hip.hipExtStreamCreateWithCUMask.restype = C.c_int
         _hip.hipExtStreamCreateWithCUMask.argtypes = [C.POINTER(C.c_void_p), C.c_uint32, C.POINTER(C.c_uint32)]
+        _hip.hipExtStreamGetCUMask.restype = C.c_int
+        _hip.hipExtStreamGetCUMask.argtypes = [C.c_void_p, C.c_uint32, C.POINTER(C.c_uint32)]
     return _hip
 
 
@@ -81,3 +83,12 @@ def masked_stream(count: int, first: int = 0, device: Any = None) -> MaskedStrea
     """A stream on ``count`` compute units starting at ``first`` (mask order) of the current device."""
     index = torch.cuda.current_device() if device is None else torch.device(device).index
     return MaskedStream(index, count, first)
+
+
+def unit_mask(stream: Any) -> Optional[bytes]:
+    """The compute units that kernels on ``stream`` may use, whoever created it: the bit array of the mask
+    order (all units where no mask was given), or None if HIP does not say.  The stream's device must be the current one."""
+    words = (torch.cuda.get_device_properties(stream.device).multi_processor_count + 31) // 32
+    mask = (C.c_uint32 * words)()
+    status = _runtime().hipExtStreamGetCUMask(C.c_void_p(int(stream.cuda_stream)), words, mask)
+    return bytes(mask) if status == 0 else None

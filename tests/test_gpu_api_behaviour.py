@@ -178,6 +178,27 @@ def test_synchronous_dispatches_run_in_line_until_the_comm_stream_is_handed_out(
         check(*outcome)
 
 
+def test_a_caller_on_few_compute_units_does_not_hold_the_dispatch(inputs):
+    """A synchronous dispatch called on a stream masked to sixteen compute units runs on the communication stream,
+    on one that may use every unit (masked or not) and on the default stream in line."""
+    from pcie_ep.streams import masked_stream
+
+    with make_buffer(tmax=TOKENS, hidden=HIDDEN, channels=2) as buffer:
+        x, idx, weights = (item.cuda() for item in inputs[0])
+        ordering = buffer._ordering
+        units = torch.cuda.get_device_properties(0).multi_processor_count
+        for caller, in_line in ((masked_stream(16).stream, False), (masked_stream(units).stream, True), (torch.cuda.default_stream(), True)):
+            torch.cuda.synchronize()
+            print(f"case: synchronous dispatch on {caller}", flush=True)
+            arm(buffer, inputs)
+            with torch.cuda.stream(caller):
+                result = buffer.dispatch(x, idx, weights, do_expand=True)
+                assert ordering._last[0] == ordering._key(caller if in_line else ordering.stream)
+                verify_dispatch(result, inputs, 0, WORLD, EXPERTS, TOPK, True, 1, False)
+            buffer.peers.wait(30_000)
+            del result
+
+
 def test_cumulative_expert_statistics_accumulate_on_the_gpu(inputs):
     with make_buffer(tmax=TOKENS, hidden=HIDDEN, channels=2) as buffer:
         total = torch.zeros(EXPERTS // WORLD, dtype=torch.int32, device="cuda")

@@ -2,7 +2,8 @@
 remembers what every operation comes after (no GPU): whichever streams the dispatches of
 one buffer run on, each comes after the one before (they share the ticket queues), after
 its inputs and after every stream that consumed a result, and a synchronous one is in
-front of what its caller's stream does next."""
+front of what its caller's stream does next.  A synchronous one runs on the caller's stream
+only where that may use every compute unit."""
 
 from __future__ import annotations
 
@@ -29,6 +30,7 @@ class FakeGpu:
         class Stream:
             def __init__(self, device=None):
                 self.device, self.cuda_stream, self.front = SimpleNamespace(index=0), next(gpu.handles), set()
+                self.units = b"\xff"
 
             def put(self):
                 operation = next(gpu.operations)
@@ -77,12 +79,16 @@ def test_every_dispatch_comes_after_the_one_before(monkeypatch, seed):
         cuda = SimpleNamespace(Stream=gpu.Stream, Event=gpu.Event, stream=gpu.Current, current_stream=lambda device=None: gpu.current)
         monkeypatch.setattr(buffer_module, "torch", SimpleNamespace(cuda=cuda))
         gpu.current = gpu.Stream()
+        monkeypatch.setattr(buffer_module, "unit_mask", lambda stream: stream.units)
         walk(gpu)
 
 
 def walk(gpu):
     ordering = _Ordering(0)
-    callers = [gpu.current] + [gpu.Stream() for _ in range(2)]
+    callers = [gpu.current] + [gpu.Stream() for _ in range(3)]
+    few_units, unknown_units, default = callers[1:]
+    few_units.units, unknown_units.units = b"\x0f", None
+    default.units, default.cuda_stream = None, 0
     dispatches, exposed = [], False
     for _ in range(8):
         gpu.current = caller = gpu.rng.choice(callers)
@@ -128,5 +134,6 @@ def walk(gpu):
                 assert dispatches[-1] in caller.put()[1]
                 ordering.saw_consumer(caller)
         assert gpu.current is caller
-        in_line = synchronous and not exposed
+        holds = caller is default or caller.units == b"\xff"
+        in_line = synchronous and not exposed and holds
         assert place[0] is (caller if in_line else ordering.stream)
