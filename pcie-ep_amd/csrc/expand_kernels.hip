@@ -7,6 +7,8 @@
 // Replaces scatter_expert_inputs (csrc/kernels/host_staged/dispatch.cuh:8-65) and
 // quantize_transport_payload (quantization.cuh:34-71).  The reference copies 2
 // bytes per thread here.
+#include <algorithm>
+
 #include "device_common.h"
 #include "launch.h"
 #include "row_codec.h"
@@ -428,22 +430,40 @@ static bool codec_vector(const void* bf16, const void* codes, int hidden) {
     return hidden % 8 == 0 && reinterpret_cast<uintptr_t>(bf16) % 16 == 0 && reinterpret_cast<uintptr_t>(codes) % 8 == 0;
 }
 
+// Workgroups of one codec launch, at most: HIP refuses a launch of 2^32 threads, and the kernels count rows in
+// 32 bits.  More rows take several launches; one of this size moves 400 MB even at 8 columns.
+constexpr int64_t kCodecMaxGroups = 1 << 22;
+
 hipError_t launch_quantize(const uint16_t* x, uint8_t* codes, float* scales, int tokens, int hidden, hipStream_t stream) {
-    if (tokens <= 0) return hipSuccess;
     const int split = codec_split(hidden), rows = kCodecWaves / split;
-    const dim3 grid(unsigned((int64_t(tokens) + rows - 1) / rows)), block(kRowKernelThreads);
-    if (codec_vector(x, codes, hidden)) hipLaunchKernelGGL(quantize_kernel<true>, grid, block, 0, stream, x, codes, scales, tokens, hidden, split);
-    else hipLaunchKernelGGL(quantize_kernel<false>, grid, block, 0, stream, x, codes, scales, tokens, hidden, split);
-    return hipGetLastError();
+    const bool vector = codec_vector(x, codes, hidden);
+    const dim3 block(kRowKernelThreads);
+    for (int64_t done = 0; done < tokens; done += kCodecMaxGroups * rows) {
+        const int count = int(std::min<int64_t>(tokens - done, kCodecMaxGroups * rows));
+        const dim3 grid(unsigned((count + rows - 1) / rows));
+        const uint16_t* from = x + size_t(done) * hidden;
+        uint8_t* to = codes + size_t(done) * hidden;
+        if (vector) hipLaunchKernelGGL(quantize_kernel<true>, grid, block, 0, stream, from, to, scales + done, count, hidden, split);
+        else hipLaunchKernelGGL(quantize_kernel<false>, grid, block, 0, stream, from, to, scales + done, count, hidden, split);
+        if (const hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_dequantize(const uint8_t* codes, const float* scales, uint16_t* out, int tokens, int hidden, hipStream_t stream) {
-    if (tokens <= 0) return hipSuccess;
     const int split = codec_split(hidden), rows = kCodecWaves / split;
-    const dim3 grid(unsigned((int64_t(tokens) + rows - 1) / rows)), block(kRowKernelThreads);
-    if (codec_vector(out, codes, hidden)) hipLaunchKernelGGL(dequantize_kernel<true>, grid, block, 0, stream, codes, scales, out, tokens, hidden, split);
-    else hipLaunchKernelGGL(dequantize_kernel<false>, grid, block, 0, stream, codes, scales, out, tokens, hidden, split);
-    return hipGetLastError();
+    const bool vector = codec_vector(out, codes, hidden);
+    const dim3 block(kRowKernelThreads);
+    for (int64_t done = 0; done < tokens; done += kCodecMaxGroups * rows) {
+        const int count = int(std::min<int64_t>(tokens - done, kCodecMaxGroups * rows));
+        const dim3 grid(unsigned((count + rows - 1) / rows));
+        const uint8_t* from = codes + size_t(done) * hidden;
+        uint16_t* to = out + size_t(done) * hidden;
+        if (vector) hipLaunchKernelGGL(dequantize_kernel<true>, grid, block, 0, stream, from, scales + done, to, count, hidden, split);
+        else hipLaunchKernelGGL(dequantize_kernel<false>, grid, block, 0, stream, from, scales + done, to, count, hidden, split);
+        if (const hipError_t status = hipGetLastError(); status != hipSuccess) return status;
+    }
+    return hipSuccess;
 }
 
 }  // namespace pcie_ep

@@ -88,6 +88,25 @@ def test_codec_splits_rests_and_unaligned_arrays(hidden, offset):
     assert torch.equal(decoded.view(torch.int16), fp8_oracle.dequantize(want_codes, want_scales).view(torch.int16))
 
 
+def test_codec_takes_more_rows_than_one_launch_can():
+    """2^26 rows are 2^32 threads, which HIP refuses in one launch (2^24 to a launch, five rows in the last)."""
+    from pcie_ep.quantization import dequantize_fp8, quantize_fp8
+
+    tokens, hidden, part = (1 << 26) + 5, 8, 1 << 24
+    x = torch.empty(tokens, hidden, dtype=torch.bfloat16, device="cuda").normal_(generator=torch.Generator(device="cuda").manual_seed(3))
+    codes, scales = quantize_fp8(x)
+    decoded = dequantize_fp8(codes, scales)
+    for begin in range(0, tokens, part):
+        end = min(tokens, begin + part - 3)  # other rows to a launch than above
+        want_codes, want_scales = quantize_fp8(x[begin:end])
+        assert torch.equal(codes[begin:end], want_codes) and torch.equal(scales[begin:end], want_scales)
+        assert torch.equal(decoded[begin:end].view(torch.int16), dequantize_fp8(want_codes, want_scales).view(torch.int16))
+        edge = slice(max(0, begin - 9), begin + 9)
+        want_codes, want_scales = fp8_oracle.quantize(x[edge].cpu())
+        assert torch.equal(codes[edge].cpu(), want_codes) and torch.equal(scales[edge].cpu(), want_scales)
+        assert torch.equal(decoded[edge].cpu().view(torch.int16), fp8_oracle.dequantize(want_codes, want_scales).view(torch.int16))
+
+
 @pytest.mark.parametrize("hidden,channels", [(7168, 8), (136, 2), (129, 2)])
 def test_fp8_wire_dispatch(hidden, channels):
     world, experts, topk = 8, 256, 8
