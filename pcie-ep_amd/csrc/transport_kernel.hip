@@ -1372,7 +1372,8 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
 // LEFT in each direction: with rem_tx and rem_rx rows still unclaimed,
 //     transmitting wavefronts : receiving wavefronts = kTxWeight * rem_tx : kRxWeight * (rem_rx - lead)
 // (one wavefront's share of the link's write rate is about 4/9 of its share of
-// the read rate), re-evaluated before every row, so the writes are spread
+// the read rate; on the FP8 wire, where a transmitted row is half the bytes, read from
+// HBM once, it is about the same), re-evaluated before every claim, so the writes are spread
 // thinly over the whole dispatch whatever the routing's send/receive ratio is.
 // `lead` makes the transmit side end a little earlier than the receive side (by
 // the time the link needs for kTxLeadBytes, at most a quarter of the rows to
@@ -1390,7 +1391,12 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
 // wavefront must not bind itself to a transmit row for them) - but only a
 // ticket its producer has already reserved (head < tail), so it never commits
 // itself to a row that does not exist yet.
-constexpr int64_t kTxWeight = 9, kRxWeight = 4;
+// FP8 rows of 7168 columns, 8 ranks, us per dispatch with 9 : 4 (the writes crowd the beginning) and with 4 : 4: 2048
+// tokens top-8 1275 / 1257, 8192 tokens 5070 / 5030, 2000 tokens hotspot top-4 872 / 848, 64-token graph replay 79 / 79;
+// 4 ranks top-2, mostly transmitting, 427 / 427.  BF16, 2048 tokens: 2436 / 2441.
+template <bool kFp8>
+constexpr int64_t kTxWeight = kFp8 ? 4 : 9;
+constexpr int64_t kRxWeight = 4;
 constexpr int64_t kTxLeadBytes = 24 << 20;
 constexpr int kMinTxWaves = 16;
 constexpr uint64_t kIdleCrossoverUs = 30;
@@ -1435,7 +1441,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 bool prefer_tx = order < kMinTxWaves && 2 * order < waves;
                 if (tx_total >= 0 && rx_total >= 0) {
                     const int rx_rows = rx_total - rx_head - (lead < rx_total / 4 ? lead : rx_total / 4);
-                    const int64_t tx_left = tx_done ? 0 : kTxWeight * (tx_total - tx_head), rx_left = rx_rows > 0 ? kRxWeight * rx_rows : 0;
+                    const int64_t tx_left = tx_done ? 0 : kTxWeight<kFp8> * (tx_total - tx_head), rx_left = rx_rows > 0 ? kRxWeight * rx_rows : 0;
                     prefer_tx = rx_done || (tx_left > 0 && 2 * order < waves &&
                                             (order < kMinTxWaves || int64_t(order) * (tx_left + rx_left) < int64_t(waves) * tx_left));
                 }
