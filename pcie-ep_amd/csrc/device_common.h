@@ -587,9 +587,11 @@ struct HealthCheck {
 // however many expert rows it is scattered to.
 constexpr int kPassItems = 16;
 
-struct RowVectors {
-    u32x4 v[kPassItems];
+template <int kItems>
+struct RowItems {
+    u32x4 v[kItems];
 };
+typedef RowItems<kPassItems> RowVectors;
 
 // Vector index of item j for this lane: j * 64 + lane (consecutive lanes touch
 // consecutive 16-byte vectors: 1 KiB contiguous per instruction).
@@ -677,18 +679,24 @@ __device__ __forceinline__ void row_store_vector(void* row, int index, const u32
     if constexpr (kVector) __builtin_nontemporal_store(value, static_cast<u32x4*>(row) + index);
     else static_cast<u32x4_any*>(row)[index] = value;
 }
+// The ragged kernels take half as many vectors in a pass (BF16 rows of up to 4096 columns in one): with 128 registers
+// a lane, as many as when these rows moved element by element, a compute unit holds four of their workgroups, and a
+// dispatch fits the units it fitted then (1000 columns, 32 channels: 130 workgroups on 33 units; on 44 with three).
+constexpr int kRaggedItems = kPassItems / 2;
 template <bool kVector>
-__device__ __forceinline__ void row_load_pass(RowVectors& row, const uint16_t* source, int first, int count, int lane) {
+constexpr int kRowPass = kVector ? kPassItems : kRaggedItems;
+template <bool kVector>
+__device__ __forceinline__ void row_load_pass(RowItems<kRowPass<kVector>>& row, const uint16_t* source, int first, int count, int lane) {
 #pragma unroll
-    for (int j = 0; j < kPassItems; ++j) {
+    for (int j = 0; j < kRowPass<kVector>; ++j) {
         const int index = first + j * kWave + lane;
         if (index < count) row.v[j] = row_load_vector<kVector>(source, index);
     }
 }
 template <bool kVector>
-__device__ __forceinline__ void row_store_pass(const RowVectors& row, uint16_t* destination, int first, int count, int lane) {
+__device__ __forceinline__ void row_store_pass(const RowItems<kRowPass<kVector>>& row, uint16_t* destination, int first, int count, int lane) {
 #pragma unroll
-    for (int j = 0; j < kPassItems; ++j) {
+    for (int j = 0; j < kRowPass<kVector>; ++j) {
         const int index = first + j * kWave + lane;
         if (index < count) row_store_vector<kVector>(destination, index, row.v[j]);
     }

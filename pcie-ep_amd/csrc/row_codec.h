@@ -21,8 +21,8 @@ __device__ __forceinline__ float wave_max(float value) {
 template <bool kVector>
 __device__ __forceinline__ void copy_row(const uint16_t* input, uint16_t* output, int hidden, int lane) {
     const int vectors = hidden / 8, rest = row_rest<kVector>(hidden);
-    for (int first = 0; first < vectors; first += kPassItems * kWave) {
-        RowVectors row;
+    for (int first = 0; first < vectors; first += kRowPass<kVector> * kWave) {
+        RowItems<kRowPass<kVector>> row;
         row_load_pass<kVector>(row, input, first, vectors, lane);
         row_store_pass<kVector>(row, output, first, vectors, lane);
     }
@@ -37,11 +37,11 @@ __device__ __forceinline__ void copy_row_to_host(const uint16_t* input, __amdgpu
     const int vectors = hidden / 8, rest = row_rest<kVector>(hidden);
     u32x4 last = {0u, 0u, 0u, 0u};
     if (rest && lane == 0) last = load_rest(reinterpret_cast<const char*>(input + vectors * 8), rest);
-    for (int first = 0; first < vectors; first += kPassItems * kWave) {
-        RowVectors row;
+    for (int first = 0; first < vectors; first += kRowPass<kVector> * kWave) {
+        RowItems<kRowPass<kVector>> row;
         row_load_pass<kVector>(row, input, first, vectors, lane);
 #pragma unroll
-        for (int j = 0; j < kPassItems; ++j) {
+        for (int j = 0; j < kRowPass<kVector>; ++j) {
             const int index = first + j * kWave + lane;
             if (index < vectors) host_store_b128(slot, uint32_t(index) * 16u, row.v[j]);
         }
@@ -65,8 +65,10 @@ __device__ __forceinline__ u32x4 quantize_vector(const u32x4& lo, const u32x4& h
 
 // BF16 row from device memory as FP8 codes into a host slot; returns the row scale.  Every
 // lane takes 16 elements (two 16-byte loads) at a time to 16 codes (one 16-byte store).
-// A row of up to 8192 elements is read once and waits in registers for its maximum.  A
-// ragged row's last codes are stored as a whole vector, zeros behind the row.
+// A row of whole vectors and of up to 8192 elements is read once and waits in registers for its maximum; a ragged
+// one is read again (from the L2; 1536 tokens of 1000 columns 232 us per dispatch, 236 with the row held), which
+// leaves its kernel the registers for a fourth workgroup on a compute unit.  A ragged row's last codes are stored as
+// a whole vector, zeros behind the row.
 template <bool kVector>
 __device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane) {
     constexpr int kGroups = kPassItems / 2;  // 16-element groups a lane holds
@@ -80,7 +82,7 @@ __device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __a
         amax = vector_amax(vector_amax(amax, last_lo), last_hi);
     }
     RowVectors row;
-    const bool resident = groups <= kGroups * kWave;
+    const bool resident = kVector && groups <= kGroups * kWave;
     if (resident) {
 #pragma unroll
         for (int j = 0; j < kGroups; ++j) {
@@ -144,8 +146,8 @@ __device__ __forceinline__ void scatter_row(const uint16_t* input, uint16_t* out
     u32x4 last = {0u, 0u, 0u, 0u};
     if (rest && lane == 0) last = load_rest(reinterpret_cast<const char*>(input + vectors * 8), rest);
     // Also a row shorter than one vector takes one pass, for its rest.
-    for (int first = 0; first == 0 || first < vectors; first += kPassItems * kWave) {
-        RowVectors row;
+    for (int first = 0; first == 0 || first < vectors; first += kRowPass<kVector> * kWave) {
+        RowItems<kRowPass<kVector>> row;
         row_load_pass<kVector>(row, input, first, vectors, lane);
         uint64_t remaining = destinations;
         while (remaining) {

@@ -1118,9 +1118,12 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
     // Whole wire vectors of a row, and with a ragged row (any length and any alignment of the destination rows:
     // one more wire vector, of which `rest` bytes of BF16 are stored).  Byte by byte such a row was one host read
     // and one store per element: 1536 tokens of 1000 columns on the FP8 wire, 8 ranks, top-4: 606 -> 315 us per dispatch.
-    constexpr int kWireItems = kFp8 ? kPassItems / 2 : kPassItems;  // a code vector fills two BF16 vectors
-    constexpr int kRowItems = kWireItems / kRows;                   // wire vectors a lane holds of one row
-    constexpr int kOutPerWire = kFp8 ? 2 : 1;
+    constexpr int kWireItems = kFp8 ? kPassItems / 2 : kRowPass<kVector>;  // wire vectors a lane holds
+    constexpr int kRowItems = kWireItems / kRows;                          // of one row
+    constexpr int kOutPerWire = kFp8 ? 2 : 1;                              // a code vector fills two BF16 vectors
+    // FP8 rows are decoded as a whole, in place, and then stored destination by destination; ragged ones vector by
+    // vector as they are stored, to all destinations, in half the registers (row_load_pass says what those are for).
+    constexpr bool kDecodeInPlace = kFp8 && kVector, kDecodeAtStore = kFp8 && !kVector;
     constexpr int kWirePass = kRowItems * kWave;
     const int wire_vectors = kFp8 ? hidden / 16 : hidden / 8;
     const int rest = kVector ? 0 : (kFp8 ? hidden % 16 : hidden % 8) * 2;
@@ -1130,7 +1133,7 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
     // Metadata first (it arrives first), payload right behind it; lanes behind a row read 0.  A ragged row's last wire
     // vector is read whole: the slot's payload is padded to 16 bytes, the padding is not used.
     u32x4 meta_vector[kRows];
-    RowVectors row;
+    RowItems<kDecodeInPlace ? 2 * kWireItems : kWireItems> row;
 #pragma unroll
     for (int r = 0; r < kRows; ++r)
         meta_vector[r] = host_load_b128(host_resource(slot_base[r] + z.meta_offset, r < count ? uint32_t(z.meta_bytes) : 0u), uint32_t(lane) * 16u);
@@ -1262,7 +1265,7 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
             if (lane < count) host_store_release(slot_ack, ack_sequence);
             PCIE_EP_PROFILE(if (sampled) { wait_memory_ops(); profile.add(kProfileRxRequestSum, profile.now() - request_begin); })
         }
-        if constexpr (kFp8) {
+        if constexpr (kDecodeInPlace) {
             // 16 codes -> 16 BF16 (two 16-byte vectors); expanded in place from the top.
 #pragma unroll
             for (int j = kWireItems - 1; j >= 0; --j) {
@@ -1272,47 +1275,40 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
                 row.v[2 * j + 1] = hi;
             }
         }
+        // Item j of a row: wire vector i = first_wire + j * 64 + lane, which with FP8 holds elements [16 i, 16 i + 16).
+        const auto store_item = [&](uint16_t* output, int j, const u32x4* value) {
+            const int index = first_wire + j * kWave + lane;
+            if (index < wire_vectors) {
+#pragma unroll
+                for (int half = 0; half < kOutPerWire; ++half) row_store_vector<kVector>(output, index * kOutPerWire + half, value[half]);
+            } else if (!kVector && rest && index == wire_vectors) {
+                // The ragged row's last wire vector.
+                char* tail = reinterpret_cast<char*>(output) + size_t(wire_vectors) * (kOutPerWire * 16);
+                if (kFp8 && rest >= 16) {
+                    row_store_vector<false>(tail, 0, value[0]);
+                    store_rest(tail + 16, rest - 16, value[kOutPerWire - 1]);
+                } else {
+                    store_rest(tail, rest, value[0]);
+                }
+            }
+        };
 #pragma unroll
         for (int r = 0; r < kRows; ++r) {
             if (r >= count) break;
-            // The ragged row's last wire vector is item (wire_vectors - first_wire) / 64 of lane wire_vectors % 64.
-            u32x4 last[kOutPerWire] = {};
-            if (!kVector && rest && last_pass) {
-                const int item = (wire_vectors - first_wire) / kWave;
+            const uint64_t destinations = __ballot(my_row[r] >= 0);
+            constexpr int kAtATime = kDecodeAtStore ? 1 : kRowItems;  // items that go to one destination before the next
 #pragma unroll
-                for (int j = 0; j < kRowItems; ++j) {
-                    if (j != item) continue;
+            for (int item = 0; item < kRowItems; item += kAtATime) {
+                u32x4 decoded[2];
+                if constexpr (kDecodeAtStore) dequantize_vector(row.v[r * kRowItems + item], bits_float(scratch[r * meta_dwords + 2]), decoded[0], decoded[1]);
+                uint64_t remaining = destinations;
+                while (remaining) {
+                    const int branch = __builtin_ctzll(remaining);
+                    remaining &= remaining - 1;
+                    uint16_t* output = output_base + size_t(__shfl(my_row[r], branch)) * hidden;
 #pragma unroll
-                    for (int half = 0; half < kOutPerWire; ++half) last[half] = row.v[(r * kRowItems + j) * kOutPerWire + half];
-                }
-            }
-            uint64_t remaining = __ballot(my_row[r] >= 0);
-            while (remaining) {
-                const int branch = __builtin_ctzll(remaining);
-                remaining &= remaining - 1;
-                uint16_t* output = output_base + size_t(__shfl(my_row[r], branch)) * hidden;
-#pragma unroll
-                for (int j = 0; j < kRowItems; ++j) {
-                    const int index = first_wire + j * kWave + lane;
-                    if (index < wire_vectors) {
-                        // Wire vector i of an FP8 row holds elements [16 i, 16 i + 16): output vectors 2 i and 2 i + 1.
-#pragma unroll
-                        for (int half = 0; half < kOutPerWire; ++half)
-                            row_store_vector<kVector>(output, index * kOutPerWire + half, row.v[(r * kRowItems + j) * kOutPerWire + half]);
-                    }
-                }
-                if (!kVector && rest && last_pass && lane == wire_vectors % kWave) {
-                    char* tail = reinterpret_cast<char*>(output) + size_t(wire_vectors) * (kOutPerWire * 16);
-                    if constexpr (kFp8) {
-                        if (rest >= 16) {
-                            row_store_vector<false>(tail, 0, last[0]);
-                            store_rest(tail + 16, rest - 16, last[1]);
-                        } else {
-                            store_rest(tail, rest, last[0]);
-                        }
-                    } else {
-                        store_rest(tail, rest, last[0]);
-                    }
+                    for (int j = item; j < item + kAtATime; ++j)
+                        store_item(output, j, kDecodeAtStore ? decoded : &row.v[(r * kRowItems + j) * kOutPerWire]);
                 }
             }
         }
@@ -1541,7 +1537,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
 // no payload workgroups configured the control workgroups carry the payload
 // wavefronts themselves.
 template <bool kFp8, bool kVector, int kRows>
-__global__ void __launch_bounds__(kTransportMaxThreads) transport_kernel(DeviceState launch_state) {
+__global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transport_kernel(DeviceState launch_state) {
     // The launch argument is read where it lies, in the kernel-argument segment:
     // every field is then a scalar load from constant memory and every pointer in
     // it a global pointer.  A by-value copy would be a private object of 1 KB that

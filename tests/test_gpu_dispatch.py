@@ -26,7 +26,7 @@ def make_buffer(world=WORLD, rank=0, tmax=129, hidden=7168, topk=TOPK, experts=E
     from pcie_ep import HostStagedConfig, HostStagedEPBuffer
 
     config.setdefault("timeout_ms", 5000)
-    extra = {key: config.pop(key) for key in ("tx_waves", "rx_waves", "peer_threads", "worker_groups", "staging_numa_node") if key in config}
+    extra = {key: config.pop(key) for key in ("tx_waves", "rx_waves", "peer_threads", "worker_groups", "staging_numa_node", "comm_stream_cus") if key in config}
     return HostStagedEPBuffer(num_max_tokens_per_rank=tmax, hidden=hidden, num_topk=topk, num_experts=experts,
                               config=HostStagedConfig(**config), num_ranks=world, rank=rank, **extra)
 
@@ -191,10 +191,10 @@ def test_alignment_gaps_of_small_batches(world, experts, alignment, hidden, fuse
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("hidden", [1, 7, 9, 15, 1000, 1001, 8190, 8197])
+@pytest.mark.parametrize("hidden", [1, 7, 9, 15, 1000, 1001, 4095, 4097, 8190, 8197])
 def test_ragged_rows(hidden, fp8):
     """Rows with something behind their whole vectors, on either wire: 1 to 15 bytes, rows shorter than a
-    vector, the rest in the last item of a pass (8190) and alone in a pass of its own (8197, FP8); expanded
+    vector, the rest in the last item of a pass (4095, BF16; 8190, FP8) and alone in a pass of its own (4097 and 8197); expanded
     while receiving, by the expand kernel and not at all, with cleared gap rows between the rows; own
     tokens that start in the middle of a vector."""
     wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
@@ -214,6 +214,17 @@ def test_ragged_rows(hidden, fp8):
                 verify_dispatch(result, inputs, 0, 4, 16, 4, True, 1, False, fp8_wire=fp8)
                 verify_captured(buffer.peers, inputs, 0, 4, 16, 4, fp8_wire=fp8)
                 del result
+
+
+@pytest.mark.parametrize("hidden,fp8", [(1000, True), (4095, True), (7169, True), (1001, False), (4095, False)])
+def test_ragged_dispatches_fit_four_workgroups_to_a_compute_unit(hidden, fp8):
+    """`comm_stream_cus` is admitted by what a unit holds: a dispatch of ragged rows whose workgroups fit 32 units only
+    at four to a unit is accepted there, and runs."""
+    wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
+    with make_buffer(world=4, tmax=40, hidden=hidden, topk=4, experts=16, channels=16, comm_stream_cus=32, **wire) as buffer:
+        needed, resident = buffer.runtime.transport_residency(32)
+        assert 3 * 32 < needed <= resident
+        check_case(buffer, f"ragged-on-32-units-h{hidden}", [40, 9, 40, 33], alignment=16, fp8=fp8)
 
 
 @pytest.mark.parametrize("hidden,topk,fp8", [(1312, 8, False), (1313, 8, False), (4096, 8, True), (4095, 8, True), (4097, 8, True), (64, 13, False), (64, 14, True)])
