@@ -65,13 +65,12 @@ __device__ __forceinline__ u32x4 quantize_vector(const u32x4& lo, const u32x4& h
 
 // BF16 row from device memory as FP8 codes into a host slot; returns the row scale.  Every
 // lane takes 16 elements (two 16-byte loads) at a time to 16 codes (one 16-byte store).
-// A row of whole vectors and of up to 8192 elements is read once and waits in registers for its maximum; a ragged
+// A row of whole vectors and of up to kGroups * 1024 elements is read once and waits in registers for its maximum; a ragged
 // one is read again (from the L2; 1536 tokens of 1000 columns 232 us per dispatch, 236 with the row held), which
 // leaves its kernel the registers for a fourth workgroup on a compute unit.  A ragged row's last codes are stored as
 // a whole vector, zeros behind the row.
-template <bool kVector>
+template <bool kVector, int kGroups>  // kGroups: 16-element groups a lane holds
 __device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane) {
-    constexpr int kGroups = kPassItems / 2;  // 16-element groups a lane holds
     const int groups = hidden / 16, rest = kVector ? 0 : hidden % 16 * 2;
     float amax = 0.0f;
     u32x4 last_lo = {0u, 0u, 0u, 0u}, last_hi = {0u, 0u, 0u, 0u};
@@ -81,7 +80,7 @@ __device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __a
         if (rest > 16) last_hi = load_rest(from + 16, rest - 16);
         amax = vector_amax(vector_amax(amax, last_lo), last_hi);
     }
-    RowVectors row;
+    RowItems<2 * kGroups> row;
     const bool resident = kVector && groups <= kGroups * kWave;
     if (resident) {
 #pragma unroll
@@ -94,7 +93,7 @@ __device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __a
             }
         }
 #pragma unroll
-        for (int j = 0; j < kPassItems; ++j) amax = vector_amax(amax, row.v[j]);
+        for (int j = 0; j < 2 * kGroups; ++j) amax = vector_amax(amax, row.v[j]);
     } else {
         for (int index = lane; index < groups * 2; index += kWave) amax = vector_amax(amax, row_load_vector<false>(input, index));
     }

@@ -897,10 +897,13 @@ __device__ __forceinline__ void finish_role(const DeviceState& state, TransportQ
 // ---------------------------------------------------------------------------------------
 // TX payload worker
 // ---------------------------------------------------------------------------------------
-template <bool kFp8, bool kVector>
+// An instantiation for short rows (receive_batch) has none above kBatchedFp8Columns to hold: holding room for 8192
+// columns it kept 9 registers in scratch memory (1500 tokens of 2048 columns, 8 ranks: 362 us per dispatch, 352).
+template <bool kFp8, bool kVector, int kRows>
 __device__ __forceinline__ float tx_copy_row(const DeviceState& state, const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int lane) {
     const int hidden = state.z.dims.hidden;
-    if constexpr (kFp8) return quantize_row_to_host<kVector>(input, slot, hidden, lane);
+    constexpr int kGroups = (kRows > 1 ? kBatchedFp8Columns : kPassItems * kWave * 8) / (16 * kWave);
+    if constexpr (kFp8) return quantize_row_to_host<kVector, kGroups>(input, slot, hidden, lane);
     copy_row_to_host<kVector>(input, slot, hidden, lane);
     return 1.0f;
 }
@@ -912,7 +915,7 @@ struct WorkerCounters {
 
 // Moves the own token of transmit ticket `ticket_index` (already marked ready)
 // into its host slot and publishes it.  Returns false when the wavefront must stop.
-template <bool kFp8, bool kVector>
+template <bool kFp8, bool kVector, int kRows>
 __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int ticket_index, const Deadline& deadline,
                        WorkerCounters& counters PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
     const SegmentLayout& z = state.z;
@@ -985,7 +988,7 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         }
         if (lane == kWave - 1) test_delay(state.tx_delay);
         const __amdgpu_buffer_rsrc_t slot_resource = host_resource(slot_base, uint32_t(z.meta_offset + z.meta_bytes));
-        const float scale = tx_copy_row<kFp8, kVector>(state, state.x + size_t(token) * z.dims.hidden,
+        const float scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden,
                                                        host_resource(slot_base, uint32_t(z.meta_offset)), lane);
         if (lane == 0) scratch[2] = float_bits(scale);
         fence_lds();
@@ -1503,7 +1506,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                             if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows); profile.add(transmit ? kProfileTxRows : kProfileRxRows);)
             int count = 1;
             if (transmit) {
-                go_on = tx_row<kFp8, kVector>(state, q, scratch, lane, ticket_index, deadline, counters PCIE_EP_PROFILE(, profile, sampled));
+                go_on = tx_row<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, deadline, counters PCIE_EP_PROFILE(, profile, sampled));
             } else {
                 if constexpr (kRows > 1) {
                     const bool ready = lane < kRows && lane < end - ticket_index &&
