@@ -1424,7 +1424,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 const bool tx_backlog = tx_head < int(device_load(&q.tx_tail.value));
                 const int rx_tail = int(device_load(&q.rx_tail.value));
                 bool rx_backlog = rx_head < rx_tail;
-                // Receive tickets are there long before the first row may be requested (rx_row
+                // Receive tickets are there long before the first row may be requested (rx_rows
                 // holds the gate).  Only the first kPreGateRows of them are claimed ahead of
                 // it, by wavefronts that then wait with their addresses ready: if every
                 // wavefront did, they would all fire at once and each would have its first
@@ -1462,6 +1462,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 if (choice == 2) {
                     const int share = (rx_tail - rx_head) / waves;
                     claims = share < 1 ? 1 : (share < most_claims ? share : most_claims);
+                    if (kRows > 1 && !gate_seen && claims > kPreGateRows - rx_head) claims = kPreGateRows - rx_head;  // at least one is left: see rx_backlog
                 }
                 if (choice) idle_since = 0;
                 else {
