@@ -136,46 +136,52 @@ def test_previous_event_orders_the_dispatch_after_a_side_stream(inputs):
         assert buffer.get_comm_stream() is not torch.cuda.current_stream()
 
 
-def test_synchronous_dispatches_run_in_line_until_the_comm_stream_is_handed_out(inputs):
-    """Synchronous dispatches on two streams with asynchronous ones between them, every input still being
-    produced when its dispatch is called; then the communication stream is asked for: it comes after the
-    dispatch that ran on the caller's stream, and the next synchronous one runs on it."""
-    with make_buffer(tmax=TOKENS, hidden=HIDDEN, channels=2) as buffer:
-        x, idx, weights = (item.cuda() for item in inputs[0])
+def test_synchronous_dispatches_run_in_line_until_the_comm_stream_is_handed_out():
+    """Eager dispatches and graph replays of one buffer on two streams and the default one, synchronous and asynchronous,
+    submitted without waiting for any: each takes a few milliseconds (delayed rows), its input is still being produced
+    when it is called, and its routes are its own.  Then the communication stream is asked for: it comes after the dispatch
+    that ran on the caller's stream, and the next synchronous one runs on it.  All results are checked at the end."""
+    routes = [make_inputs(WORLD, [TOKENS] * WORLD, HIDDEN, EXPERTS, TOPK, seed=55 + step, gaussian=True)[0] for step in range(7)]
+    others = make_inputs(WORLD, [TOKENS] * WORLD, HIDDEN, EXPERTS, TOPK, seed=40, gaussian=True)[1:]
+    with make_buffer(tmax=TOKENS, hidden=HIDDEN, channels=2, output_pool_size=8, enable_graph=True, timeout_ms=20_000) as buffer:
         ordering = buffer._ordering
-        first, second = torch.cuda.Stream(), torch.cuda.Stream()
+        first, second, default = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.default_stream()
+        own = [tuple(item.cuda() for item in rank) for rank in routes]
+        fixed = tuple(item.clone() for item in own[0])
+        buffer.runtime.set_test_delays(0, 0, 0, 2_000_000)
+        graph = buffer.capture_dispatch(*fixed, do_expand=True)
+        sequence = [(1, first, "eager"), (2, second, "eager"), (3, second, "asynchronous"), (4, first, "eager"), (0, second, "replay"), (0, first, "replay"),
+                    (5, first, "asynchronous"), (0, default, "replay"), (6, default, "eager"), (0, second, "asynchronous replay"), (1, second, "eager")]
+        arm(buffer, [routes[0], *others], len(sequence) + 1)
         torch.cuda.synchronize()
+        outcomes = []
 
-        def step(stream, asynchronous=False):
-            arm(buffer, inputs)
+        def step(which, stream, kind):
             with torch.cuda.stream(stream):
-                staged = torch.zeros_like(x)
-                torch.cuda._sleep(4_000_000)
-                staged.copy_(x)
-                result = buffer.dispatch(staged, idx, weights, do_expand=True, async_with_compute_stream=asynchronous)
-                if asynchronous:
+                x, idx, weights = own[which]
+                if "replay" in kind:
+                    result = graph.replay(async_with_compute_stream="asynchronous" in kind)
+                else:
+                    staged = torch.zeros_like(x)
+                    torch.cuda._sleep(4_000_000)
+                    staged.copy_(x)
+                    result = buffer.dispatch(staged, idx, weights, do_expand=True, async_with_compute_stream=kind == "asynchronous")
+                if "asynchronous" in kind:
                     result[4].current_stream_wait()
-                copies = tuple(item.clone() for item in result[:3])
-            return result, copies
+                outcomes.append((which, tuple(item.clone() for item in result[:3]), result[3:]))
 
-        def check(result, copies):
-            buffer.peers.wait(30_000)
-            verify_dispatch((*copies, *result[3:]), inputs, 0, WORLD, EXPERTS, TOPK, True, 1, False)
-
-        for stream, asynchronous in ((first, False), (second, False), (second, True), (first, False), (first, False), (first, True)):
-            outcome = step(stream, asynchronous)
-            assert ordering._last[0] == ordering._key(ordering.stream if asynchronous else stream)
-            check(*outcome)
-            del outcome
-        result, copies = step(second)
+        for which, stream, kind in sequence:
+            step(which, stream, kind)
+            assert ordering._last[0] == ordering._key(ordering.stream if "asynchronous" in kind else stream), kind
+        assert not outcomes[-5][2][1].event.query()  # nothing has been waited for: several are pending
         comm = buffer.get_comm_stream()
         comm.synchronize()
-        assert result[4].event.query()
-        check(result, copies)
-        del result, copies
-        outcome = step(first)
+        assert outcomes[-1][2][1].event.query()
+        step(2, first, "eager")
         assert ordering._last[0] == ordering._key(comm)
-        check(*outcome)
+        buffer.peers.wait(30_000)
+        for which, copies, rest in outcomes:
+            verify_dispatch((*copies, *rest), [routes[which], *others], 0, WORLD, EXPERTS, TOPK, True, 1, False)
 
 
 def test_a_caller_on_few_compute_units_does_not_hold_the_dispatch(inputs):

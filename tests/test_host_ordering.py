@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import itertools
 import random
+import threading
 from types import SimpleNamespace
 
 import pytest
@@ -71,16 +72,45 @@ class Launched(Exception):
     pass
 
 
-@pytest.mark.parametrize("seed", range(6))
-def test_every_dispatch_comes_after_the_one_before(monkeypatch, seed):
-    rng = random.Random(seed)
-    for _ in range(50):
+@pytest.fixture
+def model(monkeypatch):
+    def start(rng):
         gpu = FakeGpu(rng)
         cuda = SimpleNamespace(Stream=gpu.Stream, Event=gpu.Event, stream=gpu.Current, current_stream=lambda device=None: gpu.current)
         monkeypatch.setattr(buffer_module, "torch", SimpleNamespace(cuda=cuda))
-        gpu.current = gpu.Stream()
         monkeypatch.setattr(buffer_module, "unit_mask", lambda stream: stream.units)
-        walk(gpu)
+        gpu.current = gpu.Stream()
+        return gpu
+
+    return start
+
+
+def test_a_thread_that_asks_for_the_stream_waits_for_the_dispatch_being_placed(model):
+    gpu = model(random.Random(0))
+    ordering = _Ordering(0)
+    seen = []
+    asking = threading.Thread(target=lambda: seen.append(ordering.expose().put()[1]))
+
+    def work(stream):
+        operation, _ = stream.put()
+        asking.start()
+        asking.join(0.1)  # it can not have been handed out: this dispatch has no completion event yet
+        assert not seen
+        return operation
+
+    operation, _, _ = ordering.submit(work, synchronous=True)
+    asking.join()
+    assert operation in seen[0]
+    place = []
+    ordering.submit(place.append, synchronous=True)
+    assert place == [ordering.stream]
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_every_dispatch_comes_after_the_one_before(model, seed):
+    rng = random.Random(seed)
+    for _ in range(50):
+        walk(model(rng))
 
 
 def walk(gpu):
