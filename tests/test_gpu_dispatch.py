@@ -230,13 +230,15 @@ def test_ragged_dispatches_fit_four_workgroups_to_a_compute_unit(hidden, fp8):
 @pytest.mark.parametrize("hidden,topk,fp8", [(1312, 8, False), (1313, 8, False), (4096, 8, True), (4095, 8, True), (4097, 8, True), (64, 13, False), (64, 14, True)])
 def test_short_rows_are_received_in_pairs(hidden, topk, fp8):
     """Both sides of the line up to which a wavefront takes two rows at a time: longest rows, ragged ones that
-    fill the last register of a pair's half, and the largest metadata.  More tokens than wavefronts, so that
-    pairs are taken; rings of one slot, where the second row of a pair comes only after the first was
-    acknowledged; both layouts."""
+    fill the last register of a pair's half, and the largest metadata; both layouts.  A wavefront claims its share of the
+    tickets that are there, so few wavefronts make the claims large: two of them take claims of eight (pairs of neighbouring
+    slots, of two channels and of two sources, and the odd last one) from rings of 64 slots, and what rings of one slot
+    hold, where the second row of a claim comes only after the first was acknowledged; four are the smallest ordinary workgroup."""
     wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
-    for channels, slots in ((16, 64), (2, 1)):
-        with make_buffer(tmax=400, hidden=hidden, topk=topk, channels=channels, payload_slots=slots, descriptor_slots=slots, **wire) as buffer:
-            tokens = [400] * 8 if slots > 1 else [40, 7, 40, 0, 1, 33, 40, 12]
+    for channels, slots, waves in ((16, 64, 1), (2, 1, 1), (3, 5, 2)):
+        with make_buffer(tmax=200, hidden=hidden, topk=topk, channels=channels, payload_slots=slots, descriptor_slots=slots, worker_groups=1,
+                         tx_waves=waves, rx_waves=waves, **wire) as buffer:
+            tokens = [200] * 8 if slots > 1 else [40, 7, 40, 0, 1, 33, 40, 12]
             check_case(buffer, f"pairs-h{hidden}-k{topk}-s{slots}", tokens, alignment=16, fp8=fp8)
             check_case(buffer, f"pairs-h{hidden}-k{topk}-s{slots}-unique", tokens, expand=False, seed=9, fp8=fp8)
 
