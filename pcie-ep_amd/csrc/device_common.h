@@ -24,7 +24,7 @@ constexpr int kWave = 64;
 #define PCIE_EP_PROFILE(...)
 #endif
 constexpr int kProfileFields = 32;
-constexpr int kProfileSampleStride = 8;  // every 8th row of a payload wavefront is timed in detail
+constexpr int kProfileSampleStride = 8;  // every 8th move (a row, or a pair of short received ones) of a payload wavefront is timed in detail
 
 constexpr uint64_t kPrefixFailed = ~uint64_t(0);
 // Set in the claim word of the receive prefixes once their producer has put its
@@ -267,7 +267,7 @@ enum ProfileField : int {
     kProfileFirstClaimNs = 4,
     kProfileLastRowNs,           // end of this wavefront's last row
     kProfileTxRows, kProfileRxRows,
-    kProfileSampledTxRows, kProfileSampledRxRows,  // rows timed in detail (every kProfileSampleStride-th)
+    kProfileSampledTxRows, kProfileSampledRxRows,  // moves timed in detail (every kProfileSampleStride-th)
     kProfileTicketWaitSum,       // claim -> ticket marked ready (all rows)
     kProfileIdleSum,             // time with nothing to claim
     kProfileTxFlowWaitSum,       // sampled: slot ACK / descriptor credit wait

@@ -1406,7 +1406,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
     const uint64_t epoch = dispatch_epoch(state);
     Deadline deadline(now_ticks());
     WorkerCounters counters;
-    PCIE_EP_PROFILE(RoleProfile profile(state.clock_khz); uint64_t idle_begin = 0; int rows_moved = 0;)
+    PCIE_EP_PROFILE(RoleProfile profile(state.clock_khz); uint64_t idle_begin = 0; int moves = 0;)
     bool prefixes_known = false, gate_open = false;
     const int lead = int(kTxLeadBytes / int64_t(state.z.meta_offset + state.z.meta_bytes));
     // A wavefront that may be wanted for transmitting binds itself to one batch at a time.
@@ -1503,8 +1503,8 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 if (broadcast_first(aborted(q) ? 1 : 0)) go_on = false;
                 break;
             }
-            PCIE_EP_PROFILE(profile.first(kProfileFirstTaggedNs); profile.add(kProfileTicketWaitSum, profile.now() - claim_begin); const bool sampled = rows_moved++ % kProfileSampleStride == 0;
-                            if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows); profile.add(transmit ? kProfileTxRows : kProfileRxRows);)
+            PCIE_EP_PROFILE(profile.first(kProfileFirstTaggedNs); profile.add(kProfileTicketWaitSum, profile.now() - claim_begin); const bool sampled = moves++ % kProfileSampleStride == 0;
+                            if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows);)
             int count = 1;
             if (transmit) {
                 go_on = tx_row<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, deadline, counters PCIE_EP_PROFILE(, profile, sampled));
@@ -1517,7 +1517,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 go_on = rx_rows<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, count, counters, deadline, gate_open, prefixes_known PCIE_EP_PROFILE(, profile, sampled));
             }
             ticket_index += count;
-            PCIE_EP_PROFILE(profile.last(kProfileLastRowNs);)
+            PCIE_EP_PROFILE(profile.add(transmit ? kProfileTxRows : kProfileRxRows, uint64_t(count)); profile.last(kProfileLastRowNs);)
         }
         if (!go_on) break;
     }
@@ -1533,7 +1533,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
         }
         if (counters.reads) atomicAdd(stats + kStatHostReads, static_cast<unsigned long long>(counters.reads));
     }
-    PCIE_EP_PROFILE(profile.values[kProfileItems] = uint64_t(rows_moved); profile.save(state.profiling, 2 * state.z.dims.channels + order, lane);)
+    PCIE_EP_PROFILE(profile.values[kProfileItems] = uint64_t(moves); profile.save(state.profiling, 2 * state.z.dims.channels + order, lane);)
 }
 
 // Workgroup b < C is the control workgroup of channel b (wavefront 0 TX control,

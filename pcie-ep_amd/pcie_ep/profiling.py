@@ -12,6 +12,8 @@ receive prefixes ``[2C + W + 2]`` (the last two hold records only where those ar
 roles of their own; ``read`` folds their stamps into the leader's and RX control 0's).  Stamps (``*_ns``) are
 nanoseconds of the device wall clock, sums are accumulated nanoseconds; a zero
 stamp means the event did not happen.  Intervals of different roles overlap.
+A payload wavefront's ``items`` and ``sampled_*`` count moves: one row, or up to two short rows
+received together; ``tx_rows`` and ``rx_rows`` count rows.
 """
 
 from __future__ import annotations

@@ -12,6 +12,11 @@ and compared too (TX parity).
 
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -241,6 +246,31 @@ def test_short_rows_are_received_in_pairs(hidden, topk, fp8):
             tokens = [200] * 8 if slots > 1 else [40, 7, 40, 0, 1, 33, 40, 12]
             check_case(buffer, f"pairs-h{hidden}-k{topk}-s{slots}", tokens, alignment=16, fp8=fp8)
             check_case(buffer, f"pairs-h{hidden}-k{topk}-s{slots}-unique", tokens, expand=False, seed=9, fp8=fp8)
+
+
+def test_profiling_records_count_every_row_of_a_pair():
+    """The per-role records (profiling build, a process of its own): rows received and transmitted equal the
+    dispatch's statistics, and fewer moves than rows: pairs are taken."""
+    program = """
+import sys
+sys.path[:0] = ["tests", "pcie-ep_amd", "."]
+import torch
+from helpers import make_inputs, run_dispatch
+from test_gpu_dispatch import make_buffer
+from pcie_ep import profiling
+with make_buffer(tmax=200, hidden=64, channels=4, payload_slots=64, descriptor_slots=64, worker_groups=1, tx_waves=1, rx_waves=1) as buffer:
+    result, _ = run_dispatch(buffer, make_inputs(8, [200] * 8, 64, 256, 8))
+    records = profiling.read(buffer.runtime)["workers"]
+    total = {name: int(records[:, profiling.WORKER.index(name)].sum()) for name in ("items", "tx_rows", "rx_rows")}
+    stats = result[3].stats.cpu().tolist()
+    assert (total["tx_rows"], total["rx_rows"]) == (stats[0], stats[1]), (total, stats)
+    assert total["items"] < 0.75 * stats[1] + stats[0], (total, stats)
+    print("counted", total, flush=True)
+"""
+    run = subprocess.run([sys.executable, "-u", "-c", program], cwd=Path(__file__).resolve().parents[1], env=dict(os.environ, PCIE_EP_PROFILING="1"),
+                         capture_output=True, text=True, timeout=100)
+    print(run.stdout, run.stderr, flush=True)
+    assert run.returncode == 0 and "counted" in run.stdout
 
 
 def test_numa_bound_staging_segments():
