@@ -110,6 +110,9 @@ class _Ordering:
                 self.stream.wait_event(self._last[1])
         return self.stream
 
+    def last_ran_on(self, stream: Any) -> bool:
+        return self._last[0] == self._key(stream)
+
     def _holds_dispatch(self, caller: Any) -> bool:
         # The default stream cannot be masked.
         return int(caller.cuda_stream) == 0 or (self._units is not None and unit_mask(caller) == self._units)

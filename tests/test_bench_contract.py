@@ -43,6 +43,7 @@ def test_one_json_line_with_roofline_and_cpu_baseline():
     events = record["dispatch_event_us"]
     assert 0 < events["p50"] <= events["p95"] and events["mean"] > 0
     assert record["dispatch_sync_us"] > 0  # reported up to 512 tokens, where the submission cost shows
+    assert record["dispatch_sync_in_line"] is True  # the default path, not the one behind a communication stream that was asked for
     # A counted figure is reported only with a summary measured on these kernel sources; otherwise null, with a note.
     assert len(record["sources"]) == 16
     assert "traffic" in roofline and (roofline["traffic"] is not None or "traffic_note" in roofline)
