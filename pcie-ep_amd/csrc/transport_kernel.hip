@@ -1278,23 +1278,6 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
                 row.v[2 * j + 1] = hi;
             }
         }
-        // Item j of a row: wire vector i = first_wire + j * 64 + lane, which with FP8 holds elements [16 i, 16 i + 16).
-        const auto store_item = [&](uint16_t* output, int j, const u32x4* value) {
-            const int index = first_wire + j * kWave + lane;
-            if (index < wire_vectors) {
-#pragma unroll
-                for (int half = 0; half < kOutPerWire; ++half) row_store_vector<kVector>(output, index * kOutPerWire + half, value[half]);
-            } else if (!kVector && rest && index == wire_vectors) {
-                // The ragged row's last wire vector.
-                char* tail = reinterpret_cast<char*>(output) + size_t(wire_vectors) * (kOutPerWire * 16);
-                if (kFp8 && rest >= 16) {
-                    row_store_vector<false>(tail, 0, value[0]);
-                    store_rest(tail + 16, rest - 16, value[kOutPerWire - 1]);
-                } else {
-                    store_rest(tail, rest, value[0]);
-                }
-            }
-        };
 #pragma unroll
         for (int r = 0; r < kRows; ++r) {
             if (r >= count) break;
@@ -1310,8 +1293,29 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
                     remaining &= remaining - 1;
                     uint16_t* output = output_base + size_t(__shfl(my_row[r], branch)) * hidden;
 #pragma unroll
-                    for (int j = item; j < item + kAtATime; ++j)
-                        store_item(output, j, kDecodeAtStore ? decoded : &row.v[(r * kRowItems + j) * kOutPerWire]);
+                    for (int j = item; j < item + kAtATime; ++j) {
+                        // Wire vector i of an FP8 row holds elements [16 i, 16 i + 16): output vectors 2 i and 2 i + 1.
+                        const int index = first_wire + j * kWave + lane;
+                        const int held = (r * kRowItems + j) * kOutPerWire;
+                        if (index < wire_vectors) {
+#pragma unroll
+                            for (int half = 0; half < kOutPerWire; ++half)
+                                row_store_vector<kVector>(output, index * kOutPerWire + half, kDecodeAtStore ? decoded[half] : row.v[held + half]);
+                        }
+                        if constexpr (!kVector) {
+                            // The ragged row's last wire vector.
+                            if (rest && index == wire_vectors) {
+                                char* tail = reinterpret_cast<char*>(output) + size_t(wire_vectors) * (kOutPerWire * 16);
+                                const u32x4 value = kDecodeAtStore ? decoded[0] : row.v[held];
+                                if (kFp8 && rest >= 16) {
+                                    row_store_vector<false>(tail, 0, value);
+                                    store_rest(tail + 16, rest - 16, decoded[1]);
+                                } else {
+                                    store_rest(tail, rest, value);
+                                }
+                            }
+                        }
+                    }
                 }
             }
         }
