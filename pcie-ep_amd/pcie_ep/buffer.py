@@ -50,8 +50,8 @@ class _Ordering:
     caller's stream waits for the result in any case) runs on the caller's stream itself as
     long as the communication stream is this object's own and nobody has asked for it.  What
     the caller's stream has done is then in front of the dispatch and what it does next is
-    behind it without a wait across streams each way, which took 17 us of a 70 us dispatch of
-    16 tokens.  Once `expose` has handed the stream out, a program may have put work of its own
+    behind it without a wait across streams each way, which took 17 us of 70 when dispatches of
+    16 tokens followed each other (less of a lone one: part of it hides behind the submission).  Once `expose` has handed the stream out, a program may have put work of its own
     on it or rely on a dispatch being there: every later dispatch runs on it.  Nor is the
     caller's stream used where several ranks' kernels wait for each other on one GPU
     (`in_line` false): which streams those run on is their caller's arrangement.
