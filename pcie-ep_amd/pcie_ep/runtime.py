@@ -273,6 +273,10 @@ class NativeRuntime:
         }
         return result
 
+    def graph_arguments(self) -> _native.DispatchArgs:
+        """A copy of the arguments of the dispatch captured last (the graph result pool's)."""
+        return _native.DispatchArgs.from_buffer_copy(self._pools[self.config.output_pool_size].arguments)
+
     # ---- diagnostics and hooks ----------------------------------------------------------
     def pool_debug(self) -> list:
         return [pool.references() for pool in self._pools]
