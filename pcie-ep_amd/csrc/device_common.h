@@ -309,6 +309,7 @@ struct RoleProfile {
     __device__ __forceinline__ uint64_t now() const {
         const uint64_t ticks = wall_clock64();
         asm volatile("" ::: "memory");
+        if (khz == 100000) return ticks * 10;  // the usual rate, without a division
         return ticks / khz * 1000000ull + ticks % khz * 1000000ull / khz;
     }
     __device__ __forceinline__ void first(int field) { if (!values[field]) values[field] = now(); }
@@ -393,6 +394,12 @@ __device__ __forceinline__ u32x4 host_load_b128_at(const void* address) {
     u32x4 value;
     asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1\n\ts_waitcnt vmcnt(0)" : "=v"(value) : "v"(address) : "memory");
     return value;
+}
+
+// One 16-byte store to host memory at a per-lane address.  The instruction reads its data registers for one cycle
+// longer than a narrower one: nothing may write them right behind it.
+__device__ __forceinline__ void host_store_b128_at(void* address, u32x4 value) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(address), "v"(value) : "memory");
 }
 
 __device__ __forceinline__ void wait_memory_ops() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }

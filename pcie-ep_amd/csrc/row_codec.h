@@ -32,20 +32,22 @@ __device__ __forceinline__ void copy_row(const uint16_t* input, uint16_t* output
 
 // BF16 row from device memory into a host slot.  A ragged row's last vector is stored
 // whole, zeros behind the row: the slot's payload is padded to 16 bytes.
-template <bool kVector>
-__device__ __forceinline__ void copy_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane) {
+template <bool kVector, typename BeforeStores>
+__device__ __forceinline__ void copy_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane, BeforeStores before_stores) {
     const int vectors = hidden / 8, rest = row_rest<kVector>(hidden);
     u32x4 last = {0u, 0u, 0u, 0u};
     if (rest && lane == 0) last = load_rest(reinterpret_cast<const char*>(input + vectors * 8), rest);
     for (int first = 0; first < vectors; first += kRowPass<kVector> * kWave) {
         RowItems<kRowPass<kVector>> row;
         row_load_pass<kVector>(row, input, first, vectors, lane);
+        if (first == 0) before_stores();
 #pragma unroll
         for (int j = 0; j < kRowPass<kVector>; ++j) {
             const int index = first + j * kWave + lane;
             if (index < vectors) host_store_b128(slot, uint32_t(index) * 16u, row.v[j]);
         }
     }
+    if (vectors == 0) before_stores();
     if (rest && lane == 0) host_store_b128(slot, uint32_t(vectors) * 16u, last);
 }
 
@@ -69,8 +71,8 @@ __device__ __forceinline__ u32x4 quantize_vector(const u32x4& lo, const u32x4& h
 // one is read again (from the L2; 1536 tokens of 1000 columns 232 us per dispatch, 236 with the row held), which
 // leaves its kernel the registers for a fourth workgroup on a compute unit.  A ragged row's last codes are stored as
 // a whole vector, zeros behind the row.
-template <bool kVector, int kGroups>  // kGroups: 16-element groups a lane holds
-__device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane) {
+template <bool kVector, int kGroups, typename BeforeStores>  // kGroups: 16-element groups a lane holds
+__device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int hidden, int lane, BeforeStores before_stores) {
     const int groups = hidden / 16, rest = kVector ? 0 : hidden % 16 * 2;
     float amax = 0.0f;
     u32x4 last_lo = {0u, 0u, 0u, 0u}, last_hi = {0u, 0u, 0u, 0u};
@@ -102,6 +104,7 @@ __device__ __forceinline__ float quantize_row_to_host(const uint16_t* input, __a
     // Multiply by the correctly rounded FP32 reciprocal, as the reference does
     // (quantization.cuh:66; pcie_ep/quantization.py:27-29), not a division per element.
     const float inverse = 1.0f / scale;
+    before_stores();
     if (resident) {
 #pragma unroll
         for (int j = 0; j < kGroups; ++j) {

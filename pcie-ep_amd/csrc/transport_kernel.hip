@@ -72,9 +72,13 @@ namespace {
 
 constexpr int kScratchDwords = kReceiveScratchDwords;  // per wavefront: slot metadata records (of one or kMaxReceiveBatch rows)
 constexpr int kMaxWaves = 12;
+// What a payload wavefront owes the other ends (see Owed): slot ACKs (address, token), then a transmitted row's
+// channel, slot, token and descriptor ordinal per endpoint; behind them the wavefront's counters.
+constexpr int kOwedRow = 4 * kMaxReceiveBatch, kOwedDescriptors = kOwedRow + 4, kOwedCounts = kOwedDescriptors + kMaxEndpoints, kOwedDwords = kOwedCounts + 8;
 
 struct WaveScratch {
     uint32_t words[kMaxWaves][kScratchDwords];
+    uint32_t owed[kMaxWaves][kOwedDwords];
 };
 
 // Local time only: payload workers never scan the host abort flags themselves
@@ -146,8 +150,9 @@ __device__ __forceinline__ int claim_tickets(QueueCounter& head, int count, int 
     if (lane == 0) ticket = device_add(&head.value, uint32_t(count));
     return broadcast_first(int(ticket));
 }
+template <typename BeforeWaiting>
 __device__ __forceinline__ int wait_ticket(const DeviceState& state, TransportQueues& q, const uint64_t* ready, QueueCounter& head, int ticket,
-                                  uint64_t epoch, int lane, const Deadline& deadline) {
+                                  uint64_t epoch, int lane, const Deadline& deadline, BeforeWaiting before_waiting) {
     while (true) {
         int action = 0;
         if (lane == 0) {
@@ -165,6 +170,7 @@ __device__ __forceinline__ int wait_ticket(const DeviceState& state, TransportQu
         }
         action = broadcast_first(action);
         if (action) return action;
+        before_waiting();
         backoff();
     }
 }
@@ -899,25 +905,69 @@ __device__ __forceinline__ void finish_role(const DeviceState& state, TransportQ
 // ---------------------------------------------------------------------------------------
 // An instantiation for short rows (receive_batch) has none above kBatchedFp8Columns to hold: holding room for 8192
 // columns it kept 9 registers in scratch memory (1500 tokens of 2048 columns, 8 ranks: 362 us per dispatch, 352).
-template <bool kFp8, bool kVector, int kRows>
-__device__ __forceinline__ float tx_copy_row(const DeviceState& state, const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int lane) {
+template <bool kFp8, bool kVector, int kRows, typename BeforeStores>
+__device__ __forceinline__ float tx_copy_row(const DeviceState& state, const uint16_t* input, __amdgpu_buffer_rsrc_t slot, int lane, BeforeStores before_stores) {
     const int hidden = state.z.dims.hidden;
     constexpr int kGroups = (kRows > 1 ? kBatchedFp8Columns : kPassItems * kWave * 8) / (16 * kWave);
-    if constexpr (kFp8) return quantize_row_to_host<kVector, kGroups>(input, slot, hidden, lane);
-    copy_row_to_host<kVector>(input, slot, hidden, lane);
+    if constexpr (kFp8) return quantize_row_to_host<kVector, kGroups>(input, slot, hidden, lane, before_stores);
+    copy_row_to_host<kVector>(input, slot, hidden, lane, before_stores);
     return 1.0f;
 }
 
-// Counters a payload wavefront accumulates over the rows it moves, flushed once when it ends.
-struct WorkerCounters {
-    int64_t writes = 0, deliveries = 0, published = 0, credit_miss = 0, reads = 0;
+// What a payload wavefront still owes the other ends of the rows it has moved: a received row's slot ACK (lane r: row
+// r's), a transmitted row's descriptors (lane e: endpoint e's) and its retirement.  A store to host memory is
+// acknowledged one loaded round trip later, and vector memory operations complete in order: stored as soon as the row has
+// been moved, it would hold up every step towards the next row - the look at the queues, the claim, the ticket - by that
+// round trip.  The wavefront therefore stores it when it has the next row's ticket and is about to
+// touch the link again, or finds that there is no next row, and always before it waits for anybody else.
+// The record lies in LDS: in registers it would be alive across the row's vectors.
+struct Owed {
+    uint32_t* record;
+    int acks = 0;       // received rows
+    bool row = false;   // a transmitted one
+    // Few rows of the direction are left (or nobody knows yet): there may be no next row to put it off to, and the
+    // other end is waited for.
+    bool prompt = true;
 };
+// The row's own loads / stores must have completed: every caller is behind a wait_memory_ops() that is behind the row.
+__device__ __forceinline__ void settle_acks(const DeviceState& state, Owed& owed, int lane) {
+    if (lane < owed.acks) {
+        const uint32_t* ack = owed.record + 4 * lane;
+        typedef uint64_t __attribute__((address_space(1))) * GlobalWord;
+        __hip_atomic_store((GlobalWord)(uint64_t(ack[0]) | uint64_t(ack[1]) << 32), sequence(dispatch_epoch(state), int(ack[2])), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    owed.acks = 0;
+}
+__device__ __forceinline__ void settle(const DeviceState& state, TransportQueues& q, Owed& owed, int lane) {
+    settle_acks(state, owed, lane);
+    if (!owed.row) return;
+    owed.row = false;
+    const int channel = broadcast_first(int(owed.record[kOwedRow]));
+    const int ordinal = lane < state.z.endpoints ? int(owed.record[kOwedDescriptors + lane]) : -1;
+    if (ordinal >= 0) {
+        // READY, slot and token in one 16-byte store: nothing to order inside the entry.
+        const uint64_t ready = sequence(dispatch_epoch(state), ordinal);
+        host_store_b128_at(descriptor_at(state.z, state.seg[state.local_rank], channel, lane, ordinal),
+                           u32x4{uint32_t(ready), uint32_t(ready >> 32), owed.record[kOwedRow + 1], owed.record[kOwedRow + 2]});
+    }
+    if (lane == 0) {
+        if (owed.record[kOwedRow + 3]) state.prefix_tx_timestamps_ns[(channel + 1) * 2 + 1] = ticks_to_ns(state, now_ticks());
+        device_add(&q.tx_retired[channel].value, 1u);
+    }
+}
+
+// Counters a payload wavefront accumulates over the rows it moves, flushed once when it ends (in LDS, as the record above).
+enum WorkerCount : int { kCountWrites = 0, kCountDeliveries, kCountPublished, kCountCreditMiss, kCountReads, kWorkerCounts };
+__device__ __forceinline__ void count_rows(uint32_t* record, WorkerCount which, int amount, int lane) {
+    if (lane == 0) record[kOwedCounts + which] += uint32_t(amount);
+}
 
 // Moves the own token of transmit ticket `ticket_index` (already marked ready)
-// into its host slot and publishes it.  Returns false when the wavefront must stop.
+// into its host slot; what publishes it is left to settle().  Returns false when the wavefront must stop.
 template <bool kFp8, bool kVector, int kRows>
 __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int ticket_index, const Deadline& deadline,
-                       WorkerCounters& counters PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
+                       Owed& owed PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
     const SegmentLayout& z = state.z;
     const int ranks = z.dims.num_ranks, topk = z.dims.topk, me = state.local_rank;
     const int endpoint_count = z.endpoints;
@@ -959,7 +1009,8 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
             if (!slot_ok) slot_ok = host_load(ack_at(z, own, channel, slot, lane)) == previous_sequence;
             if (!credit_ok) credit_ok = credit_covers(host_load(credit_at(z, own, channel, lane)), epoch, my_descriptor, descriptors);
             if (__all(slot_ok && credit_ok)) break;
-            ++counters.credit_miss;
+            count_rows(owed.record, kCountCreditMiss, 1, lane);
+            settle(state, q, owed, lane);
             if (broadcast_first((aborted(q) || deadline.expired(state)) ? 1 : 0)) {
                 stop = true;
                 break;
@@ -988,31 +1039,34 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         }
         if (lane == kWave - 1) test_delay(state.tx_delay);
         const __amdgpu_buffer_rsrc_t slot_resource = host_resource(slot_base, uint32_t(z.meta_offset + z.meta_bytes));
-        const float scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden,
-                                                       host_resource(slot_base, uint32_t(z.meta_offset)), lane);
+        const float scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden, host_resource(slot_base, uint32_t(z.meta_offset)), lane,
+                                                       [&] { settle(state, q, owed, lane); });
         if (lane == 0) scratch[2] = float_bits(scale);
         fence_lds();
         if (lane == meta_dwords - 1 || (lane == kWave - 1 && meta_dwords > kWave)) test_delay(state.metadata_delay);
         for (int index = lane; index < meta_dwords; index += kWave)
             host_store_b32(slot_resource, uint32_t(z.meta_offset + index * 4), scratch[index]);
         // Every lane's payload and metadata stores have been acknowledged before
-        // any lane publishes a descriptor (the counters are wave-wide).
-        wait_memory_ops();
-        PCIE_EP_PROFILE(if (sampled) profile.add(kProfileTxCopySum, profile.now() - copy_begin);)
-        if (targeted) {
-            // READY, slot and token in one 16-byte store: nothing to order inside the entry.
-            const uint64_t ready = sequence(epoch, my_descriptor);
-            const u32x4 entry = {uint32_t(ready), uint32_t(ready >> 32), uint32_t(slot), uint32_t(token)};
-            host_store_b128(host_resource(descriptor_at(z, own, channel, lane, my_descriptor), 16), 0, entry);
+        // any lane publishes a descriptor (the counters are wave-wide): see settle().
+        PCIE_EP_PROFILE(if (sampled) { wait_memory_ops(); profile.add(kProfileTxCopySum, profile.now() - copy_begin); })
+        if (lane < endpoint_count) owed.record[kOwedDescriptors + lane] = uint32_t(targeted ? my_descriptor : -1);
+        if (lane == 0) {
+            owed.record[kOwedRow] = uint32_t(channel);
+            owed.record[kOwedRow + 1] = uint32_t(slot);
+            owed.record[kOwedRow + 2] = uint32_t(token);
+            owed.record[kOwedRow + 3] = ordinal == 0 ? 1u : 0u;
         }
-        if (ordinal == 0 && lane == 0) state.prefix_tx_timestamps_ns[(channel + 1) * 2 + 1] = ticks_to_ns(state, now_ticks());
-        ++counters.writes;
+        owed.row = true;
+        count_rows(owed.record, kCountWrites, 1, lane);
         // Logical deliveries count destination ranks; a relay endpoint stands for
         // all targeted ranks of its domain with one descriptor.
-        counters.deliveries += __popc(state.plan_mask[token] & ~(1u << me));
-        counters.published += __popc(endpoints);
+        count_rows(owed.record, kCountDeliveries, __popc(scratch[1] & ~(1u << me)), lane);
+        count_rows(owed.record, kCountPublished, __popc(endpoints), lane);
         fence_lds();  // scratch is reused by the next ticket
-        if (lane == 0) device_add(&q.tx_retired[channel].value, 1u);
+        if (owed.prompt) {
+            wait_memory_ops();
+            settle(state, q, owed, lane);
+        }
     }
     return true;
 }
@@ -1031,7 +1085,7 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
 // are mostly neighbouring slots of one source, so that their ACKs leave as one store.
 template <bool kFp8, bool kVector, int kRows>
 __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int first_ticket, int count,
-                       WorkerCounters& counters, const Deadline& deadline, bool& gate_open, bool& prefixes_known PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
+                       Owed& owed, const Deadline& deadline, bool& gate_open, bool& prefixes_known PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
     const SegmentLayout& z = state.z;
     const int topk = z.dims.topk, me = state.local_rank, local = z.local_experts;
     const int hidden = z.dims.hidden;
@@ -1053,8 +1107,9 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
     // this wavefront is still moving the rows.
     wait_memory_ops();
     if (lane < count) device_store(q.rx_taken + (first_ticket + lane) % kRing, sequence(epoch, first_ticket + lane));
-    uint64_t* slot_ack = nullptr;  // lane r: row r's
-    uint64_t ack_sequence = 0;
+    settle(state, q, owed, lane);  // in front of this row's requests and before any wait below
+    fence_lds();
+    uint32_t* owed_ack = owed.record + 4 * (lane < kRows ? lane : 0);
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
         source[r] = entry(r, 0);
@@ -1067,8 +1122,10 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
         uint64_t* ack = replica ? replica_ack_at(z, state.seg[source[r]], channel[r], z.dims.rank_domain[me], slot, me)
                                 : ack_at(z, state.seg[source[r]], channel[r], slot, me);
         if (lane == r) {
-            slot_ack = ack;
-            ack_sequence = payload_sequence[r];
+            // (payload_sequence[r] is this token's: checked below.)
+            owed_ack[0] = uint32_t(reinterpret_cast<uint64_t>(ack));
+            owed_ack[1] = uint32_t(reinterpret_cast<uint64_t>(ack) >> 32);
+            owed_ack[2] = uint32_t(ticket_token[r]);
         }
     }
     if (lane == kWave - 1) test_delay(state.rx_delay);
@@ -1264,9 +1321,11 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
         }
         const bool last_pass = kRows > 1 || first_wire + kWirePass >= wire_total;
         if (last_pass) {
-            // All loads of the staged rows have returned: release the host slots.
-            if (lane < count) host_store_release(slot_ack, ack_sequence);
-            PCIE_EP_PROFILE(if (sampled) { wait_memory_ops(); profile.add(kProfileRxRequestSum, profile.now() - request_begin); })
+            // All loads of the staged rows have returned: the host slots may be released.
+            wait_memory_ops();
+            owed.acks = count;
+            if (owed.prompt) settle_acks(state, owed, lane);
+            PCIE_EP_PROFILE(if (sampled) profile.add(kProfileRxRequestSum, profile.now() - request_begin);)
         }
         if constexpr (kDecodeInPlace) {
             // 16 codes -> 16 BF16 (two 16-byte vectors); expanded in place from the top.
@@ -1350,7 +1409,7 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
             }
         }
     }
-    counters.reads += count;
+    count_rows(owed.record, kCountReads, count, lane);
     PCIE_EP_PROFILE(if (sampled) profile.add(kProfileRxScatterSum, profile.now() - request_begin);)
     fence_lds();  // scratch is reused by the next tickets
     if (lane < count) {
@@ -1406,19 +1465,21 @@ constexpr uint64_t kIdleCrossoverUs = 30;
 constexpr int kPreGateRows = 32;
 
 template <bool kFp8, bool kVector, int kRows>
-__device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int order, int waves) {
+__device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, uint32_t* owed_record, int lane, int order, int waves) {
     const uint64_t epoch = dispatch_epoch(state);
     Deadline deadline(now_ticks());
-    WorkerCounters counters;
+    if (lane < kWorkerCounts) owed_record[kOwedCounts + lane] = 0;
+    Owed owed{owed_record};
     PCIE_EP_PROFILE(RoleProfile profile(state.clock_khz); uint64_t idle_begin = 0; int moves = 0;)
     bool prefixes_known = false, gate_open = false;
     const int lead = int(kTxLeadBytes / int64_t(state.z.meta_offset + state.z.meta_bytes));
     // A wavefront that may be wanted for transmitting binds itself to one batch at a time.
     const int most_claims = 2 * order < waves || kRows == 1 ? kRows : kReceiveClaims;
     uint64_t idle_since = 0;  // 0: the last look found work
-    while (true) {
+    bool go_on = true;
+    while (go_on) {
         // 0: nothing to do now, 1: transmit, 2: receive, -1: both directions are finished or the kernel aborts.
-        int choice = 0, claims = 1;
+        int choice = 0, claims = 1, prompt = 1;
         PCIE_EP_PROFILE(const uint64_t look_begin = profile.now();)
         int gate_seen = gate_open ? 1 : 0;
         if (lane == 0) {
@@ -1462,6 +1523,8 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                     // therefore never do while a row may still come in.
                     if (own_done || (prefer_tx && now - idle_since > kIdleCrossoverUs * state.clock_khz / 1000)) choice = prefer_tx ? 2 : 1;
                 }
+                const int total = choice == 1 ? tx_total : rx_total;
+                prompt = total < 0 || total - (choice == 1 ? tx_head : rx_head) <= waves;
                 // A receiving wavefront takes its share of the tickets that are there, at most most_claims.
                 if (choice == 2) {
                     const int share = (rx_tail - rx_head) / waves;
@@ -1483,6 +1546,8 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
         gate_open = broadcast_first(gate_seen) != 0;
         if (choice < 0) break;
         if (choice == 0) {
+            wait_memory_ops();
+            settle(state, q, owed, lane);
             PCIE_EP_PROFILE(if (!idle_begin) idle_begin = profile.now();)
             // Every look is seven loads of the queue counters; a couple of hundred idle wavefronts
             // looking four times a microsecond would keep the producers' own updates of those
@@ -1495,15 +1560,18 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
         QueueCounter& head = transmit ? q.tx_head : q.rx_head;
         PCIE_EP_PROFILE(profile.first(kProfileFirstClaimNs); const uint64_t claim_begin = profile.now(); if (!profile.values[kProfileFirstLookNs]) profile.values[kProfileFirstLookNs] = look_begin;)
         claims = broadcast_first(claims);
+        owed.prompt = broadcast_first(prompt) != 0;
         int ticket_index = claim_tickets(head, claims, lane);
         const int end = ticket_index + claims;
         // Several wavefronts may have seen the same backlog: a claim beyond the last
         // ticket of the dispatch is simply dropped, an earlier one waits for its tag.
         // Rows whose tickets are ready never wait for a later ticket of the same claim: a
         // source may publish that one only when it has seen these rows acknowledged.
-        bool go_on = true;
         while (go_on && ticket_index < end) {
-            if (wait_ticket(state, q, transmit ? q.tx_ready : q.rx_ready, head, ticket_index, epoch, lane, deadline) < 0) {
+            if (wait_ticket(state, q, transmit ? q.tx_ready : q.rx_ready, head, ticket_index, epoch, lane, deadline, [&] {
+                    wait_memory_ops();
+                    settle(state, q, owed, lane);
+                }) < 0) {
                 if (broadcast_first(aborted(q) ? 1 : 0)) go_on = false;
                 break;
             }
@@ -1511,31 +1579,33 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                             if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows);)
             int count = 1;
             if (transmit) {
-                go_on = tx_row<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, deadline, counters PCIE_EP_PROFILE(, profile, sampled));
+                go_on = tx_row<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, deadline, owed PCIE_EP_PROFILE(, profile, sampled));
             } else {
                 if constexpr (kRows > 1) {
                     const bool ready = lane < kRows && lane < end - ticket_index &&
                                        (lane == 0 || device_load(q.rx_ready + (ticket_index + lane) % kRing) == sequence(epoch, ticket_index + lane));
                     count = __builtin_ctzll(~__ballot(ready));
                 }
-                go_on = rx_rows<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, count, counters, deadline, gate_open, prefixes_known PCIE_EP_PROFILE(, profile, sampled));
+                go_on = rx_rows<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, count, owed, deadline, gate_open, prefixes_known PCIE_EP_PROFILE(, profile, sampled));
             }
             ticket_index += count;
             PCIE_EP_PROFILE(profile.add(transmit ? kProfileTxRows : kProfileRxRows, uint64_t(count)); profile.last(kProfileLastRowNs);)
         }
-        if (!go_on) break;
     }
+    wait_memory_ops();
+    settle(state, q, owed, lane);
     // Workers serve every channel; their counts go to channel 0's row of the
     // per-channel statistics, whose column sums are what callers read.
     if (lane == 0) {
         auto* stats = reinterpret_cast<unsigned long long*>(state.channel_stats);
-        if (counters.writes || counters.credit_miss) {
-            atomicAdd(stats + kStatHostWrites, static_cast<unsigned long long>(counters.writes));
-            atomicAdd(stats + kStatDeliveries, static_cast<unsigned long long>(counters.deliveries));
-            atomicAdd(stats + kStatDescriptors, static_cast<unsigned long long>(counters.published));
-            atomicAdd(stats + kStatTxCreditMiss, static_cast<unsigned long long>(counters.credit_miss));
+        const uint32_t* counts = owed_record + kOwedCounts;
+        if (counts[kCountWrites] || counts[kCountCreditMiss]) {
+            atomicAdd(stats + kStatHostWrites, static_cast<unsigned long long>(counts[kCountWrites]));
+            atomicAdd(stats + kStatDeliveries, static_cast<unsigned long long>(counts[kCountDeliveries]));
+            atomicAdd(stats + kStatDescriptors, static_cast<unsigned long long>(counts[kCountPublished]));
+            atomicAdd(stats + kStatTxCreditMiss, static_cast<unsigned long long>(counts[kCountCreditMiss]));
         }
-        if (counters.reads) atomicAdd(stats + kStatHostReads, static_cast<unsigned long long>(counters.reads));
+        if (counts[kCountReads]) atomicAdd(stats + kStatHostReads, static_cast<unsigned long long>(counts[kCountReads]));
     }
     PCIE_EP_PROFILE(profile.values[kProfileItems] = uint64_t(moves); profile.save(state.profiling, 2 * state.z.dims.channels + order, lane);)
 }
@@ -1562,7 +1632,7 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
     if (block < 0) return;  // a filler id
     int wave = threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
-    uint32_t* scratch = lds.words[wave];
+    uint32_t *scratch = lds.words[wave], *owed_record = lds.owed[wave];
     TransportQueues& q = *state.queues;
     const int payload_waves = state.tx_waves + state.rx_waves;
     const int payload_groups = state.worker_groups > 0 ? state.worker_groups : 0;
@@ -1655,7 +1725,7 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
     // direction's share is spread over the workgroups before it doubles up in one.
     const int groups = payload_groups ? payload_groups : channels;
     const int group = payload_groups ? block - channel_groups : block;
-    if (begun) payload_worker<kFp8, kVector, kRows>(state, q, scratch, lane, wave * groups + group, groups * payload_waves);
+    if (begun) payload_worker<kFp8, kVector, kRows>(state, q, scratch, owed_record, lane, wave * groups + group, groups * payload_waves);
     finish_role(state, q, lane, roles);
     // Every role loop has an explicit completion, abort or timeout exit and no
     // workgroup barrier follows the entry verdict.
