@@ -1074,6 +1074,13 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
 // ---------------------------------------------------------------------------------------
 // RX + scatter worker
 // ---------------------------------------------------------------------------------------
+// Loads of a row (1 KB each) that a wavefront has on the link at once.  About 130 KB in flight fill the link; whatever is
+// requested beyond that only waits, in queues that the writes, the control's polls and the tickets have to
+// pass.  (One wavefront's write of a 14 KB row, beside 188 that read, is acknowledged after 45 us with 14 loads in
+// flight each, 37 with 4, 18 with 2.)  Wavefronts are not always reading, so that fewer than 4 cost more than they save:
+// us per dispatch with all 14, with 4, with 2, with 1: 700 tokens 647 / 645 / 648 / 661, cached replay of 128 185 / 183 /
+// 189 / 193, 2000 tokens hotspot top-4 1645 / 1625 / 1641 / -, 300 tokens on 2 ranks 154 / 150 / 152 / 161.
+constexpr int kReadWindow = 4;
 // Reads the rows of receive tickets first_ticket .. first_ticket + count - 1 (already
 // marked ready, count <= kRows) from their host slots and stores them to their
 // destination rows.  Returns false when the wavefront must stop.
@@ -1202,7 +1209,10 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
         const __amdgpu_buffer_rsrc_t payload = host_resource(slot_base[r], r < count ? uint32_t(z.meta_offset) : 0u);
         // First (usually only) pass of the row.
 #pragma unroll
-        for (int j = 0; j < kRowItems; ++j) row.v[r * kRowItems + j] = host_load_b128(payload, uint32_t(j * kWave + lane) * 16u);
+        for (int j = 0; j < kRowItems; ++j) {
+            if (kRows == 1 && j >= kReadWindow && j * kWave < wire_total) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kReadWindow - 1) : "memory");
+            row.v[r * kRowItems + j] = host_load_b128(payload, uint32_t(j * kWave + lane) * 16u);
+        }
     }
     PCIE_EP_PROFILE(profile.first(kProfileFirstRequestNs);)
     const int meta_dwords = z.meta_bytes / 4;  // a multiple of four; kRows records fit the scratch (receive_batch)
