@@ -103,13 +103,14 @@ __device__ __forceinline__ void sum_chunk_records(const int32_t* first, int stri
 // totals in LDS: host stores issued, not waited for.  A mailbox block starts on a
 // 128-byte line and is stored as whole 16-byte vectors (the words behind its last
 // field are padding of the block): 17 transactions per destination instead of 65.
-__device__ __forceinline__ void store_counts(const DeviceState& state, const ChunkRecord& record, const int* totals) {
+// By `threads` threads, of which this one is number `thread`.
+__device__ __forceinline__ void store_counts(const DeviceState& state, const ChunkRecord& record, const int* totals, int thread, int threads) {
     const SegmentLayout& z = state.z;
     char* own = state.seg[state.local_rank];
     const int ranks = z.dims.num_ranks, local = z.local_experts;
     const int vectors = (z.mailbox_dwords + 3) / 4;
     const __amdgpu_buffer_rsrc_t mailboxes = host_resource(own + z.mailbox_offset, uint32_t(size_t(ranks) * z.mailbox_stride));
-    for (int index = threadIdx.x; index < ranks * vectors; index += blockDim.x) {
+    for (int index = thread; index < ranks * vectors; index += threads) {
         const int destination = index / vectors, vector = index % vectors;
         u32x4 value;
 #pragma unroll
@@ -125,7 +126,7 @@ __device__ __forceinline__ void store_counts(const DeviceState& state, const Chu
     }
     // Relay mode: what each (channel, domain) relay flow of this source will carry.
     const int domains = z.dims.domains, channels = z.dims.channels;
-    for (int index = threadIdx.x; index < domains * channels; index += blockDim.x) {
+    for (int index = thread; index < domains * channels; index += threads) {
         const int domain = index / channels, channel = index % channels;
         host_field_store(relay_mailbox_at(z, own, domain) + channel, totals[record.chan_relay() + channel * domains + domain]);
     }
@@ -576,8 +577,9 @@ __device__ __forceinline__ void prologue_chunk(const DeviceState& state, unsigne
         }
         return __syncthreads_or(outcome) != 0;
     };
+    // The leader's own ordinals are in memory before its totals are needed or the epoch's verdict is there.
+    if (kFused || !leader) write_ordinals();
     if (!leader) {
-        write_ordinals();
         if constexpr (kFused) {
             // This chunk's part of the plan is in memory: count it for the leader
             // (the counter is reset by the epoch begin).
@@ -620,9 +622,41 @@ __device__ __forceinline__ void prologue_chunk(const DeviceState& state, unsigne
     lds_barrier();
     PCIE_EP_PROFILE(profile.first(kPrologueTotalsNs);)
 
+    // The plan's totals, which only this GPU reads: four arrays, each with room up to the next multiple of four words.
+    const auto write_totals = [&]() {
+        if (state.reuse_plan) return;
+        int32_t* const bases[] = {state.plan_counts, state.plan_chan_counts, state.plan_chan_remote, state.plan_chan_relay};
+        const int first[] = {record.counts(), record.chan_counts(), record.chan_remote(), record.chan_relay(), record.error_key()};
+        int before = 0;
+#pragma unroll
+        for (int array = 0; array < 4; ++array) {
+            const int words = first[array + 1] - first[array], vectors = (words + 3) / 4;
+            const __amdgpu_buffer_rsrc_t target = plan_array(bases[array], size_t(words));
+            for (int index = (int(threadIdx.x) - before + int(blockDim.x)) % int(blockDim.x); index < vectors; index += blockDim.x) {
+                int word[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) word[k] = index * 4 + k < words ? totals[first[array] + index * 4 + k] : 0;
+                plan_store4(target, size_t(index) * 4, word[0], word[1], word[2], word[3]);
+            }
+            // The next array starts with the threads behind those that served this one.
+            before = (before + vectors) % int(blockDim.x);
+        }
+    };
+    // Transmit rows of this dispatch: every own token with a remote destination.
+    const auto store_transmit_total = [&]() {
+        int remote_tokens = 0;
+        for (int channel = 0; channel < channels; ++channel) remote_tokens += totals[record.chan_remote() + channel];
+        plan_store(&q.tx_head.total, remote_tokens);
+    };
+
     // ---- epoch verdict -----------------------------------------------------------------
-    if constexpr (kFused) begun = wait_for_word(&q.verdict.value);
-    else if (threadIdx.x == 0) *state.epoch = tag;
+    if constexpr (kFused) {
+        write_totals();
+        wait_memory_ops();  // this wavefront's part of the plan is in memory; the wait below joins the wavefronts
+        begun = wait_for_word(&q.verdict.value);
+    } else if (threadIdx.x == 0) {
+        *state.epoch = tag;
+    }
     // The leader's own findings.  Nothing of the error record is touched unless there
     // is something to record (inside the transport launch it is cleared elsewhere,
     // and `verdict` does not say that this has happened yet).
@@ -647,53 +681,59 @@ __device__ __forceinline__ void prologue_chunk(const DeviceState& state, unsigne
     }
     const uint64_t epoch = tag;
 
-    // The counts leave for the peers first; the plan's totals and the leader's own
-    // ordinals, which only this GPU reads, are written inside the stores' round trip.
-    store_counts(state, record, totals);
-    if (!state.reuse_plan) {
-        // Four arrays, each with room up to the next multiple of four words.
-        int32_t* const bases[] = {state.plan_counts, state.plan_chan_counts, state.plan_chan_remote, state.plan_chan_relay};
-        const int first[] = {record.counts(), record.chan_counts(), record.chan_remote(), record.chan_relay(), record.error_key()};
-        int before = 0;
-#pragma unroll
-        for (int array = 0; array < 4; ++array) {
-            const int words = first[array + 1] - first[array], vectors = (words + 3) / 4;
-            const __amdgpu_buffer_rsrc_t target = plan_array(bases[array], size_t(words));
-            for (int index = (int(threadIdx.x) - before + int(blockDim.x)) % int(blockDim.x); index < vectors; index += blockDim.x) {
-                int word[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) word[k] = index * 4 + k < words ? totals[first[array] + index * 4 + k] : 0;
-                plan_store4(target, size_t(index) * 4, word[0], word[1], word[2], word[3]);
-            }
-            // The next array starts with the threads behind those that served this one.
-            before = (before + vectors) % int(blockDim.x);
-        }
-    }
-    // Transmit tickets of this dispatch: every own token with a remote destination.
-    if (threadIdx.x == 0) {
-        int remote_tokens = 0;
-        for (int channel = 0; channel < channels; ++channel) remote_tokens += totals[record.chan_remote() + channel];
-        plan_store(&q.tx_head.total, remote_tokens);
-    }
-    write_ordinals();
-    PCIE_EP_PROFILE(profile.first(kPrologueLayoutNs);)
-    publish_counts(state, epoch PCIE_EP_PROFILE(, profile));
     if constexpr (kFused) {
-        // The counts are with the peers; now the own rows may follow.  Every chunk's
-        // part of the plan must be in memory before the transmit side reads it.
-        if (threadIdx.x == 0 && !state.reuse_plan) {
-            while (int(device_load(&q.plan_chunks.value)) < chunks - 1) {
-                if (now_ticks() - begin_ticks > state.timeout_ticks) {
-                    record_error(state, kErrRingProgressWait);
-                    device_store(&q.abort.value, 1u);
-                    break;
-                }
-                backoff();
+        // The upper half of the wavefronts sends the counts to the peers; the lower half does not wait for the host's
+        // acknowledgements, which take 5 us on an idle link and 10 once rows are requested: its part of the plan is in memory.
+        __shared__ int counts_stored;
+        const int lower = chunk_waves / 2, upper = chunk_waves - lower;
+        if (threadIdx.x == 0) counts_stored = 0;
+        lds_barrier();
+        if (wave >= lower) {
+            store_counts(state, record, totals, int(threadIdx.x) - lower * kWave, upper * kWave);
+            wait_memory_ops();
+            if (lane == 0 && __hip_atomic_fetch_add(&counts_stored, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == upper - 1) {
+                // Every wavefront has waited for its own stores; this is the last of them.
+                PCIE_EP_PROFILE(if (state.profiling) state.profiling[size_t(profile_row) * kProfileFields + kPrologueMailboxAckedNs] = int64_t(profile.now());)
+                host_store_release(signal_at(state.seg[state.local_rank], z.counts_ready_offset), epoch);
+                PCIE_EP_PROFILE(if (state.profiling) state.profiling[size_t(profile_row) * kProfileFields + kPrologueCountsReadyNs] = int64_t(profile.now());)
             }
+            return;
         }
-        __syncthreads();
-        if (threadIdx.x == 0) device_store(&q.plan_ready.value, epoch_flag(tag));
-        PCIE_EP_PROFILE(profile.first(kProloguePlanReadyNs);)
+        PCIE_EP_PROFILE(profile.first(kPrologueLayoutNs);)
+        // Every chunk's part of the plan must be in memory before the transmit side reads it, and the queues must have
+        // been reset (the verdict does not say so) before the total is stored.
+        if (threadIdx.x == 0) {
+            const auto reached = [&](auto there) {
+                while (!there()) {
+                    if (now_ticks() - begin_ticks > state.timeout_ticks) return false;
+                    backoff();
+                }
+                return true;
+            };
+            if (!reached([&] { return device_load(&q.begun.value) == epoch_flag(tag); }) ||
+                (!state.reuse_plan && !reached([&] { return int(device_load(&q.plan_chunks.value)) >= chunks - 1; }))) {
+                record_error(state, kErrRingProgressWait);
+                device_store(&q.abort.value, 1u);
+            }
+            store_transmit_total();
+            wait_memory_ops();
+            device_store(&q.plan_ready.value, epoch_flag(tag));
+        }
+        PCIE_EP_PROFILE(profile.first(kProloguePlanReadyNs); profile.values[kProfileExitNs] = profile.now();
+                        if (threadIdx.x == 0 && state.profiling)
+                            for (int field = 0; field < kProfileFields; ++field)
+                                if (field != kPrologueMailboxAckedNs && field != kPrologueCountsReadyNs)
+                                    state.profiling[size_t(profile_row) * kProfileFields + field] = int64_t(profile.values[field]);
+                        return;)
+    } else {
+        // The counts leave for the peers first; the plan's totals and the leader's own
+        // ordinals, which only this GPU reads, are written inside the stores' round trip.
+        store_counts(state, record, totals, int(threadIdx.x), int(blockDim.x));
+        write_totals();
+        if (threadIdx.x == 0) store_transmit_total();
+        write_ordinals();
+        PCIE_EP_PROFILE(profile.first(kPrologueLayoutNs);)
+        publish_counts(state, epoch PCIE_EP_PROFILE(, profile));
     }
     PCIE_EP_PROFILE(profile.save(state.profiling, profile_row, threadIdx.x);)
 }
