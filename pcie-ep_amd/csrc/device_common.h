@@ -66,8 +66,9 @@ static_assert(sizeof(RxEntry) == 32 && sizeof(TxEntry) == 112, "queue entry layo
 
 struct alignas(128) QueueCounter {
     uint32_t value;
-    int32_t total;  // -1 until the number of tickets is known
-    char pad[120];
+    int32_t total;   // -1 until the number of rows is known
+    int32_t direct;  // rows that are moved without a ticket
+    char pad[116];
 };
 
 struct alignas(256) TransportQueues {
@@ -78,7 +79,7 @@ struct alignas(256) TransportQueues {
     QueueCounter finished;          // role wavefronts that have ended; the last one reduces the statistics
     // Prologue inside the transport launch: value = epoch_flag(epoch) once the epoch begin has cleared the
     // diagnostics and reset the queues (begun) / has found no abort word set and the previous count mailbox
-    // consumed (verdict) / the leader has published the counts and the whole plan is in memory (plan_ready);
+    // consumed (verdict) / the whole plan is in memory (plan_ready);
     // plan_chunks counts the chunks other than the leader's whose part of the plan is in memory.
     QueueCounter begun, verdict, plan_ready, plan_chunks;
     QueueCounter rx_retired[kMaxChannels], tx_retired[kMaxChannels], rx_finished[kMaxChannels];
@@ -87,6 +88,8 @@ struct alignas(256) TransportQueues {
     RxEntry rx[kRing];
     TxEntry tx[kRing];
 };
+
+constexpr int kDrainedEpochWord = 16;  // a line of its own in the 256 bytes of the epoch word
 
 // Launch argument of every kernel: this rank's device pointers, the device
 // aliases of the pinned host segments and the plan/output pool of one dispatch
@@ -108,7 +111,7 @@ struct DeviceState {
     int prologue_chunks;     // token chunks of this dispatch's layout (0 when a cached plan is reused)
     uint64_t timeout_ticks;
     uint64_t clock_khz;  // rate of wall_clock64() on this device (hipDeviceAttributeWallClockRate)
-    uint64_t* epoch;
+    uint64_t* epoch;          // [0]: epoch of the last dispatch; [kDrainedEpochWord]: of the last one that ended with every own slot acknowledged
 
     const uint16_t* x;
     const int64_t* topk_idx;

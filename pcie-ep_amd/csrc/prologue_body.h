@@ -35,7 +35,7 @@
 //    crosses workgroups inside the one launch goes through device-scope flags:
 //    `begun` (diagnostics cleared, queues reset), `verdict` (no abort word set,
 //    previous mailbox consumed), `plan_chunks` / `plan_ready` (route plan written
-//    through to memory, transmit total known, counts published) and the abort
+//    through to memory, transmit total known) and the abort
 //    word (the prologue failed).  The epoch word is then advanced by the last
 //    role of the launch to end, so that every workgroup of the launch reads the
 //    same value at its start.
@@ -178,6 +178,7 @@ __device__ __forceinline__ void clear_epoch_state(const DeviceState& state, int 
     if (index < 8) {
         clear(&globals[index]->value, 0u);
         clear(&globals[index]->total, -1);
+        clear(&globals[index]->direct, 0);
     }
     for (int i = index; i < channels; i += count) {
         QueueCounter* counters[] = {&q.rx_retired[i], &q.tx_retired[i], &q.rx_finished[i]};

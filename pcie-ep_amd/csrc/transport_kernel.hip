@@ -9,9 +9,9 @@
 // layout, advanced_transport (advanced_dispatch.cuh:919-958).
 //
 // Design for MI355X (64-lane wavefronts, 8 XCDs):
-//  * A payload worker is ONE wavefront that owns a whole row: 14 x 16-byte
-//    loads per lane are issued back to back (896 vectors of a 14 336-byte BF16
-//    row), the row lives in registers, and the same wavefront stores it to
+//  * A payload worker is ONE wavefront that owns a whole row: its up to
+//    14 x 16-byte loads per lane (896 vectors of a 14 336-byte BF16 row) leave
+//    kReadWindow at a time, the row lives in registers, and the same wavefront stores it to
 //    every destination expert row.  The staged row is read once; there is no
 //    LDS tile and no producer/consumer hand-off (the reference stages through
 //    shared memory with 3+3 warps per ticket).
@@ -41,8 +41,10 @@
 //    here start with the queues not yet reset: one thread per workgroup waits for
 //    the epoch begin's word before its role touches them, the transmit side and
 //    the local bypass wait for the plan's word, the receive side for neither.
-//  * Workers publish their own descriptors and payload ACKs as soon as their own
-//    stores / loads have completed; control wavefronts only reserve and hand out.
+//  * Workers publish their own descriptors and payload ACKs when their own stores /
+//    loads have completed (see settle); control wavefronts only reserve and hand out.
+//  * The first tokens of every channel are copied to their slots without ticket or
+//    plan, before the first received rows are requested (see direct_row).
 //  * A payload wavefront has no fixed direction: before every row it takes the
 //    direction that needs it, in proportion to the rows left to send and to
 //    receive, so that the writes are spread thinly over the whole dispatch (row
@@ -73,12 +75,16 @@ namespace {
 constexpr int kScratchDwords = kReceiveScratchDwords;  // per wavefront: slot metadata records (of one or kMaxReceiveBatch rows)
 constexpr int kMaxWaves = 12;
 // What a payload wavefront owes the other ends (see Owed): slot ACKs (address, token), then a transmitted row's
-// channel, slot, token and descriptor ordinal per endpoint; behind them the wavefront's counters.
-constexpr int kOwedRow = 4 * kMaxReceiveBatch, kOwedDescriptors = kOwedRow + 4, kOwedCounts = kOwedDescriptors + kMaxEndpoints, kOwedDwords = kOwedCounts + 8;
+// channel, slot, token and descriptor ordinal per endpoint; behind them the words of a direct row's ticket and the
+// wavefront's counters.
+constexpr int kTicketWords = int(sizeof(TxEntry) / 4);
+constexpr int kOwedRow = 4 * kMaxReceiveBatch, kOwedDescriptors = kOwedRow + 4, kDirectTicket = kOwedDescriptors + kMaxEndpoints;
+constexpr int kOwedCounts = kDirectTicket + kTicketWords, kOwedDwords = kOwedCounts + 8;
 
 struct WaveScratch {
     uint32_t words[kMaxWaves][kScratchDwords];
     uint32_t owed[kMaxWaves][kOwedDwords];
+    int begun;
 };
 
 // Local time only: payload workers never scan the host abort flags themselves
@@ -159,8 +165,8 @@ __device__ __forceinline__ int wait_ticket(const DeviceState& state, TransportQu
             if (aborted(q)) action = -1;
             else if (device_load(ready + ticket % kRing) == sequence(epoch, ticket)) action = 1;
             else {
-                const int limit = device_load(&head.total);
-                if (limit >= 0 && ticket >= limit) action = -1;
+                const int limit = device_load(&head.total), direct = device_load(&head.direct);
+                if (limit >= 0 && ticket >= limit - direct) action = -1;
                 else if (deadline.expired(state)) {
                     record_error(state, kErrRingProgressWait);
                     raise_abort(q);
@@ -431,6 +437,73 @@ __device__ __forceinline__ int receive_prefix_verdict(const DeviceState& state, 
 // ---------------------------------------------------------------------------------------
 // TX control + guardian
 // ---------------------------------------------------------------------------------------
+// Destination ranks of a token, straight from its routes: what the plan will say (ids that are out of range count for
+// none, a repeated one for the same rank; either ends the dispatch).  Only where the prologue rides in this launch, with
+// at most eight routes per token.
+__device__ __forceinline__ uint32_t route_destinations(const DeviceState& state, int token) {
+    constexpr int kFusedTopk = 8;
+    const int topk = state.z.dims.topk, experts = state.z.dims.num_experts, local = state.z.local_experts;
+    int64_t raw[kFusedTopk];
+#pragma unroll
+    for (int branch = 0; branch < kFusedTopk; ++branch) raw[branch] = branch < topk ? state.topk_idx[size_t(token) * topk + branch] : -1;
+    uint32_t destinations = 0;
+#pragma unroll
+    for (int branch = 0; branch < kFusedTopk; ++branch)
+        if (raw[branch] >= 0 && raw[branch] < experts) destinations |= 1u << (uint32_t(raw[branch]) / uint32_t(local));
+    return destinations;
+}
+
+// Entry `ordinal` of the queue that this rank reads `source`'s descriptors from: of another domain's source, the one its
+// relay fills for this rank's domain (advanced_common.cuh:237-247).
+__device__ __forceinline__ Descriptor* descriptor_of(const DeviceState& state, int channel, int source, int ordinal) {
+    const SegmentLayout& z = state.z;
+    const int me = state.local_rank;
+    return reads_replica(z.dims, source, me) ? replica_descriptor_at(z, state.seg[source], channel, z.dims.rank_domain[me], me, ordinal)
+                                             : descriptor_at(z, state.seg[source], channel, me, ordinal);
+}
+
+// ---------------------------------------------------------------------------------------
+// Direct rows
+// ---------------------------------------------------------------------------------------
+// The host link is idle until the first received rows are requested, some 10 us into the launch, and once they are, a
+// row to be transmitted waits behind them twice: its reads from HBM pass the same queues of its XCD (10 to 20 us where
+// an idle machine takes 1.4), and its stores share the link.  The first tokens of every channel are therefore
+// transmitted by payload wavefronts that need neither ticket nor plan for it: token t by wavefront t, as it
+// enters.  Its place in the rings follows from the routes of the tokens in front of it in its channel.  The
+// metadata and the descriptors follow when the plan is there.
+//
+// As many as the link takes in that time (kDirectBytes), at most kMaxDirectRows of a channel: 64 rows of 14 KB hold the
+// first received rows up (cached replay of 128 tokens 186 us per dispatch with 32 of them, 192 with 64), 64 of 8 KB do
+// not (4 ranks, 200 tokens of 4096 columns 119 / 110).  And only in a dispatch that receives little (kDirectDispatchBytes,
+// by the rows of all other sources): a longer one ends with its receive side whatever the transmit side does, and
+// the early rows only delay it (96 aligned tokens, 9.7 MB: 145 us without, 148 with them).
+// Us per dispatch without and with: 16 tokens 52 / 48, 32 75 / 68, 64 of 4096 columns 80 / 73, 24 of 2048 (top-4) 40 / 35,
+// 2 ranks with 300 tokens 157 / 138.
+constexpr int64_t kDirectBytes = 544 << 10;
+constexpr int64_t kDirectDispatchBytes = 6 << 20;
+constexpr int kMaxDirectRows = 3;
+struct DirectRow {
+    bool valid = false;
+    float scale = 1.0f;
+};
+__device__ __forceinline__ int payload_wavefronts(const DeviceState& state) { return state.worker_groups * (state.tx_waves + state.rx_waves); }
+// How many tokens of every channel are direct rows: with the prologue in the launch, payload wavefronts of their own for
+// them, and rings that the dispatch before has left drained.
+__device__ __forceinline__ int direct_rows_per_channel(const DeviceState& state) {
+    const SegmentLayout& z = state.z;
+    const int64_t row_bytes = z.meta_offset + z.meta_bytes;
+    if (!state.fused || int64_t(z.dims.num_ranks - 1) * state.num_tokens * row_bytes > kDirectDispatchBytes || device_load(state.epoch + kDrainedEpochWord) + 1 != dispatch_epoch(state)) return 0;
+    int rows = payload_wavefronts(state) / (2 * z.dims.channels);
+    const int most = int(kDirectBytes / (z.dims.channels * row_bytes));
+    rows = rows < most ? rows : most;
+    rows = rows < kMaxDirectRows ? rows : kMaxDirectRows;
+    rows = rows < z.dims.payload_slots ? rows : z.dims.payload_slots;
+    return rows < z.dims.descriptor_slots ? rows : z.dims.descriptor_slots;
+}
+// Destination ranks of a token without the plan of this dispatch.
+__device__ __forceinline__ uint32_t early_destinations(const DeviceState& state, int token) {
+    return state.fused && !state.reuse_plan ? route_destinations(state, token) : state.plan_mask[token];
+}
 __device__ __forceinline__ void tx_control(const DeviceState& state, TransportQueues& q, int channel, int lane) {
     const SegmentLayout& z = state.z;
     const int channels = z.dims.channels, me = state.local_rank;
@@ -451,7 +524,8 @@ __device__ __forceinline__ void tx_control(const DeviceState& state, TransportQu
     int reserved[kMaxEndpoints];
 #pragma unroll
     for (int endpoint = 0; endpoint < kMaxEndpoints; ++endpoint) reserved[endpoint] = 0;
-    bool failed = !wait_for_plan(state, q, lane);
+    const int direct = broadcast_first(direct_rows_per_channel(state));
+    bool failed = false;
     int64_t stage_busy = 0, prepared_ahead = 0;
 
     for (int base = 0; base < candidates && !failed; base += kWave) {
@@ -459,7 +533,9 @@ __device__ __forceinline__ void tx_control(const DeviceState& state, TransportQu
         const int token = channel + candidate * channels;
         // Where the token is published: its destination ranks, with those of other
         // domains folded into one relay endpoint per domain (advanced_common.cuh:207-225).
-        const uint32_t remote = candidate < candidates ? endpoint_mask_of(z.dims, me, state.plan_mask[token]) : 0u;
+        uint32_t destinations = 0;
+        if (candidate < candidates) destinations = early_destinations(state, token);
+        const uint32_t remote = endpoint_mask_of(z.dims, me, destinations);
         const uint64_t batch = __ballot(remote != 0);
         if (!batch) continue;
         const int ordinal = produced + __popcll(batch & below);
@@ -475,12 +551,16 @@ __device__ __forceinline__ void tx_control(const DeviceState& state, TransportQu
         }
         // Ring history: which token occupied ordinal i (needed when a slot is reused).
         if (remote) device_store(state.chan_remote_tokens + size_t(channel) * stride + ordinal, token);
-        const int ticket_index = reserve_tickets(q.tx_tail, __popcll(batch), lane) + __popcll(batch & below);
+        // The channel's first tokens may be direct rows, which have no ticket.
+        const uint64_t ticketed = __ballot(remote != 0 && candidate >= direct);
+        int ticket_index = 0;
+        if (ticketed) ticket_index = reserve_tickets(q.tx_tail, __popcll(ticketed), lane) + __popcll(ticketed & below);
+        else wait_memory_ops();
         // Tickets prepared while an earlier payload of this channel is still in
         // flight: the control path runs ahead of the payload path (the event the
         // reference counts in stats[3]: advanced_dispatch.cuh:384-387).
         if (produced > 0 && broadcast_first(int(device_load(&q.tx_retired[channel].value))) < produced) prepared_ahead += __popcll(batch);
-        bool pending = remote != 0;
+        bool pending = (ticketed >> lane) & 1ull;
         while (true) {
             if (pending && ring_entry_free(q.tx_taken, epoch, ticket_index)) {
                 const uint32_t at = uint32_t(ticket_index % kRing) * uint32_t(sizeof(TxEntry));
@@ -650,10 +730,7 @@ struct RxLane {
     }
     // Entry `ordinal` of the lane's queue (entry 0 of the own queue for a lane without one: never loaded).
     __device__ __forceinline__ Descriptor* entry(const DeviceState& state, int channel, int ordinal) const {
-        const SegmentLayout& z = state.z;
-        const int me = state.local_rank;
-        char* segment = state.seg[member ? source : me];
-        return replica ? replica_descriptor_at(z, segment, channel, my_domain, me, ordinal) : descriptor_at(z, segment, channel, me, ordinal);
+        return descriptor_of(state, channel, member ? source : state.local_rank, ordinal);
     }
 };
 __device__ __forceinline__ RxFirstPoll rx_first_poll(const DeviceState& state, int channel, int lane) {
@@ -896,8 +973,11 @@ __device__ __forceinline__ void finish_role(const DeviceState& state, TransportQ
     }
     if (lane == 0) state.transport_timestamps_ns[0] = span == INT64_MAX ? 0 : span;
     if (lane == 1) state.transport_timestamps_ns[1] = span;
+    const uint64_t epoch = dispatch_epoch(state);
+    // Every own slot has been acknowledged unless the dispatch failed: the next one may write them at once.
+    if (lane == 0 && !aborted(q) && load_error_code(state) == 0) state.epoch[kDrainedEpochWord] = epoch;
     // Prologue inside this launch: every workgroup has read the epoch word by now.
-    if (lane == 0 && state.fused) *state.epoch = dispatch_epoch(state);
+    if (lane == 0 && state.fused) *state.epoch = epoch;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -912,6 +992,34 @@ __device__ __forceinline__ float tx_copy_row(const DeviceState& state, const uin
     if constexpr (kFp8) return quantize_row_to_host<kVector, kGroups>(input, slot, hidden, lane, before_stores);
     copy_row_to_host<kVector>(input, slot, hidden, lane, before_stores);
     return 1.0f;
+}
+
+// Payload wavefront `order` transmits the payload of its direct row, if it has one, and leaves the words of its ticket in `ticket`.
+template <bool kFp8, bool kVector, int kRows>
+__device__ __forceinline__ DirectRow direct_row(const DeviceState& state, uint32_t* ticket, int order, int lane) {
+    const SegmentLayout& z = state.z;
+    const int channels = z.dims.channels, me = state.local_rank, token = order;
+    DirectRow row;
+    if (!state.fused || token >= state.num_tokens || token >= channels * kMaxDirectRows || token >= channels * broadcast_first(direct_rows_per_channel(state))) return row;
+    // Lane c: the channel's candidate c.
+    const int channel = token % channels, candidate = token / channels;
+    uint32_t remote = 0;
+    if (lane <= candidate) remote = endpoint_mask_of(z.dims, me, early_destinations(state, channel + lane * channels));
+    const uint32_t endpoints = uint32_t(__shfl(int(remote), candidate));
+    if (endpoints == 0) return row;
+    const uint64_t in_front = lanes_below(candidate);
+    const int ordinal = __popcll(__ballot(remote != 0) & in_front);
+    // Lane 4 + e: descriptor ordinal of endpoint e (TxEntry).
+    uint32_t word = lane == 0 ? uint32_t(token) : lane == 1 ? uint32_t(ordinal) : lane == 2 ? endpoints : uint32_t(channel);
+    for (int endpoint = 0; endpoint < z.endpoints; ++endpoint) {
+        const int before = __popcll(__ballot((remote >> endpoint) & 1u) & in_front);
+        if (lane == 4 + endpoint) word = uint32_t(before);
+    }
+    if (lane < kTicketWords) ticket[lane] = word;
+    row.scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden,
+                                                  host_resource(slot_at(z, state.seg[me], channel, ordinal), uint32_t(z.meta_offset)), lane, [] {});
+    row.valid = true;
+    return row;
 }
 
 // What a payload wavefront still owes the other ends of the rows it has moved: a received row's slot ACK (lane r: row
@@ -963,11 +1071,11 @@ __device__ __forceinline__ void count_rows(uint32_t* record, WorkerCount which, 
     if (lane == 0) record[kOwedCounts + which] += uint32_t(amount);
 }
 
-// Moves the own token of transmit ticket `ticket_index` (already marked ready)
-// into its host slot; what publishes it is left to settle().  Returns false when the wavefront must stop.
-template <bool kFp8, bool kVector, int kRows>
-__device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int ticket_index, const Deadline& deadline,
-                       Owed& owed PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
+// Moves the own token of transmit ticket `ticket_index` (already marked ready), or of the direct row whose payload is on
+// its way, into its host slot; what publishes it is left to settle().  Returns false when the wavefront must stop.
+template <bool kFp8, bool kVector, int kRows, bool kDirect>
+__device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int ticket_index, float direct_scale,
+                       const Deadline& deadline, Owed& owed, bool& plan_known PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
     const SegmentLayout& z = state.z;
     const int ranks = z.dims.num_ranks, topk = z.dims.topk, me = state.local_rank;
     const int endpoint_count = z.endpoints;
@@ -980,13 +1088,21 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
     {
         // Copy the ticket out of the ring (one dword per lane), then free its entry.
         const uint32_t entry_base = uint32_t(ticket_index % kRing) * uint32_t(sizeof(TxEntry));
-        const uint32_t word = device_load_b32(ring, entry_base + uint32_t(lane < int(sizeof(TxEntry) / 4) ? lane : 0) * 4u);
+        uint32_t word;
+        if constexpr (kDirect) {
+            word = owed.record[kDirectTicket + (lane < kTicketWords ? lane : 0)];
+            if (lane == 0) device_add(reinterpret_cast<uint32_t*>(&q.tx_head.direct), 1u);
+        } else {
+            word = device_load_b32(ring, entry_base + uint32_t(lane < kTicketWords ? lane : 0) * 4u);
+        }
         const int token = __shfl(int(word), 0), ordinal = __shfl(int(word), 1);
         const uint32_t endpoints = uint32_t(__shfl(int(word), 2));
         const int channel = __shfl(int(word), 3);
         const int my_descriptor = __shfl(int(word), 4 + (lane < endpoint_count ? lane : 0));
-        wait_memory_ops();
-        if (lane == 0) device_store(q.tx_taken + ticket_index % kRing, sequence(epoch, ticket_index));
+        if constexpr (!kDirect) {
+            wait_memory_ops();
+            if (lane == 0) device_store(q.tx_taken + ticket_index % kRing, sequence(epoch, ticket_index));
+        }
         const int slot = ordinal % slots;
         const bool targeted = lane < endpoint_count && ((endpoints >> lane) & 1u);
         if (ordinal == 0 && lane == 0) state.prefix_tx_timestamps_ns[(channel + 1) * 2] = ticks_to_ns(state, now_ticks());
@@ -996,6 +1112,12 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         // (advanced_dispatch.cuh:158-187).  One lane per endpoint.
         bool slot_ok = true, credit_ok = true;
         uint64_t previous_sequence = 0;
+        if (!plan_known) {
+            // A direct row's payload is on its way; everything else of it, and all of any other row, follows the plan.
+            settle(state, q, owed, lane);
+            if (!wait_for_plan(state, q, lane)) return false;
+            plan_known = true;
+        }
         if (ordinal >= slots) {
             const int previous_token = device_load(state.chan_remote_tokens + size_t(channel) * stride + ordinal - slots);
             const uint32_t previous_remote = endpoint_mask_of(z.dims, me, state.plan_mask[previous_token]);
@@ -1039,8 +1161,10 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         }
         if (lane == kWave - 1) test_delay(state.tx_delay);
         const __amdgpu_buffer_rsrc_t slot_resource = host_resource(slot_base, uint32_t(z.meta_offset + z.meta_bytes));
-        const float scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden, host_resource(slot_base, uint32_t(z.meta_offset)), lane,
-                                                       [&] { settle(state, q, owed, lane); });
+        float scale = direct_scale;
+        if constexpr (!kDirect)
+            scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden, host_resource(slot_base, uint32_t(z.meta_offset)), lane,
+                                                      [&] { settle(state, q, owed, lane); });
         if (lane == 0) scratch[2] = float_bits(scale);
         fence_lds();
         if (lane == meta_dwords - 1 || (lane == kWave - 1 && meta_dwords > kWave)) test_delay(state.metadata_delay);
@@ -1487,18 +1611,21 @@ template <int kRows>
 constexpr Share kTxShare = kRows > 1 ? Share{1, 2} : Share{2, 3};
 
 template <bool kFp8, bool kVector, int kRows>
-__device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, uint32_t* owed_record, int lane, int order, int waves) {
+__device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, uint32_t* owed_record, int lane, int order, int waves, DirectRow start) {
     const uint64_t epoch = dispatch_epoch(state);
     Deadline deadline(now_ticks());
     if (lane < kWorkerCounts) owed_record[kOwedCounts + lane] = 0;
     Owed owed{owed_record};
     PCIE_EP_PROFILE(RoleProfile profile(state.clock_khz); uint64_t idle_begin = 0; int moves = 0;)
-    bool prefixes_known = false, gate_open = false;
+    bool prefixes_known = false, gate_open = false, plan_known = state.fused == 0;
     const int lead = int(kTxLeadBytes / int64_t(state.z.meta_offset + state.z.meta_bytes));
     // A wavefront that may be wanted for transmitting binds itself to one batch at a time.
     const int most_claims = 2 * order < waves || kRows == 1 ? kRows : kReceiveClaims;
     uint64_t idle_since = 0;  // 0: the last look found work
+    fence_lds();
     bool go_on = true;
+    // (Its ticket's words are in the record.)
+    if (start.valid) go_on = tx_row<kFp8, kVector, kRows, true>(state, q, scratch, lane, 0, start.scale, deadline, owed, plan_known PCIE_EP_PROFILE(, profile, false));
     while (go_on) {
         // 0: nothing to do now, 1: transmit, 2: receive, -1: both directions are finished or the kernel aborts.
         int choice = 0, claims = 1, prompt = 1;
@@ -1520,7 +1647,10 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                     gate_seen = (device_load(state.receive_prefix_state) & kPrefixRequested) != 0;
                     rx_backlog = gate_seen != 0;
                 }
-                const int tx_total = device_load(&q.tx_head.total), rx_total = device_load(&q.rx_head.total);
+                // Tickets of the dispatch: its rows but for the direct ones.
+                int tx_total = device_load(&q.tx_head.total);
+                const int rx_total = device_load(&q.rx_head.total), tx_direct = device_load(&q.tx_head.direct);
+                if (tx_total >= 0) tx_total -= tx_direct;
                 const bool tx_done = tx_total >= 0 && tx_head >= tx_total, rx_done = rx_total >= 0 && rx_head >= rx_total;
                 // Totals unknown: a handful of wavefronts start to transmit, the others
                 // wait for the first descriptors.
@@ -1601,7 +1731,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                             if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows);)
             int count = 1;
             if (transmit) {
-                go_on = tx_row<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, deadline, owed PCIE_EP_PROFILE(, profile, sampled));
+                go_on = tx_row<kFp8, kVector, kRows, false>(state, q, scratch, lane, ticket_index, 1.0f, deadline, owed, plan_known PCIE_EP_PROFILE(, profile, sampled));
             } else {
                 if constexpr (kRows > 1) {
                     const bool ready = lane < kRows && lane < end - ticket_index &&
@@ -1697,10 +1827,18 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
     if (!payload_groups && block < channel_groups && wave == 1) receive_channel = block;
     RxFirstPoll first_poll{{0u, 0u, 0u, 0u}, false};
     if (receive_channel >= 0) first_poll = rx_first_poll(state, receive_channel, lane);
+    // Position of a payload wavefront among all of them, wavefront-major: a
+    // direction's share is spread over the workgroups before it doubles up in one.
+    DirectRow direct;
+    if (payload_groups && block >= channel_groups && block < channel_groups + payload_groups && wave < payload_waves)
+        direct = direct_row<kFp8, kVector, kRows>(state, owed_record + kDirectTicket, wave * payload_groups + block - channel_groups, lane);
     PrefixFirstLook first_look{0, false};
     if (prefix_producer) first_look = prefix_first_look(state, lane);
     if (state.fused) {
-        begun = __syncthreads_or(threadIdx.x == 0 ? int(wait_for_begin(state, q)) : 0) != 0;
+        // (LDS only: the reads and stores issued above stay in flight.)
+        if (threadIdx.x == blockDim.x - kWave) lds.begun = int(wait_for_begin(state, q));
+        lds_barrier();
+        begun = lds.begun != 0;
     } else if (__syncthreads_or(threadIdx.x == 0 ? int(load_error_code(state) != 0) : 0)) {
         return;  // the prologue kernel in front of this one failed
     }
@@ -1743,11 +1881,9 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
         wave -= 2;
     }
     if (wave >= payload_waves) return;
-    // Position of this wavefront among all payload wavefronts, wavefront-major: a
-    // direction's share is spread over the workgroups before it doubles up in one.
     const int groups = payload_groups ? payload_groups : channels;
     const int group = payload_groups ? block - channel_groups : block;
-    if (begun) payload_worker<kFp8, kVector, kRows>(state, q, scratch, owed_record, lane, wave * groups + group, groups * payload_waves);
+    if (begun) payload_worker<kFp8, kVector, kRows>(state, q, scratch, owed_record, lane, wave * groups + group, groups * payload_waves, direct);
     finish_role(state, q, lane, roles);
     // Every role loop has an explicit completion, abort or timeout exit and no
     // workgroup barrier follows the entry verdict.

@@ -248,6 +248,20 @@ def test_short_rows_are_received_in_pairs(hidden, topk, fp8):
             check_case(buffer, f"pairs-h{hidden}-k{topk}-s{slots}-unique", tokens, expand=False, seed=9, fp8=fp8)
 
 
+@pytest.mark.parametrize("world,hidden,slots,descriptors,fp8", [(8, 1024, 64, 64, False), (2, 4096, 1, 1, False), (4, 1001, 2, 3, False), (8, 1000, 64, 2, True),
+                                                                (8, 7168, 3, 64, True)])
+def test_first_rows_of_a_channel_go_ahead_of_the_plan(world, hidden, slots, descriptors, fp8):
+    """Up to three tokens of every channel are transmitted without a ticket, where the dispatch before has drained the
+    rings: as many as channels, one less and one more, two and three times as many and beyond; tokens among them that
+    go nowhere or stay on this rank; rings that hold fewer; a dispatch too large for it (6 MB of rows to come) between."""
+    wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
+    with make_buffer(world=world, tmax=900, hidden=hidden, channels=4, payload_slots=slots, descriptor_slots=descriptors, **wire) as buffer:
+        for repeat, own in enumerate((3, 4, 5, 8, 13, 40, 900, 1, 0, 12)):
+            tokens = [own] + [max(0, own - 3 * r) for r in range(1, world)]
+            for pattern in ("random", "partial", "local", "multicast")[: 1 if own > 40 else 4]:
+                check_case(buffer, f"first-rows-w{world}-h{hidden}", tokens, pattern, expand=repeat % 2 == 0, seed=60 + repeat, fp8=fp8)
+
+
 def test_profiling_records_count_every_row_of_a_pair():
     """The per-role records (profiling build, a process of its own): rows received and transmitted equal the
     dispatch's statistics, and fewer moves than rows: pairs are taken."""
