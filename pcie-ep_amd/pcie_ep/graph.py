@@ -36,8 +36,8 @@ class GraphDispatch:
         self._open = True
         # The capture holds one kernel, or with the stand-alone expand two, and nothing else: a replay launches them with
         # the captured arguments as an eager dispatch would.  Between two launches of the instantiated graph the GPU idles
-        # for 13.2 us, between two of the kernel for 5.6 (cached replay of 128 tokens 183 us / 175, 64 tokens on the FP8
-        # wire 79 / 70).  Where the scratch is the static one the graph is launched: ordering its replays
+        # for 13.2 us, between two of the kernel for 5.6 (cached replay of 128 tokens 187 us / 181, 64 tokens on the FP8
+        # wire 77 / 74).  Where the scratch is the static one the graph is launched: ordering its replays
         # against other runtimes' is the caller's, and a fresh launch would refuse one that is in flight.
         self._launch = _native.library().pcie_ep_dispatch
         self._arguments = arguments
