@@ -1577,8 +1577,8 @@ __device__ __forceinline__ bool rx_rows(const DeviceState& state, TransportQueue
 // when its receivers have acknowledged it, and that round trip then hides
 // behind the last received rows instead of following them.  The rule corrects
 // itself: a direction that falls behind has more left and gets more wavefronts;
-// at most kTxShare of the wavefronts transmit and, while anything is left to send, at
-// least kMinTxWaves.  Until both totals are known (the receive total comes with
+// at most transmit_wavefronts() of them transmit and, while anything is left to send, at
+// least kMinTxWaves of those.  Until both totals are known (the receive total comes with
 // the receive prefixes) those kMinTxWaves transmit and everybody else waits for
 // the first descriptors.  A wavefront whose direction has nothing to
 // claim takes a ticket of the other direction instead - at once when its own
@@ -1597,19 +1597,6 @@ constexpr int64_t kTxLeadBytes = 24 << 20;
 constexpr int kMinTxWaves = 16;
 constexpr uint64_t kIdleCrossoverUs = 30;
 constexpr int kPreGateRows = 32;
-// The share of the payload wavefronts that may transmit while rows are left to receive.  Requests of both directions wait
-// in the same queues on their way to the link: a rank that sends as much as it receives used the link's two halves one
-// after the other with one transmitting wavefront per receiving one, because a transmitting wavefront spends
-// more of its time off the link (claim, plan, the row's reads from HBM).  64 MB each way by a bare kernel: 2.1 ms with
-// two reading wavefronts per writing one, 1.4 with one, 1.12 for either direction alone.  Us per dispatch with a half
-// and with two thirds: 2 ranks, 1000 tokens of 4096 columns 277 / 246, 300 of 7168 167 / 161; 8 ranks unchanged.
-// Short rows (received in pairs) keep a half: 1536 tokens of 1000 columns on the FP8 wire 232 / 243.
-struct Share {
-    int numerator, denominator;
-};
-template <int kRows>
-constexpr Share kTxShare = kRows > 1 ? Share{1, 2} : Share{2, 3};
-
 template <bool kFp8, bool kVector, int kRows>
 __device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, uint32_t* owed_record, int lane, int order, int waves, DirectRow start) {
     const uint64_t epoch = dispatch_epoch(state);
@@ -1619,6 +1606,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
     PCIE_EP_PROFILE(RoleProfile profile(state.clock_khz); uint64_t idle_begin = 0; int moves = 0;)
     bool prefixes_known = false, gate_open = false, plan_known = state.fused == 0;
     const int lead = int(kTxLeadBytes / int64_t(state.z.meta_offset + state.z.meta_bytes));
+    const int transmitters = transmit_wavefronts(waves, kRows);
     // A wavefront that may be wanted for transmitting binds itself to one batch at a time.
     const int most_claims = 2 * order < waves || kRows == 1 ? kRows : kReceiveClaims;
     uint64_t idle_since = 0;  // 0: the last look found work
@@ -1654,11 +1642,11 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 const bool tx_done = tx_total >= 0 && tx_head >= tx_total, rx_done = rx_total >= 0 && rx_head >= rx_total;
                 // Totals unknown: a handful of wavefronts start to transmit, the others
                 // wait for the first descriptors.
-                bool prefer_tx = order < kMinTxWaves && kTxShare<kRows>.denominator * order < kTxShare<kRows>.numerator * waves;
+                bool prefer_tx = order < kMinTxWaves && order < transmitters;
                 if (tx_total >= 0 && rx_total >= 0) {
                     const int rx_rows = rx_total - rx_head - (lead < rx_total / 4 ? lead : rx_total / 4);
                     const int64_t tx_left = tx_done ? 0 : kTxWeight<kFp8> * (tx_total - tx_head), rx_left = rx_rows > 0 ? kRxWeight * rx_rows : 0;
-                    prefer_tx = rx_done || (tx_left > 0 && kTxShare<kRows>.denominator * order < kTxShare<kRows>.numerator * waves &&
+                    prefer_tx = rx_done || (tx_left > 0 && order < transmitters &&
                                             (order < kMinTxWaves || int64_t(order) * (tx_left + rx_left) < int64_t(waves) * tx_left));
                 }
                 const bool own_backlog = prefer_tx ? tx_backlog : rx_backlog, other_backlog = prefer_tx ? rx_backlog : tx_backlog;
@@ -1671,7 +1659,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                     // everything has been received.  A transmit row waits for its receivers (slot ACK,
                     // descriptor credit); if every wavefront of a rank could end up in such a wait, two
                     // ranks whose receivers are each other's kernels could wait for each other for ever.
-                    // The wavefronts that do not transmit by the rule above (at least a third of them)
+                    // The wavefronts that do not transmit by the rule above (transmit_wavefronts())
                     // therefore never do while a row may still come in.
                     if (own_done || (prefer_tx && now - idle_since > kIdleCrossoverUs * state.clock_khz / 1000)) choice = prefer_tx ? 2 : 1;
                 }

@@ -52,6 +52,22 @@ constexpr int kStatFields = 8;
 constexpr size_t kSignalBytes = 128;  // one writer per 128-byte line
 constexpr size_t kPageBytes = 4096;
 
+// Of `waves` payload wavefronts that receive `batch` rows at a time, the first so many may transmit while rows are left
+// to receive.  The others never do: a transmitting wavefront waits for its receivers, and two ranks whose wavefronts all
+// waited so would wait for each other until the timeout.  From two wavefronts on, at least one therefore only receives.
+//
+// Two thirds for rows moved one at a time.  Requests of both directions wait in the same queues on their way to the
+// link: a rank that sends as much as it receives used the link's two halves one after the other with one transmitting
+// wavefront per receiving one, because a transmitting wavefront spends more of its time off the link (claim, plan, the
+// row's reads from HBM).  64 MB each way by a bare kernel: 2.1 ms with two reading wavefronts per writing one, 1.4 with
+// one, 1.12 for either direction alone.  Us per dispatch with a half and with two thirds: 2 ranks, 1000 tokens of 4096
+// columns 277 / 246, 300 of 7168 167 / 161; 8 ranks unchanged.
+// Half for short rows, received in pairs: 1536 tokens of 1000 columns on the FP8 wire 232 / 243.
+PCIE_EP_HD int transmit_wavefronts(int waves, int batch) {
+    if (batch > 1) return (waves + 1) / 2;
+    return waves > 1 ? 2 * waves / 3 : waves;
+}
+
 // Device error codes: values are part of the Python result contract
 // (csrc/kernels/host_staged/common.cuh:26-38).
 enum ErrorCode : int {

@@ -97,6 +97,15 @@ def test_two_runtimes_dispatch_to_each_other(slots, descriptors):
     run_world(2, [96, 71], 1024, 4, 16, ROUNDS, channels=2, payload_slots=slots, descriptor_slots=descriptors, worker_groups=8)
 
 
+@pytest.mark.parametrize("shape", [dict(worker_groups=1, tx_waves=1, rx_waves=1, channels=2), dict(worker_groups=-1, tx_waves=1, rx_waves=1, channels=1),
+                                   dict(worker_groups=1, tx_waves=1, rx_waves=2, channels=1)], ids=["2-waves", "2-waves-with-the-controls", "3-waves"])
+def test_two_runtimes_with_few_payload_wavefronts(shape):
+    """Rows moved one at a time, one-slot rings, two or three payload wavefronts per rank: one of them must keep
+    receiving while the others wait for the peer's acknowledgements."""
+    run_world(2, [40, 33], 2048, 4, 16, ROUNDS[:3], payload_slots=1, descriptor_slots=1, **shape)
+    run_world(2, [40, 33], 4608, 4, 16, ROUNDS[:2], payload_slots=1, descriptor_slots=1, stage=7, wire_dtype="fp8_e4m3", **shape)
+
+
 def test_two_runtimes_full_width_rows_fp8_wire():
     run_world(2, [64, 64], 7168, 8, 64, ROUNDS[:2], channels=4, worker_groups=8, stage=7, wire_dtype="fp8_e4m3")
 

@@ -68,3 +68,16 @@ def test_relay_failure_paths(relay_program):
     assert outcome.returncode == 0, report
     assert "relay failure test passed" in outcome.stdout, report
     assert "Sanitizer" not in outcome.stderr, report
+
+
+def test_a_payload_wavefront_always_only_receives(tmp_path):
+    """A transmitting wavefront waits for its receivers; if all of two ranks' did, those ranks would wait for each
+    other.  The rule that keeps one back, over every number of payload wavefronts."""
+    if shutil.which("g++") is None:
+        pytest.skip("no host compiler")
+    binary = tmp_path / "transmit_share"
+    built = subprocess.run(["g++", "-std=c++20", "-O1", "-Wall", f"-I{CSRC}", str(ROOT / "tests" / "transmit_share_test.cpp"), "-o", str(binary)],
+                           capture_output=True, text=True, timeout=300)
+    assert built.returncode == 0, built.stderr[-3000:]
+    outcome = subprocess.run([str(binary)], capture_output=True, text=True, timeout=60)
+    assert outcome.returncode == 0, outcome.stdout + outcome.stderr
