@@ -75,11 +75,11 @@ namespace {
 constexpr int kScratchDwords = kReceiveScratchDwords;  // per wavefront: slot metadata records (of one or kMaxReceiveBatch rows)
 constexpr int kMaxWaves = 12;
 // What a payload wavefront owes the other ends (see Owed): slot ACKs (address, token), then a transmitted row's
-// channel, slot, token and descriptor ordinal per endpoint; behind them the words of a direct row's ticket and the
-// wavefront's counters.
+// channel, slot, token and descriptor ordinal per endpoint; behind them the words of a direct row's ticket, its scale
+// and the wavefront's counters.
 constexpr int kTicketWords = int(sizeof(TxEntry) / 4);
 constexpr int kOwedRow = 4 * kMaxReceiveBatch, kOwedDescriptors = kOwedRow + 4, kDirectTicket = kOwedDescriptors + kMaxEndpoints;
-constexpr int kOwedCounts = kDirectTicket + kTicketWords, kOwedDwords = kOwedCounts + 8;
+constexpr int kDirectScale = kDirectTicket + kTicketWords, kOwedCounts = kDirectScale + 1, kOwedDwords = kOwedCounts + 8;
 
 struct WaveScratch {
     uint32_t words[kMaxWaves][kScratchDwords];
@@ -482,10 +482,6 @@ __device__ __forceinline__ Descriptor* descriptor_of(const DeviceState& state, i
 constexpr int64_t kDirectBytes = 544 << 10;
 constexpr int64_t kDirectDispatchBytes = 6 << 20;
 constexpr int kMaxDirectRows = 3;
-struct DirectRow {
-    bool valid = false;
-    float scale = 1.0f;
-};
 __device__ __forceinline__ int payload_wavefronts(const DeviceState& state) { return state.worker_groups * (state.tx_waves + state.rx_waves); }
 // How many tokens of every channel are direct rows: with the prologue in the launch, payload wavefronts of their own for
 // them, and rings that the dispatch before has left drained.
@@ -994,19 +990,19 @@ __device__ __forceinline__ float tx_copy_row(const DeviceState& state, const uin
     return 1.0f;
 }
 
-// Payload wavefront `order` transmits the payload of its direct row, if it has one, and leaves the words of its ticket in `ticket`.
+// Payload wavefront `order` transmits the payload of its direct row, if it has one, and leaves the words of its ticket and
+// behind them the row's scale in `ticket`.  Whether it had one.
 template <bool kFp8, bool kVector, int kRows>
-__device__ __forceinline__ DirectRow direct_row(const DeviceState& state, uint32_t* ticket, int order, int lane) {
+__device__ __forceinline__ bool direct_row(const DeviceState& state, uint32_t* ticket, int order, int lane) {
     const SegmentLayout& z = state.z;
     const int channels = z.dims.channels, me = state.local_rank, token = order;
-    DirectRow row;
-    if (!state.fused || token >= state.num_tokens || token >= channels * kMaxDirectRows || token >= channels * broadcast_first(direct_rows_per_channel(state))) return row;
+    if (!state.fused || token >= state.num_tokens || token >= channels * kMaxDirectRows || token >= channels * broadcast_first(direct_rows_per_channel(state))) return false;
     // Lane c: the channel's candidate c.
     const int channel = token % channels, candidate = token / channels;
     uint32_t remote = 0;
     if (lane <= candidate) remote = endpoint_mask_of(z.dims, me, early_destinations(state, channel + lane * channels));
     const uint32_t endpoints = uint32_t(__shfl(int(remote), candidate));
-    if (endpoints == 0) return row;
+    if (endpoints == 0) return false;
     const uint64_t in_front = lanes_below(candidate);
     const int ordinal = __popcll(__ballot(remote != 0) & in_front);
     // Lane 4 + e: descriptor ordinal of endpoint e (TxEntry).
@@ -1016,10 +1012,10 @@ __device__ __forceinline__ DirectRow direct_row(const DeviceState& state, uint32
         if (lane == 4 + endpoint) word = uint32_t(before);
     }
     if (lane < kTicketWords) ticket[lane] = word;
-    row.scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden,
-                                                  host_resource(slot_at(z, state.seg[me], channel, ordinal), uint32_t(z.meta_offset)), lane, [] {});
-    row.valid = true;
-    return row;
+    const float scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden,
+                                                          host_resource(slot_at(z, state.seg[me], channel, ordinal), uint32_t(z.meta_offset)), lane, [] {});
+    if (lane == 0) ticket[kTicketWords] = float_bits(scale);
+    return true;
 }
 
 // What a payload wavefront still owes the other ends of the rows it has moved: a received row's slot ACK (lane r: row
@@ -1073,8 +1069,10 @@ __device__ __forceinline__ void count_rows(uint32_t* record, WorkerCount which, 
 
 // Moves the own token of transmit ticket `ticket_index` (already marked ready), or of the direct row whose payload is on
 // its way, into its host slot; what publishes it is left to settle().  Returns false when the wavefront must stop.
-template <bool kFp8, bool kVector, int kRows, bool kDirect>
-__device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int ticket_index, float direct_scale,
+// One copy of this code serves both: with a second one for direct rows five of the eight kernels kept up to eight
+// registers in scratch memory.
+template <bool kFp8, bool kVector, int kRows>
+__device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues& q, uint32_t* scratch, int lane, int ticket_index, bool direct,
                        const Deadline& deadline, Owed& owed, bool& plan_known PCIE_EP_PROFILE(, RoleProfile& profile, bool sampled)) {
     const SegmentLayout& z = state.z;
     const int ranks = z.dims.num_ranks, topk = z.dims.topk, me = state.local_rank;
@@ -1089,7 +1087,7 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         // Copy the ticket out of the ring (one dword per lane), then free its entry.
         const uint32_t entry_base = uint32_t(ticket_index % kRing) * uint32_t(sizeof(TxEntry));
         uint32_t word;
-        if constexpr (kDirect) {
+        if (direct) {
             word = owed.record[kDirectTicket + (lane < kTicketWords ? lane : 0)];
             if (lane == 0) device_add(reinterpret_cast<uint32_t*>(&q.tx_head.direct), 1u);
         } else {
@@ -1099,7 +1097,7 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         const uint32_t endpoints = uint32_t(__shfl(int(word), 2));
         const int channel = __shfl(int(word), 3);
         const int my_descriptor = __shfl(int(word), 4 + (lane < endpoint_count ? lane : 0));
-        if constexpr (!kDirect) {
+        if (!direct) {
             wait_memory_ops();
             if (lane == 0) device_store(q.tx_taken + ticket_index % kRing, sequence(epoch, ticket_index));
         }
@@ -1161,10 +1159,10 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
         }
         if (lane == kWave - 1) test_delay(state.tx_delay);
         const __amdgpu_buffer_rsrc_t slot_resource = host_resource(slot_base, uint32_t(z.meta_offset + z.meta_bytes));
-        float scale = direct_scale;
-        if constexpr (!kDirect)
-            scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden, host_resource(slot_base, uint32_t(z.meta_offset)), lane,
-                                                      [&] { settle(state, q, owed, lane); });
+        float scale;
+        if (direct) scale = bits_float(owed.record[kDirectScale]);
+        else scale = tx_copy_row<kFp8, kVector, kRows>(state, state.x + size_t(token) * z.dims.hidden, host_resource(slot_base, uint32_t(z.meta_offset)), lane,
+                                                       [&] { settle(state, q, owed, lane); });
         if (lane == 0) scratch[2] = float_bits(scale);
         fence_lds();
         if (lane == meta_dwords - 1 || (lane == kWave - 1 && meta_dwords > kWave)) test_delay(state.metadata_delay);
@@ -1597,8 +1595,9 @@ constexpr int64_t kTxLeadBytes = 24 << 20;
 constexpr int kMinTxWaves = 16;
 constexpr uint64_t kIdleCrossoverUs = 30;
 constexpr int kPreGateRows = 32;
+
 template <bool kFp8, bool kVector, int kRows>
-__device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, uint32_t* owed_record, int lane, int order, int waves, DirectRow start) {
+__device__ __forceinline__ void payload_worker(const DeviceState& state, TransportQueues& q, uint32_t* scratch, uint32_t* owed_record, int lane, int order, int waves, bool direct) {
     const uint64_t epoch = dispatch_epoch(state);
     Deadline deadline(now_ticks());
     if (lane < kWorkerCounts) owed_record[kOwedCounts + lane] = 0;
@@ -1612,14 +1611,14 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
     uint64_t idle_since = 0;  // 0: the last look found work
     fence_lds();
     bool go_on = true;
-    // (Its ticket's words are in the record.)
-    if (start.valid) go_on = tx_row<kFp8, kVector, kRows, true>(state, q, scratch, lane, 0, start.scale, deadline, owed, plan_known PCIE_EP_PROFILE(, profile, false));
+    direct = broadcast_first(direct ? 1 : 0) != 0;  // uniform, for the compiler too
     while (go_on) {
         // 0: nothing to do now, 1: transmit, 2: receive, -1: both directions are finished or the kernel aborts.
-        int choice = 0, claims = 1, prompt = 1;
+        // A direct row comes first and needs neither a look nor a ticket.
+        int choice = direct ? 1 : 0, claims = 1, prompt = 1;
         PCIE_EP_PROFILE(const uint64_t look_begin = profile.now();)
         int gate_seen = gate_open ? 1 : 0;
-        if (lane == 0) {
+        if (lane == 0 && !direct) {
             if (aborted(q)) choice = -1;
             else {
                 const int tx_head = int(device_load(&q.tx_head.value)), rx_head = int(device_load(&q.rx_head.value));
@@ -1701,25 +1700,25 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
         PCIE_EP_PROFILE(profile.first(kProfileFirstClaimNs); const uint64_t claim_begin = profile.now(); if (!profile.values[kProfileFirstLookNs]) profile.values[kProfileFirstLookNs] = look_begin;)
         claims = broadcast_first(claims);
         owed.prompt = broadcast_first(prompt) != 0;
-        int ticket_index = claim_tickets(head, claims, lane);
+        int ticket_index = direct ? 0 : claim_tickets(head, claims, lane);
         const int end = ticket_index + claims;
         // Several wavefronts may have seen the same backlog: a claim beyond the last
         // ticket of the dispatch is simply dropped, an earlier one waits for its tag.
         // Rows whose tickets are ready never wait for a later ticket of the same claim: a
         // source may publish that one only when it has seen these rows acknowledged.
         while (go_on && ticket_index < end) {
-            if (wait_ticket(state, q, transmit ? q.tx_ready : q.rx_ready, head, ticket_index, epoch, lane, deadline, [&] {
+            if (!direct && wait_ticket(state, q, transmit ? q.tx_ready : q.rx_ready, head, ticket_index, epoch, lane, deadline, [&] {
                     wait_memory_ops();
                     settle(state, q, owed, lane);
                 }) < 0) {
                 if (broadcast_first(aborted(q) ? 1 : 0)) go_on = false;
                 break;
             }
-            PCIE_EP_PROFILE(profile.first(kProfileFirstTaggedNs); profile.add(kProfileTicketWaitSum, profile.now() - claim_begin); const bool sampled = moves++ % kProfileSampleStride == 0;
+            PCIE_EP_PROFILE(profile.first(kProfileFirstTaggedNs); profile.add(kProfileTicketWaitSum, profile.now() - claim_begin); const bool sampled = !direct && moves++ % kProfileSampleStride == 0;
                             if (sampled) profile.add(transmit ? kProfileSampledTxRows : kProfileSampledRxRows);)
             int count = 1;
             if (transmit) {
-                go_on = tx_row<kFp8, kVector, kRows, false>(state, q, scratch, lane, ticket_index, 1.0f, deadline, owed, plan_known PCIE_EP_PROFILE(, profile, sampled));
+                go_on = tx_row<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, direct, deadline, owed, plan_known PCIE_EP_PROFILE(, profile, sampled));
             } else {
                 if constexpr (kRows > 1) {
                     const bool ready = lane < kRows && lane < end - ticket_index &&
@@ -1728,6 +1727,7 @@ __device__ __forceinline__ void payload_worker(const DeviceState& state, Transpo
                 }
                 go_on = rx_rows<kFp8, kVector, kRows>(state, q, scratch, lane, ticket_index, count, owed, deadline, gate_open, prefixes_known PCIE_EP_PROFILE(, profile, sampled));
             }
+            direct = false;
             ticket_index += count;
             PCIE_EP_PROFILE(profile.add(transmit ? kProfileTxRows : kProfileRxRows, uint64_t(count)); profile.last(kProfileLastRowNs);)
         }
@@ -1817,7 +1817,7 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
     if (receive_channel >= 0) first_poll = rx_first_poll(state, receive_channel, lane);
     // Position of a payload wavefront among all of them, wavefront-major: a
     // direction's share is spread over the workgroups before it doubles up in one.
-    DirectRow direct;
+    bool direct = false;
     if (payload_groups && block >= channel_groups && block < channel_groups + payload_groups && wave < payload_waves)
         direct = direct_row<kFp8, kVector, kRows>(state, owed_record + kDirectTicket, wave * payload_groups + block - channel_groups, lane);
     PrefixFirstLook first_look{0, false};
