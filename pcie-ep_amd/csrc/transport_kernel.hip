@@ -73,19 +73,21 @@ namespace pcie_ep {
 namespace {
 
 constexpr int kScratchDwords = kReceiveScratchDwords;  // per wavefront: slot metadata records (of one or kMaxReceiveBatch rows)
-constexpr int kMaxWaves = 12;
 // What a payload wavefront owes the other ends (see Owed): slot ACKs (address, token), then a transmitted row's
 // channel, slot, token and descriptor ordinal per endpoint; behind them the words of a direct row's ticket, its scale
 // and the wavefront's counters.
 constexpr int kTicketWords = int(sizeof(TxEntry) / 4);
 constexpr int kOwedRow = 4 * kMaxReceiveBatch, kOwedDescriptors = kOwedRow + 4, kDirectTicket = kOwedDescriptors + kMaxEndpoints;
-constexpr int kDirectScale = kDirectTicket + kTicketWords, kOwedCounts = kDirectScale + 1, kOwedDwords = kOwedCounts + 8;
+constexpr int kDirectScale = kDirectTicket + kTicketWords, kOwedCounts = kDirectScale + 1, kOwedDwords = kOwedCounts + 7;
 
+// One of these per wavefront of the workgroup, in the LDS that the launch asks for (transport_lds_bytes), where a workgroup of
+// the prologue has its tables.  Sized for the largest workgroup and beside those tables, they took the ragged kernels from
+// four workgroups on a compute unit to three from 640 experts on (16 ranks, 32 channels).
 struct WaveScratch {
-    uint32_t words[kMaxWaves][kScratchDwords];
-    uint32_t owed[kMaxWaves][kOwedDwords];
-    int begun;
+    uint32_t words[kScratchDwords];
+    uint32_t owed[kOwedDwords];
 };
+static_assert(kOwedCounts + 5 <= kOwedDwords && sizeof(WaveScratch) % 16 == 0, "room for every counter, vectors on 16-byte boundaries");
 
 // Local time only: payload workers never scan the host abort flags themselves
 // (hundreds of wavefronts doing so would be PCIe traffic of their own); the
@@ -1765,14 +1767,16 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
 #else
     const DeviceState& state = launch_state;  // the host pass only parses the kernel
 #endif
-    __shared__ WaveScratch lds;
-    extern __shared__ __align__(16) unsigned char prologue_lds[];  // sized by the launcher when the prologue rides in this launch
+    // The tables of a workgroup of the prologue, or one WaveScratch per wavefront of any other.
+    extern __shared__ __align__(16) unsigned char dynamic_lds[];
+    __shared__ int epoch_begun;
     const int channels = state.z.dims.channels;
     int block = transport_block(transport_grid(state), int(blockIdx.x));
     if (block < 0) return;  // a filler id
     int wave = threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
-    uint32_t *scratch = lds.words[wave], *owed_record = lds.owed[wave];
+    WaveScratch& own_scratch = reinterpret_cast<WaveScratch*>(dynamic_lds)[wave];
+    uint32_t *scratch = own_scratch.words, *owed_record = own_scratch.owed;
     TransportQueues& q = *state.queues;
     const int payload_waves = state.tx_waves + state.rx_waves;
     const int payload_groups = state.worker_groups > 0 ? state.worker_groups : 0;
@@ -1796,7 +1800,7 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
                 if (wave >= 2) return;
                 return finish_role(state, q, lane, roles);
             }
-            prologue_chunk<8, true>(state, prologue_lds, waves_per_group, state.prologue_chunks, block - 1);
+            prologue_chunk<8, true>(state, dynamic_lds, waves_per_group, state.prologue_chunks, block - 1);
             if (wave == 0) finish_role(state, q, lane, roles);
             return;
         }
@@ -1824,9 +1828,9 @@ __global__ void __launch_bounds__(kTransportMaxThreads, kVector ? 3 : 4) transpo
     if (prefix_producer) first_look = prefix_first_look(state, lane);
     if (state.fused) {
         // (LDS only: the reads and stores issued above stay in flight.)
-        if (threadIdx.x == blockDim.x - kWave) lds.begun = int(wait_for_begin(state, q));
+        if (threadIdx.x == blockDim.x - kWave) epoch_begun = int(wait_for_begin(state, q));
         lds_barrier();
-        begun = lds.begun != 0;
+        begun = epoch_begun != 0;
     } else if (__syncthreads_or(threadIdx.x == 0 ? int(load_error_code(state) != 0) : 0)) {
         return;  // the prologue kernel in front of this one failed
     }
@@ -1899,25 +1903,27 @@ static auto transport_instance(const DeviceState& state) {
     return vector ? transport_kernel<false, true, 1> : transport_kernel<false, false, 1>;
 }
 
+// LDS that a launch asks for beyond what the kernel declares.
+static size_t transport_lds_bytes(const DeviceState& state, int threads) {
+    const size_t scratch = size_t(threads / kWave) * sizeof(WaveScratch);
+    const size_t tables = state.fused ? prologue_lds_bytes(state.z, threads / kWave) : 0;
+    return scratch > tables ? scratch : tables;
+}
+
 // How many transport workgroups one compute unit holds at once (registers, LDS and
 // wavefront slots of the instantiation that `state` selects).
 hipError_t transport_workgroups_per_unit(const DeviceState& state, int* per_unit) {
     const int threads = transport_threads(state);
     if (threads > kTransportMaxThreads) return hipErrorInvalidValue;
-    const size_t lds = state.fused ? prologue_lds_bytes(state.z, threads / kWave) : 0;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_unit, transport_instance(state), threads, lds);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_unit, transport_instance(state), threads, transport_lds_bytes(state, threads));
 }
 
 hipError_t launch_transport(const DeviceState& state, hipStream_t stream) {
     const dim3 grid(transport_grid(state).blocks), block(transport_threads(state));
     if (int(block.x) > kTransportMaxThreads) return hipErrorInvalidValue;
-    size_t dynamic_lds = 0;
-    if (state.fused) {
-        // The prologue's chunks are the workgroup's own wavefronts; the conditions are those of fused_prologue_fits().
-        if (!fused_prologue_fits(state.z, int(block.x), state.z.dims.max_tokens)) return hipErrorInvalidValue;
-        dynamic_lds = prologue_lds_bytes(state.z, int(block.x) / kWave);
-    }
-    hipLaunchKernelGGL(transport_instance(state), grid, block, dynamic_lds, stream, state);
+    // The prologue's chunks are the workgroup's own wavefronts; the conditions are those of fused_prologue_fits().
+    if (state.fused && !fused_prologue_fits(state.z, int(block.x), state.z.dims.max_tokens)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(transport_instance(state), grid, block, transport_lds_bytes(state, int(block.x)), stream, state);
     return hipGetLastError();
 }
 

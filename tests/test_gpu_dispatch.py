@@ -232,6 +232,16 @@ def test_ragged_dispatches_fit_four_workgroups_to_a_compute_unit(hidden, fp8):
         check_case(buffer, f"ragged-on-32-units-h{hidden}", [40, 9, 40, 33], alignment=16, fp8=fp8)
 
 
+@pytest.mark.parametrize("experts,hidden,fp8", [(640, 1001, False), (704, 1000, True), (704, 4095, False)])
+def test_ragged_dispatches_of_many_experts_fit_four_workgroups_to_a_compute_unit(experts, hidden, fp8):
+    """The same where the layout tables of the one-launch prologue fill most of a workgroup's share of the LDS."""
+    wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
+    with make_buffer(world=16, tmax=40, hidden=hidden, topk=4, experts=experts, channels=32, comm_stream_cus=40, **wire) as buffer:
+        needed, resident = buffer.runtime.transport_residency(40)
+        assert 3 * 40 < needed <= resident
+        check_case(buffer, f"ragged-on-40-units-e{experts}-h{hidden}", [40, 9, 40, 33] + [3] * 12, fp8=fp8)
+
+
 @pytest.mark.parametrize("hidden,topk,fp8", [(1312, 8, False), (1313, 8, False), (4096, 8, True), (4095, 8, True), (4097, 8, True), (64, 13, False), (64, 14, True)])
 def test_short_rows_are_received_in_pairs(hidden, topk, fp8):
     """Both sides of the line up to which a wavefront takes two rows at a time: longest rows, ragged ones that

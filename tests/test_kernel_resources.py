@@ -46,3 +46,11 @@ def test_no_kernel_keeps_registers_in_scratch_memory(kernels):
         assert kernels[symbol][".vgpr_count"] > 64 and kernels[symbol][".group_segment_fixed_size"] > 0  # the right fields were read
     spilled = {symbol: fields for symbol, fields in kernels.items() if fields[".vgpr_spill_count"] or fields[".private_segment_fixed_size"]}
     assert not spilled
+
+
+def test_the_transport_kernels_declare_next_to_no_lds(kernels):
+    """A workgroup's scratch and the prologue's tables share the LDS that a launch asks for: four workgroups of the
+    largest prologue that then fits (40 960 bytes each of a compute unit's 160 KB) must not be pushed out by what is declared."""
+    for symbol, fields in kernels.items():
+        if "transport_kernel" in symbol:
+            assert fields[".group_segment_fixed_size"] <= 512, symbol
