@@ -220,11 +220,16 @@ int pcie_ep_set_test_delays(pcie_ep_runtime* runtime, uint64_t metadata_ns, uint
 int pcie_ep_set_test_prefix_delay_ns(pcie_ep_runtime* runtime, uint64_t delay_ns);
 int pcie_ep_set_test_control_abort_after_ns(pcie_ep_runtime* runtime, uint64_t delay_ns);
 int pcie_ep_set_test_skip_counts_ack_source(pcie_ep_runtime* runtime, int32_t source);
-/* Overwrite the device-side epoch counter (synchronises the device).  Only for
- * testing epoch exhaustion (error 20 once the epoch would reach 2^32:
+/* Overwrite the device-side epoch counter (synchronises the device); the next
+ * dispatch does not take its rings for drained.  Only for testing epoch exhaustion (error 20 once the epoch would reach 2^32:
  * csrc/kernels/host_staged/advanced_layout.cuh:44-48); no counterpart in the
  * reference, which has no test of that path. */
 int pcie_ep_set_test_epoch(pcie_ep_runtime* runtime, uint64_t epoch);
+/* Rows that the last dispatch of this runtime (pcie_ep_dispatch, not the static-scratch
+ * form) transmitted ahead of its route plan, and the epoch of its last dispatch that
+ * ended with every own slot acknowledged: the condition for such rows in the next one.
+ * Synchronises the device; for tests. */
+int pcie_ep_early_rows(pcie_ep_runtime* runtime, int32_t* rows, uint64_t* drained_epoch);
 
 /* ---- NUMA relay (numa_mode = 1) ------------------------------------------- */
 

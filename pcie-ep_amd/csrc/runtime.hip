@@ -834,7 +834,19 @@ int pcie_ep_set_test_skip_counts_ack_source(pcie_ep_runtime* rt, int32_t source)
 int pcie_ep_set_test_epoch(pcie_ep_runtime* rt, uint64_t epoch) {
     if (!rt || rt->closed) return set_error(PCIE_EP_E_STATE, "advanced runtime is closed or closing");
     HIP_TRY(hipDeviceSynchronize());
+    // A number set by hand says nothing about the rings: the next dispatch does not take them for drained.
+    const uint64_t never_drained = ~uint64_t(0) - 1;
+    HIP_TRY(hipMemcpy(rt->epoch + kDrainedEpochWord, &never_drained, sizeof never_drained, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(rt->epoch, &epoch, sizeof epoch, hipMemcpyHostToDevice));
+    return 0;
+}
+
+int pcie_ep_early_rows(pcie_ep_runtime* rt, int32_t* rows, uint64_t* drained_epoch) {
+    if (!rt || rt->closed) return set_error(PCIE_EP_E_STATE, "advanced runtime is closed or closing");
+    if (!rows || !drained_epoch) return set_error(PCIE_EP_E_INVALID, "bad early row arguments");
+    HIP_TRY(hipDeviceSynchronize());
+    HIP_TRY(hipMemcpy(rows, &rt->queues->tx_head.direct, sizeof *rows, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(drained_epoch, rt->epoch + kDrainedEpochWord, sizeof *drained_epoch, hipMemcpyDeviceToHost));
     return 0;
 }
 

@@ -301,6 +301,13 @@ class NativeRuntime:
     def set_test_epoch(self, epoch: int) -> None:
         _native.check(self._lib.pcie_ep_set_test_epoch(self._require(), epoch), invalid=RuntimeError)
 
+    def early_rows(self) -> tuple:
+        """(rows the last dispatch transmitted ahead of its route plan, epoch of the last dispatch that left the rings
+        drained).  Waits for the device; for tests."""
+        rows, drained = C.c_int32(), C.c_uint64()
+        _native.check(self._lib.pcie_ep_early_rows(self._require(), C.byref(rows), C.byref(drained)), invalid=RuntimeError)
+        return int(rows.value), int(drained.value)
+
     def host_signal_store(self, segment_rank: int, which: int, index: int, value: int) -> None:
         _native.check(self._lib.pcie_ep_host_signal_store(self._require(), segment_rank, which, index, value))
 

@@ -12,6 +12,7 @@ and compared too (TX parity).
 
 from __future__ import annotations
 
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -21,6 +22,7 @@ import pytest
 import torch
 
 from helpers import make_inputs, run_dispatch, verify_captured, verify_dispatch
+from pcie_ep import _native
 
 pytestmark = pytest.mark.gpu
 
@@ -263,13 +265,30 @@ def test_short_rows_are_received_in_pairs(hidden, topk, fp8):
 def test_first_rows_of_a_channel_go_ahead_of_the_plan(world, hidden, slots, descriptors, fp8):
     """Up to three tokens of every channel are transmitted without a ticket, where the dispatch before has drained the
     rings: as many as channels, one less and one more, two and three times as many and beyond; tokens among them that
-    go nowhere or stay on this rank; rings that hold fewer; a dispatch too large for it (6 MB of rows to come) between."""
+    go nowhere or stay on this rank; rings that hold fewer; a dispatch too large for it (6 MB of rows to come) between.
+    Exactly those rows are counted as such, and none behind an epoch that is not known to have drained the rings."""
     wire = {"stage": 7, "wire_dtype": "fp8_e4m3"} if fp8 else {}
-    with make_buffer(world=world, tmax=900, hidden=hidden, channels=4, payload_slots=slots, descriptor_slots=descriptors, **wire) as buffer:
-        for repeat, own in enumerate((3, 4, 5, 8, 13, 40, 900, 1, 0, 12)):
+    channels = 4
+    with make_buffer(world=world, tmax=1000, hidden=hidden, channels=channels, payload_slots=slots, descriptor_slots=descriptors, **wire) as buffer:
+        sizes, shape = buffer.runtime.sizes, [C.c_int32() for _ in range(4)]
+        _native.check(_native.library().pcie_ep_profile_shape(buffer.runtime.handle, *(C.byref(value) for value in shape)))
+        row_bytes = (int(sizes.payload_bytes) + 15) // 16 * 16 + int(sizes.meta_bytes)
+        early = channels * min(3, shape[3].value // (2 * channels), (544 << 10) // (channels * row_bytes), slots, descriptors)
+        assert early >= channels
+        epoch = 0
+        for repeat, own in enumerate((3, 4, 5, 8, 13, 40, 1000, 1, 0, 12)):
             tokens = [own] + [max(0, own - 3 * r) for r in range(1, world)]
-            for pattern in ("random", "partial", "local", "multicast")[: 1 if own > 40 else 4]:
+            too_large = (world - 1) * own * row_bytes > 6 << 20
+            assert too_large == (own == 1000)
+            for pattern in ("random", "partial", "local", "multicast")[: 1 if too_large else 4]:
+                by_hand = repeat in (3, 9) and pattern == "partial"
+                if by_hand:
+                    buffer.runtime.set_test_epoch(epoch)
                 check_case(buffer, f"first-rows-w{world}-h{hidden}", tokens, pattern, expand=repeat % 2 == 0, seed=60 + repeat, fp8=fp8)
+                epoch += 1
+                idx = make_inputs(world, tokens, hidden, EXPERTS, TOPK, pattern, seed=60 + repeat)[0][1]
+                remote = int(((idx >= 0) & (idx // (EXPERTS // world) != 0)).any(dim=1)[:early].sum())
+                assert buffer.runtime.early_rows() == (0 if too_large or by_hand else remote, epoch)
 
 
 def test_profiling_records_count_every_row_of_a_pair():

@@ -172,6 +172,22 @@ def test_expanded_capacity_overflow_is_code_16(inputs):
         failing_dispatch(buffer, inputs, 16)
 
 
+@pytest.mark.parametrize("fault,code", [(FAULT_NO_LAST_ACK, 15), (FAULT_WRONG_SEQUENCE, 18), (FAULT_NO_COUNTS_READY, 12)])
+def test_a_failed_dispatch_does_not_count_as_drained(inputs, fault, code):
+    """The first rows of a dispatch are stored into slots that nobody has checked: the one before must have ended with
+    all of them acknowledged.  A failed one leaves the epoch of the last that did."""
+    with small_buffer() as buffer:
+        result, _ = run_dispatch(buffer, inputs)
+        verify_dispatch(result, inputs, 0, WORLD, EXPERTS, TOPK, True, 1, False)
+        del result
+        rows, drained = buffer.runtime.early_rows()
+        assert rows > 0 and drained == 1
+        buffer.peers.inject_fault(5, fault)
+        print(f"case: fault {fault} at rank 5, second dispatch", flush=True)
+        failing_dispatch(buffer, inputs, code)
+        assert buffer.runtime.early_rows()[1] == 1
+
+
 def test_epoch_exhaustion_is_code_20(inputs):
     """Sequences carry the epoch in their upper 32 bits; a buffer whose epoch would
     reach 2^32 stops with a terminal error instead of wrapping."""
