@@ -73,7 +73,7 @@ struct alignas(128) QueueCounter {
 
 struct alignas(256) TransportQueues {
     QueueCounter rx_tail, tx_tail;  // tickets reserved by producers (fetch-add)
-    QueueCounter rx_head, tx_head;  // tickets claimed by workers (fetch-add); .total = tickets of this dispatch
+    QueueCounter rx_head, tx_head;  // tickets claimed by workers (fetch-add); .total = rows of this dispatch, .total - .direct = its tickets
     QueueCounter abort;             // value != 0: every role exits
     QueueCounter local_head;        // own tokens (then padding gaps) claimed for the local bypass
     QueueCounter finished;          // role wavefronts that have ended; the last one reduces the statistics

@@ -510,9 +510,10 @@ __device__ __forceinline__ void prologue_chunk(const DeviceState& state, unsigne
         }
         PCIE_EP_PROFILE(profile.first(kPrologueChunkTotalsNs);)
     }
-    // This chunk's part of the route plan: every token's stable ordinals.  Nothing
-    // in this workgroup reads them; the leader writes its own after the counts are
-    // on their way to the peers.
+    // This chunk's part of the route plan: every token's stable ordinals.  Nothing in
+    // this workgroup reads them.  Inside the transport launch the leader writes its own
+    // ahead of the epoch's verdict (the plan is announced right behind that); as a kernel
+    // of its own, after the counts are on their way to the peers.
     const auto write_ordinals = [&]() {
         if (live && !stalled) {
             const uint64_t below = lanes_below(lane);

@@ -11,8 +11,8 @@
 // Design for MI355X (64-lane wavefronts, 8 XCDs):
 //  * A payload worker is ONE wavefront that owns a whole row: its up to
 //    14 x 16-byte loads per lane (896 vectors of a 14 336-byte BF16 row) leave
-//    kReadWindow at a time, the row lives in registers, and the same wavefront stores it to
-//    every destination expert row.  The staged row is read once; there is no
+//    kReadWindow at a time (see there), the row lives in registers, and the same
+//    wavefront stores it to every destination expert row.  The staged row is read once; there is no
 //    LDS tile and no producer/consumer hand-off (the reference stages through
 //    shared memory with 3+3 warps per ticket).
 //  * Control wavefronts work on 64 candidates at a time with ballots: TX control
@@ -39,8 +39,9 @@
 //    tickets and flags arrive tens of microseconds late.
 //  * With the prologue in the same launch (one launch per dispatch), the roles
 //    here start with the queues not yet reset: one thread per workgroup waits for
-//    the epoch begin's word before its role touches them, the transmit side and
-//    the local bypass wait for the plan's word, the receive side for neither.
+//    the epoch begin's word before its role touches them; rows to transmit and the
+//    local bypass wait for the plan's word, the transmit controls (which hand out
+//    tickets straight from the routes) and the receive side do not.
 //  * Workers publish their own descriptors and payload ACKs when their own stores /
 //    loads have completed (see settle); control wavefronts only reserve and hand out.
 //  * The first tokens of every channel are copied to their slots without ticket or
@@ -116,9 +117,13 @@ __device__ __forceinline__ bool wait_for_begin(const DeviceState& state, Transpo
     }
     return true;
 }
-// ... and read the route plan once the leader has published the counts and every
-// chunk's part of the plan is in memory.  False when the prologue failed (abort) or
-// never finished (timeout, recorded as a ring-progress error).
+// ... and read the route plan, or publish a row, once the epoch's verdict is there and every chunk's part of the plan
+// is in memory.  The own counts may then still be on their way to the peers: a descriptor can become visible
+// before `counts_ready`.  No receiver is misled by that.  A descriptor carries its epoch and ordinal, a slot its
+// epoch and token; a transport kernel on the other end copies such a row only behind its gate, when the counts of all sources have been
+// requested, and places it by prefixes made of them; a relay worker and an emulated peer take up an epoch when they see its
+// `counts_ready`, and only then look at its descriptors.  False when the prologue failed (abort) or never finished (timeout, recorded as
+// a ring-progress error).
 __device__ __forceinline__ bool wait_for_plan(const DeviceState& state, TransportQueues& q, int lane) {
     if (!state.fused) return true;
     const uint32_t tag = epoch_flag(dispatch_epoch(state));
@@ -479,7 +484,7 @@ __device__ __forceinline__ Descriptor* descriptor_of(const DeviceState& state, i
 // not (4 ranks, 200 tokens of 4096 columns 119 / 110).  And only in a dispatch that receives little (kDirectDispatchBytes,
 // by the rows of all other sources): a longer one ends with its receive side whatever the transmit side does, and
 // the early rows only delay it (96 aligned tokens, 9.7 MB: 145 us without, 148 with them).
-// Us per dispatch without and with: 16 tokens 52 / 48, 32 75 / 68, 64 of 4096 columns 80 / 73, 24 of 2048 (top-4) 40 / 35,
+// Us per dispatch without and with: 16 tokens 50.2 / 48.2, 32 75 / 68, 64 of 4096 columns 80 / 73, 24 of 2048 (top-4) 40 / 35,
 // 2 ranks with 300 tokens 157 / 138.
 constexpr int64_t kDirectBytes = 544 << 10;
 constexpr int64_t kDirectDispatchBytes = 6 << 20;
@@ -1204,6 +1209,8 @@ __device__ __forceinline__ bool tx_row(const DeviceState& state, TransportQueues
 // flight each, 37 with 4, 18 with 2.)  Wavefronts are not always reading, so that fewer than 4 cost more than they save:
 // us per dispatch with all 14, with 4, with 2, with 1: 700 tokens 647 / 645 / 648 / 661, cached replay of 128 185 / 183 /
 // 189 / 193, 2000 tokens hotspot top-4 1645 / 1625 / 1641 / -, 300 tokens on 2 ranks 154 / 150 / 152 / 161.
+// It spaces the first pass of a row that is received alone: all of the row up to 8192 columns (4096 of ragged BF16 rows).
+// A pass behind the first is requested whole, as are short rows received two at a time.
 constexpr int kReadWindow = 4;
 // Reads the rows of receive tickets first_ticket .. first_ticket + count - 1 (already
 // marked ready, count <= kRows) from their host slots and stores them to their
