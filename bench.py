@@ -19,7 +19,7 @@ transport kernel against the pinned hipMemcpy peak of the same run) and
 ``cpu_baseline`` (layout + expand in PyTorch on the host cores).  The default run
 adds one compact record per further workload of the metric — ``fp8`` (FP8 wire,
 heavy-tailed inputs), ``hotspot_top4``, ``t4096``, ``eager_small_t``
-(T in 16..2048) and ``graph_replay_us`` (cached layout + hipGraph replay) —
+(T in 16..2048) and ``graph_replay_us`` (cached layout + captured replay) —
 each timed the same way and each with a ``parity`` flag from an untimed
 dispatch checked bit for bit against the oracle.
 """
@@ -373,8 +373,8 @@ def compact(run, tokens, topk):
 
 
 def graph_replay_sweep(topk, channels, sizes=(16, 128, 512, 2048, 8192), replays=20, inputs_by_size=None):
-    """Cached layout + hipGraph replay: the plan is built by one eager dispatch,
-    the dispatch is captured with that plan, `replays` GPU-only replays are
+    """Cached layout + replay of a captured dispatch: the plan is built by one eager
+    dispatch, the dispatch is captured with that plan, `replays` replays are
     timed back to back (mean microseconds per replay, by size), and one more,
     untimed, is checked against the oracle."""
     import torch
@@ -384,8 +384,7 @@ def graph_replay_sweep(topk, channels, sizes=(16, 128, 512, 2048, 8192), replays
     out = {}
     requested = replays
     for tokens in sizes:
-        # The shortest replay needs more of them between the synchronisations that bracket the timed region (at
-        # larger sizes more than a few dozen launches of one instantiated graph in flight make hipGraphLaunch block).
+        # The shortest replay needs more of them between the synchronisations that bracket the timed region.
         replays = max(requested, 100) if tokens <= 16 else requested
         inputs = (inputs_by_size or {}).get(tokens) or build_inputs(tokens, topk, "uniform", False)
         with make_buffer(tokens, topk, "bf16", channels, fuse=True, graph=True) as buffer:

@@ -1,5 +1,6 @@
-"""One dispatch captured into a hipGraph (``torch.cuda.CUDAGraph`` on ROCm) and
-replayed without any CPU-side work on the kernels.
+"""One dispatch captured once (``torch.cuda.CUDAGraph`` on ROCm) and replayed with
+its addresses, options and result pool frozen: a replay admits nothing, allocates
+nothing and looks up no pool or plan.
 
 Contract (the reference's pcie_ep/graph.py:20-202; API.md): a buffer prepares at
 most one ``GraphDispatch``; it is bound to the addresses of its inputs and to the
@@ -12,7 +13,13 @@ tensor's current contents.
 Implementation: capture and replay both go through the buffer's single launch
 path (``HostStagedEPBuffer._launch``) — a replay is the same admitted request
 with the launch of the captured kernels as its work instead of ``runtime.dispatch`` —
-so stream ordering, consumer tracking and result wrapping exist once.
+so stream ordering, consumer tracking and result wrapping exist once.  A replay
+submits those kernels as ordinary launches with the captured arguments; the
+instantiated graph itself is launched only where the dispatch was captured with the
+static scratch.  What the arguments do not hold is the runtime's and is read when a
+replay is submitted: test delays, the skipped counts acknowledgement, and kernel
+timing, which therefore covers replays (not those of the static scratch, whose
+kernels keep the values of the capture).
 """
 
 from __future__ import annotations
